@@ -6,133 +6,58 @@
 // untransposed), each with its own leading dim; batched forms take per-axis batch strides or pointer
 // arrays.  beta = 0 never reads C.
 //
-// Tiling.  A workgroup owns a BM x BN tile of C and each of its waves a (16 TM) x (16 TN) block of it,
-// held as TM x TN 16 x 16 accumulator tiles (4 floats per lane each).  K advances 16 at a time
-// through two LDS stages: the next step's panels are loaded into registers while the matrix cores
-// work on the current one, stored into the other stage, and one barrier per step separates the two.
-// Each operand keeps its global layout in LDS (layouts at Panel below): a K-contiguous operand's
-// fragment is one 16-byte LDS read, an M/N-contiguous one's four 4-byte reads.  The MFMAs take the B
-// fragment first and so produce C^T tiles: each lane holds 4 consecutive columns of a row of C, and
-// the epilogue writes (and, for beta != 0, reads) C 16 bytes at a time.
+// Tiling.  A workgroup owns a BM x BN tile of C and each of its waves a (16 TM) x (16 TN) block of it (or of its
+// share of K, gemm_tile.hpp), held as TM x TN 16 x 16 accumulator tiles (4 floats per lane each).  Each operand
+// keeps its global layout in LDS, so every operand layout runs without a transposing pass.  The MFMAs take
+// the B fragment first and so produce C^T tiles: each lane holds consecutive columns of a row of C, and the
+// epilogue writes (and, for beta != 0, reads) C 16 bytes at a time.
 //
 // k mapping.  One MFMA multiplies a 16 x 4 slice of A by a 4 x 16 slice of B, quarter-wave q (lanes
-// 16 q .. 16 q + 15) holding one k.  In each stage of 16 k, quarter q gives the s-th MFMA (s = 0..3)
+// 16 q .. 16 q + 15) holding one k.  In each half panel of 16 k, quarter q gives the s-th MFMA (s = 0..3)
 // the value at k = 4 q + s, for A and B alike, so a K-contiguous operand feeds four MFMAs from one
 // 16-byte LDS read.
 //
 // Summation order (blocked, like the reference's register blocks summed from zero and added into C,
-// kernels_avx2.c:234-247): K is cut into panels of 32 k (two stages).  A panel's 32 products of an
-// output element are summed from zero, four per MFMA (eight MFMAs), and the panel sum is added into the
-// element's running total (one fp32 add per 32 k).  A small panel sum is not rounded against the whole
-// running total, so the error of a K-term dot product grows like that of a blocked sum rather than like
-// K sequential additions.  The order is a property of the kernel alone: the same for every tile size
-// and grid, so results are identical run to run and on any device.  It differs from the reference's
-// serial order, so the parity bar is the fp32 error bound of a K-term dot product.
+// kernels_avx2.c:234-247): K is cut into panels of 32 k.  A panel's 32 products of an output element are summed
+// from zero, four per MFMA (eight MFMAs), and the panel sum is added into a running total (one fp32 add per 32 k);
+// where a tile's waves split K, wave group g of S sums panels g, g + S, ... so and the S totals are added in
+// order.  A small panel sum is not rounded against the whole running total, so the error of a K-term dot product
+// grows like that of a blocked sum rather than like K sequential additions.  A panel that K ends inside comes
+// first.  The tile, and with it the split, is chosen from the problem's shape and layout alone (sg_pick), so
+// results are identical run to run and on any device.  The order differs from the reference's serial one, so
+// the parity bar is the fp32 error bound of a K-term dot product.
 //
-// Tile sizes: 256 x 256 (8 waves of 8 x 4 tiles) when the problem has at least as many such tiles as
-// the device has CUs, else 128 x 128 (4 waves of 4 x 4) or 64 x 64 (4 waves of 2 x 2).  Blocks are
-// remapped so each XCD (blocks b with b % 8 equal) works a contiguous run of tiles, and tiles run in
-// groups of 8 tile-rows so neighbouring blocks share panels in L2.
-#include "common.hpp"
+// Kernels: k_sgemm_dma (256 x 256 tiles, panels loaded straight into LDS) for aligned problems that give every CU
+// such tiles, the register-staged tiles of gemm_tile.hpp for the rest.  Blocks are remapped so each XCD
+// (blocks b with b % 8 equal) works a contiguous run of tiles, and tiles run in groups of 8 tile-rows so
+// neighbouring blocks share panels in L2.
+#include "gemm.hpp"
 
 namespace nchip {
-
 
 constexpr int kSgBK = 16;      // k per stage
 constexpr int kSgPanel = 2;    // stages per summation panel (32 k)
 
-constexpr int kSgGroupM = 8;   // tile-rows per group in the block order
-
-// MINB: workgroups per CU the register allocation leaves room for
-template <int TM_, int TN_, int WGM_, int WGN_, int MINB_>
+// The direct-to-LDS tile: TM x TN 16 x 16 accumulator tiles per wave, WGM x WGN waves
+template <int TM_, int TN_, int WGM_, int WGN_>
 struct SgCfg {
     static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_;
-    static constexpr int MINB = MINB_;
     static constexpr int NT = 64 * WGM * WGN;
     static constexpr int BM = 16 * TM * WGM, BN = 16 * TN * WGN;
     // bytes of one stage of an operand panel in LDS (R rows by 16 k, either layout)
     static constexpr int SLAB_A = 64 * BM, SLAB_B = 64 * BN;
     static constexpr int STAGE = SLAB_A + SLAB_B;
-    static constexpr size_t LDS = 2 * (size_t)STAGE;
 };
-using SgBig = SgCfg<8, 4, 2, 4, 1>;    // 256 x 256
-using SgMid = SgCfg<4, 4, 2, 2, 2>;    // 128 x 128
-using SgSmall = SgCfg<2, 2, 2, 2, 4>;  // 64 x 64
+using SgBig = SgCfg<8, 4, 2, 4>;  // 256 x 256
 
-struct SgBatch {
-    int nb;  // 0: one matrix per operand
-    int64_t shape[NC_HIP_MAX_DIMS];
-    int64_t st[3][NC_HIP_MAX_DIMS];  // element strides of A, B, C per batch axis
-};
-
-struct SgArgs {
-    const float *A, *B;
-    float *C;
-    const float *const *pa;  // pointer-array batches (instead of strides) when set
-    const float *const *pb;
-    float *const *pc;
-    int64_t lda, ldb, ldc;
-    int M, N, K;
-    float alpha, beta;
-    const float *bias;  // N floats added to every row after alpha A B + beta C, or none
-    int tiles_m, tiles_n;
-    SgBatch bat;
-};
-
-// ---- operand panels ------------------------------------------------------------------------------
-// One stage of an operand: R rows (M or N) by 16 k, loaded as 16-byte chunks spread over the
-// workgroup's threads, kept in registers while the previous stage is multiplied, then stored to LDS.
-//   * K-contiguous operand: chunk u is row u / 4, k 4 (u % 4) .. + 3; in LDS rows of 64 bytes, logical
-//     chunk c of row r at chunk c ^ kc_swz(r), so the 16-byte fragment reads spread over all banks;
-//   * M/N-contiguous operand: chunk u is k-row u / (R / 4), rows 4 (u % (R / 4)) .. + 3; in LDS 16
-//     k-rows of R floats (R >= 64), the chunk of rows 4 c .. 4 c + 3 of k-row k at chunk c ^ mn_swz(k),
-//     so the four quarter-waves' fragment reads (k-rows k, k + 4, k + 8, k + 12 of 16 consecutive
-//     rows) land in different banks.  Either layout is 64 R bytes per stage, with no padding, so a
-//     load straight into LDS fills it 1 KiB at a time.
-template <int R, bool KC, int NT>
-struct Panel {
-    static constexpr int UNITS = 4 * R;
-    static constexpr int UPT = (UNITS + NT - 1) / NT;  // chunks per thread
-    static constexpr bool GUARD = UNITS % NT != 0;     // some threads own fewer chunks
-};
-
-// global-memory views, so loads are global_load (counted by vmcnt alone) rather than flat
-typedef const __attribute__((address_space(1))) float gfloat;
-typedef const __attribute__((address_space(1))) f4 gf4;
-
-// row and k of unit u's first chunk within the stage
-template <int R, bool KC>
-__device__ __forceinline__ void unit_pos(int u, int &row, int &k) {
-    if constexpr (KC) {
-        row = u >> 2, k = (u & 3) * 4;
-    } else {
-        row = (u % (R / 4)) * 4, k = u / (R / 4);
-    }
-}
-
-// 4 floats at (row .. row + 3 or k .. k + 3), zero past the matrix; VEC: 16-byte aligned rows, so a
-// chunk wholly inside is one load
-template <bool KC, bool VEC>
-__device__ __forceinline__ f4 load4(const float *p, int64_t ld, int rows, int K, int row, int k) {
-    f4 v = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (KC) {
-        if (row >= rows || k >= K) return v;
-        gfloat *s = (gfloat *)(p + (int64_t)row * ld + k);
-        if (VEC && k + 4 <= K) return *(gf4 *)s;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (k + j < K) v[j] = s[j];
-    } else {
-        if (k >= K || row >= rows) return v;
-        gfloat *s = (gfloat *)(p + (int64_t)k * ld + row);
-        if (VEC && row + 4 <= rows) return *(gf4 *)s;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (row + j < rows) v[j] = s[j];
-    }
-    return v;
-}
-
+// ---- operand panels of the direct-to-LDS kernel ---------------------------------------------------
+// One stage of an operand: R rows (M or N) by 16 k in 16-byte chunks.
+//   * K-contiguous operand: rows of 64 bytes, logical chunk c of row r at chunk c ^ kc_swz(r), so the 16-byte
+//     fragment reads spread over all banks;
+//   * M/N-contiguous operand: 16 k-rows of R floats (R >= 64), the chunk of rows 4 c .. 4 c + 3 of k-row k at
+//     chunk c ^ mn_swz(k), so the four quarter-waves' fragment reads (k-rows k, k + 4, k + 8, k + 12 of 16
+//     consecutive rows) land in different banks.  Either layout is 64 R bytes per stage, with no padding, so
+//     a load straight into LDS fills it 1 KiB at a time.
 // The chunk permutation of K-contiguous panel row r (an XOR mask on its four 16-byte chunks).
 // (r >> 1) & 3 leaves the 16-byte fragment reads of the 16 rows and 4 quarter-waves free of bank
 // conflicts (SQ_LDS_BANK_CONFLICT reads 0; (r >> 2) & 3 read a third to a half of the LDS cycles).
@@ -142,19 +67,6 @@ __device__ __forceinline__ int kc_swz(int r) { return (r >> 1) & 3; }
 // so XOR-ing bits 2-3 of the chunk index with q puts the four quarters' 16 rows in four disjoint
 // groups of 16 banks (the 64 banks of 4 bytes, since a k-row's 4 R bytes are a multiple of 256).
 __device__ __forceinline__ int mn_swz(int k) { return ((k >> 2) & 3) << 2; }
-
-// LDS store of one chunk
-template <int R, bool KC>
-__device__ __forceinline__ void unit_store(char *slab, int u, f4 v) {
-    int row, k;
-    unit_pos<R, KC>(u, row, k);
-    if constexpr (KC) {
-        const int c = k >> 2;
-        *(f4 *)(slab + row * 64 + ((c ^ kc_swz(row)) << 4)) = v;
-    } else {
-        *(f4 *)(slab + k * R * 4 + (((row >> 2) ^ mn_swz(k)) << 4)) = v;
-    }
-}
 
 // The four values (s = 0..3) of panel row r that quarter-wave q gives the stage's MFMAs.
 template <int R, bool KC>
@@ -166,124 +78,6 @@ __device__ __forceinline__ f4 fragment(const char *slab, int r, int q) {
         const float *b = (const float *)slab + 4 * q * R + 4 * ((r >> 2) ^ (q << 2)) + (r & 3);
         return f4{b[0], b[R], b[2 * R], b[3 * R]};
     }
-}
-
-// One operand's stage loads: registers, FAST source pointers, load and store.
-template <int R, bool KC, int NT, bool VEC, bool FAST>
-struct Loader {
-    using P = Panel<R, KC, NT>;
-    f4 reg[P::UPT];
-    gfloat *src[FAST ? P::UPT : 1];
-    const float *p;
-    int64_t ld;
-    int rows, K, r0, t;
-
-    // FAST problems (aligned rows, K a multiple of 16, an M/N-contiguous operand's row count a
-    // multiple of 4): rows past the matrix are clamped onto its last row (last 4-row chunk), so every
-    // load is in bounds and unconditional; what those rows produce is never stored
-    __device__ __forceinline__ void init(const float *p_, int64_t ld_, int rows_, int K_, int r0_, int t_) {
-        p = p_, ld = ld_, rows = rows_, K = K_, r0 = r0_, t = t_;
-        if constexpr (FAST) {
-#pragma unroll
-            for (int i = 0; i < P::UPT; i++) {
-                int row, k;
-                unit_pos<R, KC>(t + i * NT, row, k);
-                row = KC ? min(r0 + row, rows - 1) : min(r0 + row, rows - 4);
-                src[i] = (gfloat *)(KC ? p + (int64_t)row * ld + k : p + (int64_t)k * ld + row);
-            }
-        }
-    }
-    __device__ __forceinline__ bool owns(int i) const { return !P::GUARD || t + i * NT < P::UNITS; }
-    __device__ __forceinline__ void load(int k0) {
-#pragma unroll
-        for (int i = 0; i < P::UPT; i++) {
-            if (!owns(i)) continue;
-            if constexpr (FAST) {
-                reg[i] = *(gf4 *)(src[i] + (KC ? k0 : (int64_t)k0 * ld));
-            } else {
-                int row, k;
-                unit_pos<R, KC>(t + i * NT, row, k);
-                reg[i] = load4<KC, VEC>(p, ld, rows, K, r0 + row, k0 + k);
-            }
-        }
-    }
-    __device__ __forceinline__ void store(char *slab) const {
-#pragma unroll
-        for (int i = 0; i < P::UPT; i++)
-            if (owns(i)) unit_store<R, KC>(slab, t + i * NT, reg[i]);
-    }
-};
-
-// element offset of batch matrix `idx` for operand o (0 A, 1 B, 2 C)
-__device__ __forceinline__ int64_t batch_off(const SgBatch &bt, int o, int64_t idx) {
-    int64_t off = 0;
-    for (int d = bt.nb - 1; d >= 0; d--) {
-        const int64_t e = bt.shape[d];
-        off += (idx % e) * bt.st[o][d];
-        idx /= e;
-    }
-    return off;
-}
-
-// The workgroup's tile: block -> (batch matrix, tile) with XCD-contiguous runs and groups of
-// kSgGroupM tile-rows; the batch matrix's operands.
-struct TileAt {
-    int m0, n0;
-    const float *A, *B;
-    float *C;
-};
-
-template <int BM, int BN>
-__device__ __forceinline__ TileAt locate(const SgArgs &p) {
-    int64_t id = blockIdx.x;
-    const int64_t nblk = gridDim.x;
-    if ((nblk & 7) == 0) id = (id & 7) * (nblk >> 3) + (id >> 3);
-    const int64_t per_batch = (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t batch = id / per_batch;
-    const int tile = (int)(id % per_batch);
-    const int per_group = kSgGroupM * p.tiles_n;
-    const int first_m = (tile / per_group) * kSgGroupM;
-    const int gsize = min(p.tiles_m - first_m, kSgGroupM);
-    TileAt at;
-    at.m0 = (first_m + (tile % per_group) % gsize) * BM;
-    at.n0 = ((tile % per_group) / gsize) * BN;
-    if (p.pa) {
-        at.A = p.pa[batch], at.B = p.pb[batch], at.C = p.pc[batch];
-    } else {
-        at.A = p.A + batch_off(p.bat, 0, batch), at.B = p.B + batch_off(p.bat, 1, batch);
-        at.C = p.C + batch_off(p.bat, 2, batch);
-    }
-    return at;
-}
-
-// The register-staged kernels keep a panel accumulator per tile beside the running totals: the
-// stage's fragments are read, its MFMAs (s = 0..3, the B fragment first: the tile is C^T, so each lane
-// ends up holding 4 consecutive columns of a row of C) add into the accumulators, and after a panel's
-// last stage the accumulators are added into the totals and cleared.
-template <class Cfg, bool AK, bool BK>
-__device__ __forceinline__ void stage_acc(const char *cur, f4 (&acc)[Cfg::TM][Cfg::TN], int wm, int wn, int fr, int fq) {
-    f4 a[Cfg::TM], b[Cfg::TN];
-#pragma unroll
-    for (int i = 0; i < Cfg::TM; i++) a[i] = fragment<Cfg::BM, AK>(cur, (wm * Cfg::TM + i) * 16 + fr, fq);
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; j++) b[j] = fragment<Cfg::BN, BK>(cur + Cfg::SLAB_A, (wn * Cfg::TN + j) * 16 + fr, fq);
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-#pragma unroll
-        for (int i = 0; i < Cfg::TM; i++)
-#pragma unroll
-            for (int j = 0; j < Cfg::TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j][s], a[i][s], acc[i][j], 0, 0, 0);
-}
-
-template <class Cfg>
-__device__ __forceinline__ void fold(f4 (&tot)[Cfg::TM][Cfg::TN], f4 (&acc)[Cfg::TM][Cfg::TN]) {
-#pragma unroll
-    for (int i = 0; i < Cfg::TM; i++)
-#pragma unroll
-        for (int j = 0; j < Cfg::TN; j++) {
-            tot[i][j] = tot[i][j] + acc[i][j];
-            acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-        }
 }
 
 // A wave's stores of one row block's final totals during the last panel: C row (tile row + fr) of row
@@ -364,90 +158,24 @@ __device__ __forceinline__ void panel_mfma(const char *c0, const char *c1, f4 (&
 }
 
 // C = alpha acc + beta C (+ bias[n]) over the wave's tiles.  acc[i][j] is the 16 x 16 tile C^T: lane l,
-// element v holds row (tile row + l % 16), column (tile column + 4 (l / 16) + v).  The bias is added to
-// the rounded alpha acc + beta C, as a separate broadcast add of it would.
+// element v holds row (tile row + l % 16), column (tile column + 4 (l / 16) + v).
 template <class Cfg>
 __device__ __forceinline__ void write_tiles(const SgArgs &p, const TileAt &at, const f4 (&acc)[Cfg::TM][Cfg::TN],
                                             int wm, int wn, int fr, int fq) {
-    constexpr int kTM = Cfg::TM, kTN = Cfg::TN;
-    const bool vec_c = ((uintptr_t)at.C & 15) == 0 && p.ldc % 4 == 0;
-    const bool vec_b = ((uintptr_t)p.bias & 15) == 0;
 #pragma unroll
-    for (int i = 0; i < kTM; i++) {
-        const int m = at.m0 + (wm * kTM + i) * 16 + fr;
+    for (int i = 0; i < Cfg::TM; i++) {
+        const int m = at.m0 + (wm * Cfg::TM + i) * 16 + fr;
         if (m >= p.M) continue;
-        float *crow = at.C + (int64_t)m * p.ldc;
 #pragma unroll
-        for (int j = 0; j < kTN; j++) {
-            const int n = at.n0 + (wn * kTN + j) * 16 + 4 * fq;
-            f4 r = p.alpha * acc[i][j];
-            if (vec_c && n + 4 <= p.N) {
-                f4 *c = (f4 *)(crow + n);
-                if (p.beta != 0.0f) r = r + p.beta * *c;
-                if (p.bias) {
-                    if (vec_b) r = r + *(const f4 *)(p.bias + n);
-                    else r = r + f4{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
-                }
-                *c = r;
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    if (n + v >= p.N) break;
-                    float *c = crow + n + v;
-                    const float t = p.beta != 0.0f ? r[v] + p.beta * *c : r[v];
-                    *c = p.bias ? t + p.bias[n + v] : t;
-                }
-            }
+        for (int j = 0; j < Cfg::TN; j++) {
+            const int n = at.n0 + (wn * Cfg::TN + j) * 16 + 4 * fq;
+            if (n < p.N) write4(p, at.C + (int64_t)m * p.ldc, n, acc[i][j]);
         }
     }
-}
-
-template <class Cfg, bool AK, bool BK, bool VEC, bool FAST>
-__global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void k_sgemm(SgArgs p) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const TileAt at = locate<Cfg::BM, Cfg::BN>(p);
-    const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
-    const int wm = wid / Cfg::WGN, wn = wid % Cfg::WGN, fr = lane & 15, fq = lane >> 4;
-
-    Loader<Cfg::BM, AK, Cfg::NT, VEC, FAST> la;
-    Loader<Cfg::BN, BK, Cfg::NT, VEC, FAST> lb;
-    la.init(at.A, p.lda, p.M, p.K, at.m0, t);
-    lb.init(at.B, p.ldb, p.N, p.K, at.n0, t);
-
-    f4 acc[Cfg::TM][Cfg::TN], tot[Cfg::TM][Cfg::TN];  // panel accumulators, running totals
-#pragma unroll
-    for (int i = 0; i < Cfg::TM; i++)
-#pragma unroll
-        for (int j = 0; j < Cfg::TN; j++) acc[i][j] = tot[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-
-    const int nk = (p.K + kSgBK - 1) / kSgBK;
-    if (nk > 0) {
-        la.load(0);
-        lb.load(0);
-        la.store(smem);
-        lb.store(smem + Cfg::SLAB_A);
-        __syncthreads();
-    }
-    for (int kt = 0; kt < nk; kt++) {
-        if (kt + 1 < nk) {
-            la.load((kt + 1) * kSgBK);
-            lb.load((kt + 1) * kSgBK);
-        }
-        stage_acc<Cfg, AK, BK>(smem + (kt & 1) * Cfg::STAGE, acc, wm, wn, fr, fq);
-        if (kt % kSgPanel == kSgPanel - 1 || kt + 1 == nk) fold<Cfg>(tot, acc);
-        // the other stage was last read before the previous barrier, so it can be refilled now
-        if (kt + 1 < nk) {
-            char *next = smem + ((kt + 1) & 1) * Cfg::STAGE;
-            la.store(next);
-            lb.store(next + Cfg::SLAB_A);
-        }
-        __syncthreads();
-    }
-    write_tiles<Cfg>(p, at, tot, wm, wn, fr, fq);
 }
 
 // ------------------------------------------------------------------------------------------------
-// Large FAST problems with K a multiple of 32: the 256 x 256 tile, its operand panels loaded straight
+// Large aligned problems with K a multiple of 32: the 256 x 256 tile, its operand panels loaded straight
 // from global memory into LDS (global_load_lds_dwordx4) a summation panel (two stages) ahead through
 // four LDS stages, with no staging registers and no LDS write instructions; one barrier per summation
 // panel.  A stage of an R-row panel is R / 16 load
@@ -455,7 +183,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MINB) void k_sgemm(SgArgs p) {
 // belongs at position l % 4 under the row's permutation) or 256 / R k-rows of a M/N-contiguous one
 // (lane l: k-row l / (R / 4), position l % (R / 4), loading the rows the k-row's permutation puts
 // there).  The 32 instructions of a stage (16 for A, 16 for B) are dealt four to a wave.  Rows past
-// the matrix are clamped as in the staged kernel's FAST loads.
+// the matrix are clamped onto its last row (last 4-row chunk), so every load is in bounds.
 constexpr int kSgDmaStages = 4;
 
 template <class Cfg>
@@ -554,31 +282,6 @@ __global__ __launch_bounds__(Cfg::NT, 1) void k_sgemm_dma(SgArgs p) {
     if (!stream_st) write_tiles<Cfg>(p, at, tot, wm, wn, fr, fq);
 }
 
-template <class Cfg, bool AK, bool BK, bool VEC, bool FAST>
-static void sg_attr() {
-    // dynamic LDS above 64 KiB has to be allowed per kernel, once per device
-    static bool done[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64 || done[dev]) return;
-    (void)hipFuncSetAttribute((const void *)k_sgemm<Cfg, AK, BK, VEC, FAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)Cfg::LDS);
-    done[dev] = true;
-}
-
-template <class Cfg, bool AK, bool BK, bool VEC, bool FAST>
-static int sg_launch(SgArgs &p, int64_t count, hipStream_t st, const char *what) {
-    p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
-    p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
-    const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * count;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
-    sg_attr<Cfg, AK, BK, VEC, FAST>();
-    hipLaunchKernelGGL((k_sgemm<Cfg, AK, BK, VEC, FAST>), dim3((unsigned)blocks), dim3(Cfg::NT), Cfg::LDS, st, p);
-    return check_launch(what);
-}
-
-#ifndef SG_DMA
-#define SG_DMA 1
-#endif
 template <class Cfg, bool AK, bool BK>
 static int sg_launch_dma(SgArgs &p, int64_t count, hipStream_t st, const char *what) {
     p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
@@ -596,39 +299,74 @@ static int sg_launch_dma(SgArgs &p, int64_t count, hipStream_t st, const char *w
     return check_launch(what);
 }
 
-// the register-staged kernels (128 x 128 and 64 x 64 tiles), by operand layout and load width
-template <class Cfg>
-static int sg_layouts(SgArgs &p, int ta, int tb, bool vec, bool fast, int64_t count, hipStream_t st, const char *what) {
-    const bool ak = !ta, bk = tb != 0;
-#define NC_SG_CASE(AK_, BK_)                                                                \
-    if (ak == AK_ && bk == BK_)                                                             \
-        return fast ? sg_launch<Cfg, AK_, BK_, true, true>(p, count, st, what)              \
-               : vec  ? sg_launch<Cfg, AK_, BK_, true, false>(p, count, st, what)           \
-                      : sg_launch<Cfg, AK_, BK_, false, false>(p, count, st, what);
-    NC_SG_CASE(true, true)
-    NC_SG_CASE(true, false)
-    NC_SG_CASE(false, true)
-    NC_SG_CASE(false, false)
-#undef NC_SG_CASE
-    return NC_HIP_OK;
-}
+// ------------------------------------------------------------------------------------------------
+// Which tile.  A problem's time on a tile shape is close to a0 + a1 P + L (s0 + s1 P) microseconds, with P its 32-k
+// panels and L the most tiles a CU of a 256-CU part gets: a the latency of a tile that has a CU to itself beyond its
+// share of the matrix cores, s what each tile adds.  The coefficients are least-squares fits (4% off on average, 17% at
+// most) of this kernel's times at L = 1, 2, 3, 4, 6 and K = 256, 2048, for 0, 1 and 2 operands that are M/N-contiguous;
+// the tiles are the ones that a choice by them over sizes from 1 to 8192 takes, and together cost 0.2% over the whole
+// family of shapes tried.  Small tiles split K over the waves of a workgroup: a product with few tiles still fills
+// the chip (x[8,4096] W[4096,4096]^T: 109 us on the 64 x 64 tile that was the smallest, 14 us on 16 x 16 with 16
+// waves).  The choice fixes how K is split, so it depends on the shape and layout alone: planned for kPlanCUs,
+// never for the device.
+struct SgTile {
+    int bm, bn;
+    float c[3][4];  // a0, a1, s0, s1 by M/N-contiguous operands
+};
+static const SgTile kSgTiles[] = {  // in the order of sg_tile_run
+    {128, 64, {{2.95f, 0.410f, 2.01f, 0.975f}, {3.65f, 0.459f, 1.36f, 1.032f}, {4.24f, 0.316f, 1.11f, 1.267f}}},
+    {96, 96, {{3.45f, 0.049f, 2.35f, 1.346f}, {2.94f, 0.089f, 3.19f, 1.353f}, {3.16f, 0.079f, 3.33f, 1.369f}}},
+    {96, 64, {{2.85f, 0.367f, 1.28f, 0.710f}, {3.25f, 0.330f, 1.25f, 0.810f}, {4.04f, 0.346f, 1.00f, 0.899f}}},
+    {96, 64, {{2.98f, 0.131f, 1.94f, 0.746f}, {2.29f, 0.039f, 2.53f, 0.949f}, {2.43f, 0.048f, 2.73f, 1.015f}}},
+    {64, 96, {{3.10f, 0.118f, 1.94f, 0.753f}, {2.11f, 0.026f, 2.88f, 0.981f}, {2.15f, 0.065f, 2.62f, 1.061f}}},
+    {64, 64, {{2.42f, 0.242f, 1.26f, 0.486f}, {2.90f, 0.227f, 0.95f, 0.561f}, {2.89f, 0.305f, 1.02f, 0.565f}}},
+    {64, 64, {{2.98f, 0.075f, 1.39f, 0.520f}, {2.86f, 0.113f, 1.41f, 0.582f}, {2.83f, 0.142f, 1.35f, 0.601f}}},
+    {64, 32, {{1.73f, 0.004f, 1.99f, 0.332f}, {2.00f, -0.002f, 1.82f, 0.386f}, {1.71f, 0.020f, 2.07f, 0.412f}}},
+    {32, 64, {{1.71f, 0.010f, 2.12f, 0.313f}, {1.82f, 0.012f, 1.96f, 0.390f}, {1.75f, 0.013f, 2.07f, 0.409f}}},
+    {32, 32, {{2.74f, 0.063f, 0.65f, 0.162f}, {2.67f, 0.064f, 0.65f, 0.192f}, {2.75f, 0.062f, 0.71f, 0.195f}}},
+    {32, 32, {{2.82f, -0.014f, 1.40f, 0.188f}, {2.19f, -0.004f, 1.73f, 0.218f}, {1.93f, 0.003f, 1.98f, 0.206f}}},
+    {32, 16, {{3.55f, -0.028f, 1.08f, 0.114f}, {3.12f, -0.024f, 1.30f, 0.137f}, {3.24f, -0.026f, 1.18f, 0.155f}}},
+    {16, 32, {{3.10f, -0.022f, 1.15f, 0.114f}, {3.37f, -0.023f, 1.21f, 0.135f}, {3.06f, -0.025f, 1.35f, 0.156f}}},
+    {16, 16, {{3.61f, -0.031f, 1.37f, 0.063f}, {3.65f, -0.034f, 1.43f, 0.086f}, {3.61f, -0.033f, 1.39f, 0.094f}}},
+};
+// The 256 x 256 direct-to-LDS kernel, one tile per CU at a time
+static const float kSgDma[4] = {3.0f, 0.0f, 8.3f, 8.05f};
 
 static int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// The 256 x 256 direct-to-LDS kernel for aligned problems (16-byte rows, K a multiple of 32: whole
-// summation panels) with at least a tile per CU; otherwise the largest register-staged tile that still
-// gives every CU a tile, else the smallest.
+static float sg_cost(const float *c, int64_t tiles, float panels) {
+    const float per_cu = (float)((tiles + kPlanCUs - 1) / kPlanCUs);
+    const float t = c[0] + c[1] * panels + per_cu * (c[2] + c[3] * panels);
+    return t > 4.5f ? t : 4.5f;  // a launch
+}
+
+// the cheapest tile's id, or -1 for the direct-to-LDS kernel (dma: the problem is one it takes)
+static int sg_pick(const SgArgs &p, bool ak, bool bk, bool dma, int64_t count) {
+    const float panels = (float)((p.K + 31) / 32);
+    const int mc = !ak + !bk;
+    int best = -1;
+    float least = dma ? sg_cost(kSgDma, tiles_of(p.M, p.N, SgBig::BM, SgBig::BN) * count, panels) : 3e38f;
+    for (int i = 0; i < (int)(sizeof(kSgTiles) / sizeof(kSgTiles[0])); i++) {
+        const SgTile &t = kSgTiles[i];
+        const float c = sg_cost(t.c[mc], tiles_of(p.M, p.N, t.bm, t.bn) * count, panels);
+        if (c < least) least = c, best = i;
+    }
+    return best;
+}
+
+// Runs the problem on the cheapest kernel for it; the direct-to-LDS one takes aligned problems (16-byte rows, K a
+// multiple of 32: whole summation panels).
 static int sg_run(SgArgs &p, int ta, int tb, int64_t count, hipStream_t st, const char *what) {
     // 16-byte loads need every matrix's rows 16-byte aligned: the matrices behind a pointer array may
-    // start anywhere, so those take the scalar loads
+    // start anywhere
     bool vec = !p.pa && aligned16(p.A) && aligned16(p.B) && p.lda % 4 == 0 && p.ldb % 4 == 0;
     for (int d = 0; d < p.bat.nb; d++) vec = vec && p.bat.st[0][d] % 4 == 0 && p.bat.st[1][d] % 4 == 0;
     const bool ak = !ta, bk = tb != 0;
-    const bool fast = vec && p.K % kSgBK == 0 && (ak || p.M % 4 == 0) && (bk || p.N % 4 == 0);
-    const int64_t cus = num_cus();
-    // the DMA kernel clamps M/N-contiguous chunks onto the last 4 rows: at least 4 rows there
-    const bool dma = SG_DMA && fast && p.K > 0 && p.K % (kSgBK * kSgPanel) == 0 && (ak || p.M >= 4) && (bk || p.N >= 4);
-    if (dma && tiles_of(p.M, p.N, SgBig::BM, SgBig::BN) * count >= cus) {
+    // M/N-contiguous chunks are clamped onto the last 4 rows: at least 4 rows there, and whole chunks
+    const bool dma = vec && p.K > 0 && p.K % (kSgBK * kSgPanel) == 0 && (ak || (p.M >= 4 && p.M % 4 == 0)) &&
+                     (bk || (p.N >= 4 && p.N % 4 == 0));
+    const int id = sg_pick(p, ak, bk, dma, count);
+    if (id < 0) {
 #define NC_SG_DMA(AK_, BK_) \
     if (ak == AK_ && bk == BK_) return sg_launch_dma<SgBig, AK_, BK_>(p, count, st, what);
         NC_SG_DMA(true, true)
@@ -637,9 +375,8 @@ static int sg_run(SgArgs &p, int ta, int tb, int64_t count, hipStream_t st, cons
         NC_SG_DMA(false, false)
 #undef NC_SG_DMA
     }
-    if (tiles_of(p.M, p.N, SgMid::BM, SgMid::BN) * count >= cus)
-        return sg_layouts<SgMid>(p, ta, tb, vec, fast, count, st, what);
-    return sg_layouts<SgSmall>(p, ta, tb, vec, fast, count, st, what);
+    if (ak) return bk ? sg_tile_nt(p, id, count, st, what) : sg_tile_nn(p, id, count, st, what);
+    return bk ? sg_tile_tt(p, id, count, st, what) : sg_tile_tn(p, id, count, st, what);
 }
 
 static bool fits_int(int64_t v) { return v >= 0 && v <= INT32_MAX; }
