@@ -279,6 +279,46 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds) {
 }
 #pragma clang diagnostic pop
 
+// ------------------------------------------------------------------------------------------------
+// Rows of any length and 4-byte alignment as 16-byte pieces: piece j is columns 4 j .. 4 j + 3, ceil(C / 4) of them, the
+// last one short where C is not a multiple of 4.  f4u is a 16-byte access at any 4-byte aligned address (one
+// dwordx4 instruction, as for an aligned one).
+// ------------------------------------------------------------------------------------------------
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// piece j of a row of C floats, `pad` in the places past its end; AL: the row is 16-byte aligned and C % 4 == 0
+template <bool AL>
+__device__ __forceinline__ f4 row_load(const float *row, int C, int j, float pad) {
+    if constexpr (AL) {
+        return __builtin_nontemporal_load((const f4 *)row + j);
+    } else {
+        if (4 * j + 4 <= C) return __builtin_nontemporal_load((const f4u *)(row + 4 * j));
+        f4 v = {pad, pad, pad, pad};
+#pragma unroll
+        for (int e = 0; e < 3; e++)
+            if (4 * j + e < C) v[e] = row[4 * j + e];
+        return v;
+    }
+}
+// the same, all pads for a piece past the row
+__device__ __forceinline__ f4 row_load_or(const float *row, int C, int j, float pad) {
+    return 4 * j < C ? row_load<false>(row, C, j, pad) : f4{pad, pad, pad, pad};
+}
+// A short piece shares its cache line with the next row's first one: rows that are not aligned are stored through
+// the caches, where the two meet, aligned ones past them.
+template <bool AL>
+__device__ __forceinline__ void row_store(f4 v, float *row, int C, int j) {
+    if constexpr (AL) {
+        __builtin_nontemporal_store(v, (f4 *)row + j);
+    } else if (4 * j + 4 <= C) {
+        *(f4u *)(row + 4 * j) = v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 3; e++)
+            if (4 * j + e < C) row[4 * j + e] = v[e];
+    }
+}
+
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 // ------------------------------------------------------------------------------------------------

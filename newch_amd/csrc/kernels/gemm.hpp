@@ -28,9 +28,7 @@ struct SgArgs {
     SgBatch bat;
 };
 
-// global-memory views, so loads are global_load (counted by vmcnt alone) rather than flat; f4u: 16 bytes
-// at any 4-byte aligned address (one global_load_dwordx4 either way on this target)
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+// global-memory views, so loads are global_load (counted by vmcnt alone) rather than flat
 typedef const __attribute__((address_space(1))) float gfloat;
 typedef const __attribute__((address_space(1))) f4 gf4;
 typedef const __attribute__((address_space(1))) f4u gf4u;

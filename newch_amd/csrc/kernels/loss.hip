@@ -12,12 +12,11 @@
 // terms, so the recomputed prob can differ from the probabilities the reference saves in its last
 // bits: the gradient matches the reference's at the reductions' tolerance, not bit for bit.
 //
-// cross entropy forward, one wave per row with the row in registers (C % 4 == 0, C <= 4096, 16-byte
-// aligned): the max, the row sum of exp(x - m) (hardware exponential: the sum is only compared at the
-// reductions' tolerance), logf, and the label's log-probability (its logit read back as one uniform
+// cross entropy forward, one wave per row with the row in registers (C <= 1024): the max, the row sum of
+// exp(x - m) (hardware exponential: the sum is only compared at the reductions' tolerance), logf, and the label's log-probability (its logit read back as one uniform
 // load rather than picked out of the registers) added to lane 0's fp64 accumulator.  The next row is
-// loaded before the current one is reduced.  Other
-// shapes: one workgroup per row, the same arithmetic over the (L2-resident) row.
+// loaded before the current one is reduced.  Longer rows: one workgroup per row, the same arithmetic, the row in
+// registers up to 65536 floats.
 //
 // Loss sums: fp64 per lane (or per thread), wave sums, workgroup partials added in wave order, and
 // one ordered combine (k_loss_finish): loss = -S / N (mean; NaN for N = 0, 0/0 as the reference) or
@@ -65,18 +64,23 @@ __device__ __forceinline__ void block_sum_min(double v, unsigned long long k, do
     }
 }
 
-template <int VPL>
+// AL: C % 4 == 0 and 16-byte aligned rows; otherwise the last piece's places past the row hold -inf, which the
+// maximum skips and whose exponential is 0
+template <int VPL, bool AL>
 __device__ __forceinline__ void ce_fwd_rows(const float *__restrict__ x, const int32_t *__restrict__ lab,
                                             f2 *__restrict__ stats, double *__restrict__ part,
                                             unsigned long long *__restrict__ badpart, int64_t N, int C) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int nv = C / 4;
+    const int nv = AL ? C / 4 : (C + 3) / 4;
     const int64_t stride = (int64_t)gridDim.x * kLWaves;
     auto load = [&](int64_t r, f4 *v) {
-        const f4 *xr = (const f4 *)(x + r * C);
+        const float *xr = x + r * C;
 #pragma unroll
-        for (int k = 0; k < VPL; k++)
-            if (lane + k * kWave < nv) v[k] = __builtin_nontemporal_load(xr + lane + k * kWave);
+        for (int k = 0; k < VPL; k++) {
+            if (lane + k * kWave >= nv) continue;
+            if constexpr (AL) v[k] = __builtin_nontemporal_load((const f4 *)xr + lane + k * kWave);
+            else v[k] = row_load<false>(xr, C, lane + k * kWave, -__builtin_inff());
+        }
     };
     // the label's logit, one wave-uniform 4-byte load (the row is in cache); an out-of-range label
     // reads column 0 and is not used
@@ -98,13 +102,15 @@ __device__ __forceinline__ void ce_fwd_rows(const float *__restrict__ x, const i
         m = row_max_finish(m, lane0_f32(v[0].x));  // lane 0 holds the row's first element
         // exp(x - m) as exp2((x - m) log2e): the difference first, so the exponent's error is relative
         // to x - m, not to m (x log2e - m log2e would carry m log2e's rounding, 1e-4 at |m| = 1e3); each
-        // lane's terms (at most 64, each in (0, 1]) in fp32, the 64 lane sums in fp64
-        float s = 0.0f;
+        // lane's terms (at most 64, each in (0, 1]) in fp32 on aligned rows and in fp64 on others, the 64 lane
+        // sums in fp64
+        using sum_t = std::conditional_t<AL, float, double>;
+        sum_t s = 0;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
             if (lane + k * kWave < nv)
-                s += (exp_sum_term(v[k].x - m) + exp_sum_term(v[k].y - m)) +
-                     (exp_sum_term(v[k].z - m) + exp_sum_term(v[k].w - m));
+                s += ((sum_t)exp_sum_term(v[k].x - m) + (sum_t)exp_sum_term(v[k].y - m)) +
+                     ((sum_t)exp_sum_term(v[k].z - m) + (sum_t)exp_sum_term(v[k].w - m));
         }
         const float ls = logf((float)wave_sum((double)s));
         if (lane == 0) {
@@ -162,22 +168,111 @@ __device__ __forceinline__ void ce_fwd_rows(const float *__restrict__ x, const i
 }
 
 // rows of up to 1024 floats: at most 64 VGPRs (8 waves per SIMD), so the grid of 8 workgroups per CU
-// is resident at once; longer rows keep the compiler's allocation
-template <int VPL>
+// is resident at once
+template <int VPL, bool AL>
 __global__ __attribute__((amdgpu_waves_per_eu(8, 8))) __launch_bounds__(kLB) void k_ce_fwd_reg(
     const float *__restrict__ x, const int32_t *__restrict__ lab, f2 *__restrict__ stats, double *__restrict__ part,
     unsigned long long *__restrict__ badpart, int64_t N, int C) {
-    ce_fwd_rows<VPL>(x, lab, stats, part, badpart, N, C);
+    ce_fwd_rows<VPL, AL>(x, lab, stats, part, badpart, N, C);
 }
 
+// Aligned rows of up to 4096 floats: the same with the compiler's register allocation
 template <int VPL>
 __global__ __launch_bounds__(kLB) void k_ce_fwd_reg_long(const float *__restrict__ x, const int32_t *__restrict__ lab,
                                                          f2 *__restrict__ stats, double *__restrict__ part,
                                                          unsigned long long *__restrict__ badpart, int64_t N, int C) {
-    ce_fwd_rows<VPL>(x, lab, stats, part, badpart, N, C);
+    ce_fwd_rows<VPL, true>(x, lab, stats, part, badpart, N, C);
 }
 
-// Any row length / alignment: one workgroup per row (rows in a grid-stride loop), the same
+// Other rows, up to 65536 floats of any length and alignment: a workgroup of NT threads per row, the row in
+// its registers (VPT 16-byte pieces a thread, read once), rows in a grid-stride loop; the row sum in fp64
+// throughout.  HBM-bound; the element-by-element two-pass kernel that longer rows still take ran [2048, 50257] in
+// 576 us, [4096, 6000] in 76 us (here 77 and 20).  With 1024 threads only one or two workgroups fit a CU, so a barrier
+// between the maximum and the sum would have all of them load, then all of them compute (90 us): EARLY, each wave
+// takes its own maximum m_w and sums exp(x - m_w) as soon as its part of the row is there, and wave 0 forms the
+// row's maximum m and the sum of s_w exp(m_w - m), in fp64 and wave order.  Smaller workgroups overlap as they are, and
+// the fp64 exponentials of the exchange would cost them more (16384 rows of 2048: 26 against 33 us); a second register
+// set with the next row requested ahead took their occupancy (32 us there).
+template <int VPT, int NT>
+__global__ __launch_bounds__(NT) void k_ce_fwd_wg(const float *__restrict__ x, const int32_t *__restrict__ lab,
+                                                  f2 *__restrict__ stats, double *__restrict__ part,
+                                                  unsigned long long *__restrict__ badpart, int64_t N, int C) {
+    constexpr int W = NT / kWave;
+    constexpr bool EARLY = NT >= 1024;
+    // the exchange slots alternate: a set is rewritten only after the next row's barrier
+    __shared__ float shm[2][W], sh0[2];
+    __shared__ double shs[2][W];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+    double acc = 0.0;  // thread 0: the negated log-probabilities of this workgroup's labels
+    unsigned long long mybad = kNoBad;
+    auto load = [&](int64_t r, f4 *v) {
+#pragma unroll
+        for (int k = 0; k < VPT; k++) v[k] = row_load_or(x + r * C, C, t + k * NT, -__builtin_inff());
+    };
+    auto row = [&](int64_t r, const f4 *v, int par) {
+        float m = -__builtin_inff();
+#pragma unroll
+        for (int k = 0; k < VPT; k++)
+            m = __builtin_fmaxf(m, __builtin_fmaxf(__builtin_fmaxf(v[k].x, v[k].y), __builtin_fmaxf(v[k].z, v[k].w)));
+        m = wave_max_nan_skip(m);
+        if (lane == 0) shm[par][wv] = m;
+        if (t == 0) sh0[par] = v[0].x;
+        if constexpr (EARLY) {
+            // a wave of nothing but -inf (and NaN): exp(x - 0) is 0 (NaN) for each, and its sum counts as it is
+            if (m == -__builtin_inff()) m = 0.0f;
+        } else {
+            lds_barrier();
+            m = shm[par][0];
+#pragma unroll
+            for (int i = 1; i < W; i++) m = __builtin_fmaxf(m, shm[par][i]);
+            m = row_max_finish(m, sh0[par]);
+        }
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < VPT; k++) {
+            if (4 * (t + k * NT) >= C) break;
+            s += ((double)exp_sum_term(v[k].x - m) + (double)exp_sum_term(v[k].y - m)) +
+                 ((double)exp_sum_term(v[k].z - m) + (double)exp_sum_term(v[k].w - m));
+        }
+        s = wave_sum(s);
+        if (lane == 0) shs[par][wv] = s;
+        lds_barrier();
+        if (wv != 0) return;
+        double tot = 0.0;
+        if constexpr (EARLY) {
+            const float mw = lane < W ? shm[par][lane] : -__builtin_inff();
+            m = row_max_finish(wave_max_nan_skip(mw), sh0[par]);
+            if (lane < W) {
+                tot = shs[par][lane];
+                if (mw != -__builtin_inff()) tot *= exp((double)mw - (double)m);
+                else if (m == mw) tot = __builtin_nan("");  // a row of -inf: x - m is NaN
+            }
+            tot = wave_sum(tot);
+        } else {
+#pragma unroll
+            for (int i = 0; i < W; i++) tot += shs[par][i];
+        }
+        if (lane == 0) {
+            const float ls = logf((float)tot);
+            const int32_t L = lab[r];
+            if (L >= 0 && L < C) acc -= (double)((x[r * C + L] - m) - ls);
+            else mybad = bad_key(r, L) < mybad ? bad_key(r, L) : mybad;
+            stats[r] = f2{m, ls};
+        }
+    };
+    int par = 0;
+    for (int64_t r = blockIdx.x; r < N; r += gridDim.x, par ^= 1) {
+        f4 v[VPT];
+        load(r, v);
+        row(r, v, par);
+    }
+    if (t == 0) {
+        part[blockIdx.x] = acc;
+        badpart[blockIdx.x] = mybad;
+    }
+}
+
+// Any row length: one workgroup per row (rows in a grid-stride loop), the same
 // statistics and label term; the row is re-read from L2 for the exp sum.
 __device__ __forceinline__ float block_max_nan_skip(float v, float *sh) {
     v = wave_max_nan_skip(v);
@@ -344,6 +439,49 @@ __global__ __launch_bounds__(kCeB) void k_ce_bwd4(const f4 *__restrict__ x, cons
     }
 }
 
+// The same for rows that are not a multiple of 4 long (C >= 4): a lane owns an aligned float4 of the whole [N, C] array,
+// whose elements belong to one row or to two neighbouring ones; the last n % 4 elements go one a lane.
+template <bool ACC>
+__global__ __launch_bounds__(kCeB) void k_ce_bwd4_any(const float *__restrict__ x, const f2 *__restrict__ stats,
+                                                      const int32_t *__restrict__ lab, const float *__restrict__ gout,
+                                                      float *__restrict__ gi, int64_t N, uint32_t n, IntDiv row) {
+    const float s = gout[0] / (float)(N ? N : 1);
+    const uint32_t e = (blockIdx.x * kCeB + threadIdx.x) * 4, C = row.d;
+    if (e >= n) return;
+    const uint32_t r = row.div(e), c = e - r * C;
+    const bool two = c + 4 > C && e + (C - c) < n;  // the item crosses into row r + 1
+    const f2 st0 = stats[r], st1 = two ? stats[r + 1] : st0;
+    const int32_t l0 = lab[r], l1 = two ? lab[r + 1] : -1;
+    const bool whole = e + 4 <= n;
+    f4 p = {0.f, 0.f, 0.f, 0.f}, o = {0.f, 0.f, 0.f, 0.f};
+    if (whole) {
+        p = __builtin_nontemporal_load((const f4 *)(x + e));
+        if (ACC) o = __builtin_nontemporal_load((const f4 *)(gi + e));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            if (e + j < n) {
+                p[j] = x[e + j];
+                if (ACC) o[j] = gi[e + j];
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const bool next = c + j >= C;
+        const int32_t col = (int32_t)(next ? c + j - C : c + j);
+        float v = o[j] + s * ce_prob(p[j], next ? st1 : st0);
+        if ((next ? l1 : l0) == col) v = v - s;
+        o[j] = v;
+    }
+    if (whole) {
+        __builtin_nontemporal_store(o, (f4 *)(gi + e));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            if (e + j < n) gi[e + j] = o[j];
+    }
+}
+
 template <bool ACC>
 __global__ __launch_bounds__(kLB) void k_ce_bwd1(const float *__restrict__ x, const f2 *__restrict__ stats,
                                                  const int32_t *__restrict__ lab, const float *__restrict__ gout,
@@ -368,18 +506,18 @@ __global__ __launch_bounds__(kLB) void k_nll_bwd(const int32_t *__restrict__ lab
     }
 }
 
-static int vpl_for_row(int64_t C) {
-    const int64_t nv = C / 4;
-    return nv <= 64 ? 1 : nv <= 128 ? 2 : nv <= 256 ? 4 : nv <= 512 ? 8 : nv <= 1024 ? 16 : 0;
-}
+// Rows of up to kCeWaveMax floats (aligned ones up to 4096): a wave per row; up to kCeWgMax: a workgroup per row, in
+// registers.  For 16384 rows of 2048 / 3072 / 4096 aligned floats the wave ran 26 / 36 / 55 us and the workgroup
+// 26 / 41 / 53; for 8192 rows of 2047 the workgroup 17 us, the element-by-element kernel 28.
+constexpr int64_t kCeWaveMax = 1024, kCeWgMax = 65536;
 
 #ifndef NC_CE_GRID_PER_CU
 #define NC_CE_GRID_PER_CU 8
 #endif
 // Both forwards write one fp64 loss partial per workgroup, so their grids are part of the summation
 // order: planned from the shape alone (kPlanCUs), never from the device's CU count.
-static unsigned ce_grid(int64_t N) {
-    const int64_t blocks = (N + kLWaves - 1) / kLWaves, cap = (int64_t)kPlanCUs * NC_CE_GRID_PER_CU;
+static unsigned ce_grid(int64_t N, bool wave) {
+    const int64_t blocks = wave ? (N + kLWaves - 1) / kLWaves : N, cap = (int64_t)kPlanCUs * NC_CE_GRID_PER_CU;
     return (unsigned)std::max<int64_t>(1, std::min(blocks, cap));
 }
 
@@ -389,16 +527,15 @@ static unsigned gather_grid(int64_t N) {
 }
 
 // workgroup partials of either forward: fp64 loss sums, then first-bad-row keys
-static int64_t loss_parts(int64_t N) { return std::max(ce_grid(N), gather_grid(N)); }
+static int64_t loss_parts(int64_t N, int64_t C) { return std::max(ce_grid(N, C <= kCeWaveMax), gather_grid(N)); }
 
 }  // namespace nchip
 
 using namespace nchip;
 
 extern "C" NC_HIP_API size_t nc_hip_loss_workspace(int64_t N, int64_t C) {
-    (void)C;
     if (N < 0) return 0;
-    return (size_t)loss_parts(N) * (sizeof(double) + sizeof(unsigned long long));
+    return (size_t)loss_parts(N, C) * (sizeof(double) + sizeof(unsigned long long));
 }
 
 extern "C" NC_HIP_API int nc_hip_cross_entropy_fwd(int64_t N, int64_t C, const float *x, const int32_t *lab,
@@ -415,20 +552,40 @@ extern "C" NC_HIP_API int nc_hip_cross_entropy_fwd(int64_t N, int64_t C, const f
     hipStream_t st = as_stream(stream);
     unsigned long long *b = (unsigned long long *)bad;
     double *part = (double *)ws;
-    unsigned long long *bp = (unsigned long long *)(part + loss_parts(N));
+    unsigned long long *bp = (unsigned long long *)(part + loss_parts(N, C));
     f2 *sv = (f2 *)stats;
     int nparts = 0;
     if (N > 0) {
-        const int vpl = (C % 4 == 0 && aligned16(x)) ? vpl_for_row(C) : 0;
-        const unsigned grid = ce_grid(N);
-        switch (vpl) {
-        case 1: hipLaunchKernelGGL(k_ce_fwd_reg<1>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C); break;
-        case 2: hipLaunchKernelGGL(k_ce_fwd_reg<2>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C); break;
-        case 4: hipLaunchKernelGGL(k_ce_fwd_reg<4>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C); break;
-        case 8: hipLaunchKernelGGL(k_ce_fwd_reg_long<8>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C); break;
-        case 16: hipLaunchKernelGGL(k_ce_fwd_reg_long<16>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C); break;
-        default: hipLaunchKernelGGL(k_ce_fwd_blk, grid, kLB, 0, st, x, lab, sv, part, bp, N, C); break;
-        }
+        const bool al = C % 4 == 0 && aligned16(x);
+        const unsigned grid = ce_grid(N, C <= kCeWaveMax || (al && C <= 4096));
+#define NC_CE_REG(VPL_)                                                                                                  \
+    do {                                                                                                                 \
+        if (al) hipLaunchKernelGGL((k_ce_fwd_reg<VPL_, true>), grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C);      \
+        else hipLaunchKernelGGL((k_ce_fwd_reg<VPL_, false>), grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C);        \
+    } while (0)
+#define NC_CE_WG(VPT_, NT_) hipLaunchKernelGGL((k_ce_fwd_wg<VPT_, NT_>), grid, NT_, 0, st, x, lab, sv, part, bp, N, (int)C)
+        if (C <= 256) NC_CE_REG(1);
+        else if (C <= 512) NC_CE_REG(2);
+        else if (C <= kCeWaveMax && al) hipLaunchKernelGGL((k_ce_fwd_reg<4, true>), grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C);
+        else if (C <= kCeWaveMax) NC_CE_WG(1, 256);  // the wave kernel's 64 registers do not hold an unaligned one
+        else if (C <= 2048 && al) hipLaunchKernelGGL(k_ce_fwd_reg_long<8>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C);
+        else if (C <= 4096 && al) hipLaunchKernelGGL(k_ce_fwd_reg_long<16>, grid, kLB, 0, st, x, lab, sv, part, bp, N, (int)C);
+        else if (C <= 2048) NC_CE_WG(2, 256);
+        else if (C <= 3072) NC_CE_WG(3, 256);
+        else if (C <= 4096) NC_CE_WG(4, 256);
+        else if (C <= 6144) NC_CE_WG(6, 256);
+        else if (C <= 8192) NC_CE_WG(8, 256);
+        else if (C <= 12288) NC_CE_WG(6, 512);
+        else if (C <= 16384) NC_CE_WG(8, 512);
+        else if (C <= 20480) NC_CE_WG(5, 1024);
+        else if (C <= 24576) NC_CE_WG(6, 1024);
+        else if (C <= 32768) NC_CE_WG(8, 1024);
+        else if (C <= 40960) NC_CE_WG(10, 1024);
+        else if (C <= 53248) NC_CE_WG(13, 1024);
+        else if (C <= kCeWgMax) NC_CE_WG(16, 1024);
+        else hipLaunchKernelGGL(k_ce_fwd_blk, grid, kLB, 0, st, x, lab, sv, part, bp, N, C);
+#undef NC_CE_REG
+#undef NC_CE_WG
         nparts = (int)grid;
     }
     hipLaunchKernelGGL(k_loss_finish, 1, kLB, 0, st, part, bp, nparts, N, 0, loss, b);
@@ -453,6 +610,13 @@ extern "C" NC_HIP_API int nc_hip_cross_entropy_bwd(int64_t N, int64_t C, const f
             hipLaunchKernelGGL(k_ce_bwd4<true>, grid, kCeB, 0, st, (const f4 *)x, sv, lab, gout, (f4 *)gi, N, n4, row4);
         else
             hipLaunchKernelGGL(k_ce_bwd4<false>, grid, kCeB, 0, st, (const f4 *)x, sv, lab, gout, (f4 *)gi, N, n4, row4);
+    } else if (C >= 4 && C <= INT32_MAX && aligned16(x) && aligned16(gi) && n < (int64_t)UINT32_MAX - 4 * kCeB) {
+        const unsigned grid = (unsigned)((n + 4 * kCeB - 1) / (4 * kCeB));
+        const IntDiv row((uint32_t)C);
+        if (accumulate)
+            hipLaunchKernelGGL(k_ce_bwd4_any<true>, grid, kCeB, 0, st, x, sv, lab, gout, gi, N, (uint32_t)n, row);
+        else
+            hipLaunchKernelGGL(k_ce_bwd4_any<false>, grid, kCeB, 0, st, x, sv, lab, gout, gi, N, (uint32_t)n, row);
     } else {
         const unsigned grid = stream_grid(n, kLB);
         if (accumulate) hipLaunchKernelGGL(k_ce_bwd1<true>, grid, kLB, 0, st, x, sv, lab, gout, gi, N, C);
@@ -472,7 +636,7 @@ extern "C" NC_HIP_API int nc_hip_nll_loss_fwd(int64_t N, int64_t C, const float 
     hipStream_t st = as_stream(stream);
     unsigned long long *b = (unsigned long long *)bad;
     double *part = (double *)ws;
-    unsigned long long *bp = (unsigned long long *)(part + loss_parts(N));
+    unsigned long long *bp = (unsigned long long *)(part + loss_parts(N, C));
     int nparts = 0;
     if (N > 0) {
         const unsigned grid = gather_grid(N);

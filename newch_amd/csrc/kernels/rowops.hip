@@ -1,8 +1,8 @@
 // Row kernels: softmax / log_softmax (ops_nn.c:22-71) and LayerNorm (ops_nn.c:434-522).
 //
-// A row of up to 4096 floats is held in registers by one wave64 (VPL 128-bit vectors per lane),
-// so each op reads its inputs from HBM exactly once and writes its outputs once; the row
-// statistics (max, sums) are wave64 shuffle reductions.  Longer or unaligned rows take a
+// A row is held in registers by one wave64 or one workgroup (VPL 128-bit vectors per lane), so each op
+// reads its inputs from HBM exactly once and writes its outputs once; the row statistics (max,
+// sums) are wave64 shuffle reductions.  The longest rows (and LayerNorm's unaligned ones) take a
 // workgroup-per-row path that re-reads the row from global memory (L2-resident) per pass.
 //
 // Per element the fp32 expressions are the reference's (exp8 for the softmax exponentials, the
@@ -21,17 +21,18 @@ constexpr int kWavesPerBlock = kRowB / kWave;
 // softmax, register-resident rows
 // ------------------------------------------------------------------------------------------------
 // One wave per row; the next row's loads are issued before the current row is reduced.
-template <int VPL, bool LOG>
+// AL: C % 4 == 0 and 16-byte aligned rows; otherwise the last piece's places past the row hold -inf, which the
+// maximum skips and whose exponential is 0.
+template <int VPL, bool LOG, bool AL>
 __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restrict__ x, float *__restrict__ y,
                                                            int64_t rows, int C) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int nv = C / 4;
+    const int nv = AL ? C / 4 : (C + 3) / 4;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
     auto load = [&](int64_t r, f4 *v) {
-        const f4 *xr = (const f4 *)(x + r * C);
 #pragma unroll
         for (int k = 0; k < VPL; k++)
-            if (lane + k * kWave < nv) v[k] = __builtin_nontemporal_load(xr + lane + k * kWave);
+            if (lane + k * kWave < nv) v[k] = row_load<AL>(x + r * C, C, lane + k * kWave, -__builtin_inff());
     };
     const int64_t r0 = ((int64_t)blockIdx.x * kRowB + threadIdx.x) / kWave;
     f4 v[VPL], vn[VPL];
@@ -47,14 +48,14 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
         m = wave_max_nan_skip(m);
         m = row_max_finish(m, lane0_f32(v[0].x));  // lane 0 holds the row's first element
         // the row sum: plain softmax needs exp8's values themselves (outputs); log_softmax only their
-        // sum, whose terms come from the hardware exponential (exp_sum_term)
+        // sum, whose terms come from the hardware exponential (exp_sum_term) on aligned rows
         double s = 0.0;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
             const int j = lane + k * kWave;
             if (j < nv) {
                 f4 e;
-                if (LOG) {
+                if (LOG && AL) {
                     e.x = exp_sum_term(v[k].x - m);
                     e.y = exp_sum_term(v[k].y - m);
                     e.z = exp_sum_term(v[k].z - m);
@@ -64,13 +65,13 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
                     e.y = exp8_nonpos(v[k].y - m);
                     e.z = exp8_nonpos(v[k].z - m);
                     e.w = exp8_nonpos(v[k].w - m);
-                    v[k] = e;
+                    if (!LOG) v[k] = e;
                 }
                 s += ((double)e.x + (double)e.y) + ((double)e.z + (double)e.w);
             }
         }
         const float sf = (float)wave_sum(s);
-        f4 *yr = (f4 *)(y + r * C);
+        float *yr = y + r * C;
         if (LOG) {
             const float ls = logf(sf);
 #pragma unroll
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
                     o.y = (v[k].y - m) - ls;
                     o.z = (v[k].z - m) - ls;
                     o.w = (v[k].w - m) - ls;
-                    __builtin_nontemporal_store(o, yr + j);
+                    row_store<AL>(o, yr, C, j);
                 }
             }
         } else {
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
                     o.y = inv * v[k].y;
                     o.z = inv * v[k].z;
                     o.w = inv * v[k].w;
-                    __builtin_nontemporal_store(o, yr + j);
+                    row_store<AL>(o, yr, C, j);
                 }
             }
         }
@@ -107,20 +108,19 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
 
 // One wave per row; the row's gi (when accumulating) and the next row's y, g are requested before
 // the current row is reduced.
-template <int VPL, bool LOG, bool ACC>
+template <int VPL, bool LOG, bool ACC, bool AL>
 __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restrict__ y, const float *__restrict__ g,
                                                            float *__restrict__ gi, int64_t rows, int C) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int nv = C / 4;
+    const int nv = AL ? C / 4 : (C + 3) / 4;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
     auto load = [&](int64_t r, f4 *vy, f4 *vg) {
-        const f4 *yr = (const f4 *)(y + r * C), *gr = (const f4 *)(g + r * C);
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
             const int j = lane + k * kWave;
             if (j < nv) {
-                vy[k] = __builtin_nontemporal_load(yr + j);
-                vg[k] = __builtin_nontemporal_load(gr + j);
+                vy[k] = row_load<AL>(y + r * C, C, j, 0.0f);
+                vg[k] = row_load<AL>(g + r * C, C, j, 0.0f);
             }
         }
     };
@@ -128,12 +128,12 @@ __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restri
     f4 vy[VPL], vg[VPL], ny[VPL], ng[VPL];
     if (r0 < rows) load(r0, vy, vg);
     for (int64_t r = r0; r < rows; r += stride) {
-        f4 *orow = (f4 *)(gi + r * C);
+        float *orow = gi + r * C;
         f4 go[VPL];
         if (ACC) {
 #pragma unroll
             for (int k = 0; k < VPL; k++)
-                if (lane + k * kWave < nv) go[k] = __builtin_nontemporal_load(orow + lane + k * kWave);
+                if (lane + k * kWave < nv) go[k] = row_load<AL>(orow, C, lane + k * kWave, 0.0f);
         }
         if (r + stride < rows) load(r + stride, ny, ng);
         double s = 0.0;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restri
                     o.z = o.z + vy[k].z * (vg[k].z - sf);
                     o.w = o.w + vy[k].w * (vg[k].w - sf);
                 }
-                __builtin_nontemporal_store(o, orow + j);
+                row_store<AL>(o, orow, C, j);
             }
         }
 #pragma unroll
@@ -238,6 +238,116 @@ __global__ __launch_bounds__(kRowB) void k_softmax_bwd_blk(const float *__restri
         __syncthreads();
     }
 }
+
+// Rows of more than 1024 floats (up to 65536), any length and alignment: a workgroup of NT threads per row, the row
+// in its registers (VPT 16-byte pieces a thread), so every input is read once.  The arithmetic is the wave
+// kernels'; the waves' maxima and sums meet in LDS and are combined in wave order.  HBM-bound: forward / backward of
+// [8192, 2047] 62 / 54 -> 25 / 37 us, [4096, 6000] 81 / 88 -> 36 / 52 us, [2048, 32000] 260 / 265 -> 112 / 145 us against the
+// element-by-element kernels that longer rows still take; [16384, 3072] 70 / 114 -> 69 / 104 us against a wave per row.
+template <int NT>
+__device__ __forceinline__ double wg_sum(double v, double *sh) {
+    v = wave_sum(v);
+    if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < NT / kWave; i++) t += sh[i];
+    return t;
+}
+
+template <int VPT, int NT, bool LOG>
+__global__ __launch_bounds__(NT) void k_softmax_fwd_wg(const float *__restrict__ x, float *__restrict__ y, int C) {
+    __shared__ double shd[NT / kWave];
+    __shared__ float shm[NT / kWave], sh0;
+    const int t = threadIdx.x;
+    const float *xr = x + (int64_t)blockIdx.x * C;
+    float *yr = y + (int64_t)blockIdx.x * C;
+    f4 v[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; k++) v[k] = row_load_or(xr, C, t + k * NT, -__builtin_inff());
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int k = 0; k < VPT; k++)
+        m = __builtin_fmaxf(m, __builtin_fmaxf(__builtin_fmaxf(v[k].x, v[k].y), __builtin_fmaxf(v[k].z, v[k].w)));
+    m = wave_max_nan_skip(m);
+    if ((t & (kWave - 1)) == 0) shm[t / kWave] = m;
+    if (t == 0) sh0 = v[0].x;
+    __syncthreads();
+    m = shm[0];
+#pragma unroll
+    for (int i = 1; i < NT / kWave; i++) m = __builtin_fmaxf(m, shm[i]);
+    m = row_max_finish(m, sh0);
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (4 * (t + k * NT) >= C) break;
+        f4 e;
+#pragma unroll
+        for (int c = 0; c < 4; c++) e[c] = exp8_nonpos(v[k][c] - m);
+        if (!LOG) v[k] = e;
+        s += ((double)e.x + (double)e.y) + ((double)e.z + (double)e.w);
+    }
+    const float sf = (float)wg_sum<NT>(s, shd);
+    const float ls = LOG ? logf(sf) : 0.0f, inv = LOG ? 0.0f : 1.0f / sf;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (4 * (t + k * NT) >= C) break;
+        f4 o;
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = LOG ? (v[k][c] - m) - ls : inv * v[k][c];
+        row_store<false>(o, yr, C, t + k * NT);
+    }
+}
+
+template <int VPT, int NT, bool LOG, bool ACC>
+__global__ __launch_bounds__(NT) void k_softmax_bwd_wg(const float *__restrict__ y, const float *__restrict__ g,
+                                                       float *__restrict__ gi, int C) {
+    __shared__ double shd[NT / kWave];
+    const int t = threadIdx.x;
+    const int64_t r0 = (int64_t)blockIdx.x * C;
+    f4 vy[VPT], vg[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        vy[k] = row_load_or(y + r0, C, t + k * NT, 0.0f);
+        vg[k] = row_load_or(g + r0, C, t + k * NT, 0.0f);
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        f4 e = vg[k];
+        if (!LOG) e = vg[k] * vy[k];
+        s += ((double)e.x + (double)e.y) + ((double)e.z + (double)e.w);
+    }
+    const float sf = (float)wg_sum<NT>(s, shd);
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (4 * (t + k * NT) >= C) break;
+        f4 o = ACC ? row_load<false>(gi + r0, C, t + k * NT, 0.0f) : f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            o[c] = LOG ? o[c] + (vg[k][c] - expf(vy[k][c]) * sf) : o[c] + vy[k][c] * (vg[k][c] - sf);
+        row_store<false>(o, gi + r0, C, t + k * NT);
+    }
+}
+
+// (pieces a thread, threads) of the workgroup kernels for a row length
+#define NC_WG_SWITCH(C, CALL)                                                            \
+    if ((C) <= 2048) { constexpr int VP = 2, NT = 256; CALL; }                           \
+    else if ((C) <= 3072) { constexpr int VP = 3, NT = 256; CALL; }                      \
+    else if ((C) <= 4096) { constexpr int VP = 4, NT = 256; CALL; }                      \
+    else if ((C) <= 6144) { constexpr int VP = 6, NT = 256; CALL; }                      \
+    else if ((C) <= 8192) { constexpr int VP = 8, NT = 256; CALL; }                      \
+    else if ((C) <= 12288) { constexpr int VP = 6, NT = 512; CALL; }                     \
+    else if ((C) <= 16384) { constexpr int VP = 8, NT = 512; CALL; }                     \
+    else if ((C) <= 20480) { constexpr int VP = 5, NT = 1024; CALL; }                    \
+    else if ((C) <= 24576) { constexpr int VP = 6, NT = 1024; CALL; }                    \
+    else if ((C) <= 32768) { constexpr int VP = 8, NT = 1024; CALL; }                    \
+    else if ((C) <= 40960) { constexpr int VP = 10, NT = 1024; CALL; }                   \
+    else if ((C) <= 53248) { constexpr int VP = 13, NT = 1024; CALL; }                   \
+    else { constexpr int VP = 16, NT = 1024; CALL; }
+// Rows of up to 1024 floats: a wave per row.  A ragged [65536, 197] ran 84 us forward element by element, 28 as a wave.
+constexpr int64_t kWaveRowMax = 1024, kWgRowMax = 65536;
+constexpr int64_t kWgRowMaxBwd = 32768;  // two rows in registers
 
 // ------------------------------------------------------------------------------------------------
 // LayerNorm
@@ -882,7 +992,7 @@ __global__ __launch_bounds__(kCombCols *kCombSlices) void k_ln_cols_combine(cons
 }
 
 static int vpl_for(int64_t C) {
-    const int64_t nv = C / 4;
+    const int64_t nv = (C + 3) / 4;
     if (nv <= 64) return 1;
     if (nv <= 128) return 2;
     if (nv <= 256) return 4;
@@ -990,10 +1100,18 @@ extern "C" NC_HIP_API int nc_hip_softmax_fwd(int log_form, int64_t rows, int64_t
     if (rows < 0 || C < 0) return set_error(NC_HIP_ERR_ARG, "nc_hip_softmax_fwd: negative size");
     if (rows == 0 || C == 0) return NC_HIP_OK;
     hipStream_t st = as_stream(stream);
-    const int v = (C % 4 == 0 && aligned16(x) && aligned16(y)) ? vpl_for(C) : 0;
-    if (v) {
-        if (log_form) NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_fwd_reg<VP, true>), rows_grid(rows), kRowB, 0, st, x, y, rows, (int)C))
-        else NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_fwd_reg<VP, false>), rows_grid(rows), kRowB, 0, st, x, y, rows, (int)C))
+    const bool al = C % 4 == 0 && aligned16(x) && aligned16(y);
+    const int v = C <= kWaveRowMax ? vpl_for(C) : 0;
+    if (v) {  // a wave per row
+#define NC_SM_FWD(LOG_, AL_) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_fwd_reg<VP, LOG_, AL_>), rows_grid(rows), kRowB, 0, st, x, y, rows, (int)C))
+        if (log_form && al) NC_SM_FWD(true, true)
+        else if (log_form) NC_SM_FWD(true, false)
+        else if (al) NC_SM_FWD(false, true)
+        else NC_SM_FWD(false, false)
+#undef NC_SM_FWD
+    } else if (C <= kWgRowMax && rows <= INT32_MAX) {  // a workgroup per row
+        if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, true>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
+        else NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, false>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         if (log_form) hipLaunchKernelGGL(k_softmax_fwd_blk<true>, grid, kRowB, 0, st, x, y, rows, C);
@@ -1007,13 +1125,26 @@ extern "C" NC_HIP_API int nc_hip_softmax_bwd(int log_form, int64_t rows, int64_t
     if (rows < 0 || C < 0) return set_error(NC_HIP_ERR_ARG, "nc_hip_softmax_bwd: negative size");
     if (rows == 0 || C == 0) return NC_HIP_OK;
     hipStream_t st = as_stream(stream);
-    const int v = (C % 4 == 0 && aligned16(y) && aligned16(g) && aligned16(gi)) ? vpl_for(C) : 0;
+    const bool al = C % 4 == 0 && aligned16(y) && aligned16(g) && aligned16(gi);
+    const int v = C <= kWaveRowMax ? vpl_for(C) : 0;
     const unsigned rg = rows_grid(rows);
     if (v) {
-        if (log_form && accumulate) NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, true, true>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))
-        else if (log_form) NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, true, false>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))
-        else if (accumulate) NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, false, true>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))
-        else NC_VPL_SWITCH(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, false, false>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))
+#define NC_SM_BWD(LOG_, ACC_)                                                                                                      \
+    do {                                                                                                                           \
+        if (al) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, LOG_, ACC_, true>), rg, kRowB, 0, st, y, g, gi, rows, (int)C)) \
+        else NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, LOG_, ACC_, false>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))   \
+    } while (0)
+        if (log_form && accumulate) NC_SM_BWD(true, true);
+        else if (log_form) NC_SM_BWD(true, false);
+        else if (accumulate) NC_SM_BWD(false, true);
+        else NC_SM_BWD(false, false);
+#undef NC_SM_BWD
+    } else if (C <= kWgRowMaxBwd && rows <= INT32_MAX) {
+        const dim3 grid((unsigned)rows);
+        if (log_form && accumulate) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, true>), grid, NT, 0, st, y, g, gi, (int)C))
+        else if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, false>), grid, NT, 0, st, y, g, gi, (int)C))
+        else if (accumulate) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, true>), grid, NT, 0, st, y, g, gi, (int)C))
+        else NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, false>), grid, NT, 0, st, y, g, gi, (int)C))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         if (log_form && accumulate) hipLaunchKernelGGL((k_softmax_bwd_blk<true, true>), grid, kRowB, 0, st, y, g, gi, rows, C);

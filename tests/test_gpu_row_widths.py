@@ -1,0 +1,130 @@
+"""Row kernels at the widths where they change form -- a wave or a workgroup per row, how many registers hold it -- with
+rows of 4-byte alignment and rows that hold infinities, NaN and the lowest floats, against fp64 and the oracle."""
+import numpy as np
+import pytest
+
+from newch_amd import hip, hipmem
+from oracle import pyoracle as O
+from tests.test_gpu_parity import assert_bits, assert_close64, ce_prob
+
+pytestmark = pytest.mark.gpu
+
+GUARD = np.float32(777.0)
+WIDTHS = [5, 255, 257, 513, 1023, 1025, 1028, 2047, 2052, 4095, 4097, 6145, 8191, 8196, 12289, 16383, 16385, 24577,
+          32767, 32769, 49153, 65535, 65537]
+
+
+@pytest.fixture(scope="module")
+def K():
+    return hip.Kernels()
+
+
+class Off:
+    """A float array on the device, `off` floats into its buffer, guard values on both sides."""
+
+    def __init__(self, a, off):
+        a = np.asarray(a, np.float32)
+        self.shape, self.n, self.off = a.shape, a.size, off
+        flat = np.full(a.size + off + 4, GUARD, np.float32)
+        flat[off:off + a.size] = a.ravel()
+        self.buf = hipmem.DeviceBuffer.from_numpy(flat)
+        self.ptr = self.buf.ptr + 4 * off
+
+    def read(self):
+        flat = self.buf.to_numpy(np.float32, self.n + self.off + 4)
+        assert (flat[:self.off] == GUARD).all() and (flat[self.off + self.n:] == GUARD).all(), "wrote outside"
+        return flat[self.off:self.off + self.n].reshape(self.shape)
+
+
+def logits(rng, rows, C):
+    x = (rng.standard_normal((rows, C)) * 3).astype(np.float32)
+    x[0, C - 1] = x[0].max() + 1  # the maximum in the row's last, short piece
+    x[1, C // 2] = -np.inf
+    x[2] = np.finfo(np.float32).min  # a row of the lowest float
+    return x
+
+
+@pytest.mark.parametrize("C", WIDTHS)
+@pytest.mark.parametrize("log_form", [False, True])
+def test_softmax_widths(K, C, log_form):
+    rng = np.random.default_rng(C + log_form)
+    rows = 6
+    x, g = logits(rng, rows, C), rng.standard_normal((rows, C)).astype(np.float32)
+    off = C % 3
+    print(f"softmax {rows}x{C} log={log_form} offset {off}", flush=True)
+    X, Y, G = Off(x, off), Off(np.zeros_like(x), off), Off(g, off)
+    K.softmax_fwd(log_form, rows, C, X.ptr, Y.ptr)
+    hipmem.synchronize()
+    y = Y.read()
+    x64 = x.astype(np.float64)
+    e = np.exp(x64 - x64.max(1, keepdims=True))
+    p = e / e.sum(1, keepdims=True)
+    with np.errstate(divide="ignore"):
+        want = np.log(p) if log_form else p
+    assert_close64(y, want, 1.0 if log_form else 0.0, "fwd")
+    G64 = g.astype(np.float64)
+    if log_form:
+        grad, sc = G64 - p * G64.sum(1, keepdims=True), np.abs(G64) + p * np.abs(G64).sum(1, keepdims=True)
+    else:
+        grad = p * (G64 - (G64 * p).sum(1, keepdims=True))
+        sc = p * (np.abs(G64) + (np.abs(G64) * p).sum(1, keepdims=True))
+    for acc in (False, True):
+        old = rng.standard_normal((rows, C)).astype(np.float32)
+        GI = Off(old, off)
+        K.softmax_bwd(log_form, rows, C, Y.ptr, G.ptr, GI.ptr, accumulate=acc)
+        hipmem.synchronize()
+        assert_close64(GI.read(), grad + (old if acc else 0), sc + (np.abs(old) if acc else 0), f"bwd acc={acc}")
+
+
+@pytest.mark.parametrize("C", [257, 1023, 1025, 4097, 16385, 50001])
+def test_softmax_special_rows(K, C):
+    """NaN first (the row is NaN), NaN later, all -inf, +inf: the reference's NaN pattern."""
+    rng = np.random.default_rng(C)
+    x = rng.standard_normal((5, C)).astype(np.float32)
+    x[0, 0], x[1, C - 1], x[2], x[3, 7] = np.nan, np.nan, -np.inf, np.inf
+    for log_form in (False, True):
+        X, Y = Off(x, 1), Off(np.zeros_like(x), 1)
+        K.softmax_fwd(log_form, 5, C, X.ptr, Y.ptr)
+        hipmem.synchronize()
+        y, ref = Y.read(), O.softmax_fwd(x, log_form)
+        assert (np.isnan(y) == np.isnan(ref)).all(), f"NaN pattern, log={log_form}"
+        assert_close64(y[4], ref[4].astype(np.float64), 1.0 if log_form else 0.0, "plain row")
+
+
+@pytest.mark.parametrize("C", WIDTHS + [4, 6, 1024, 50257])
+def test_cross_entropy_widths(K, C):
+    rng = np.random.default_rng(3 * C)
+    rows, off = 7, C % 2
+    x = logits(rng, rows, C)
+    lab = rng.integers(0, C, rows).astype(np.int32)
+    lab[0], lab[1], lab[3] = C - 1, 0, C - 1  # labels in a row's last and first piece
+    print(f"cross entropy {rows}x{C} offset {off}", flush=True)
+    X, S = Off(x, off), hipmem.DeviceBuffer(8 * rows)
+    L = hipmem.DeviceBuffer.from_numpy(lab)
+    loss, bad = hipmem.DeviceBuffer(4), hipmem.DeviceBuffer(8)
+    nws = K.loss_workspace(rows, C)
+    ws = hipmem.DeviceBuffer(nws)
+    K.cross_entropy_fwd(rows, C, X.ptr, L.ptr, S.ptr, loss.ptr, bad.ptr, ws.ptr, nws)
+    hipmem.synchronize()
+    assert bad.to_numpy(np.uint64, 1)[0] == np.uint64(0xFFFFFFFFFFFFFFFF)
+    # the terms as log(sum exp(x - m)) - (x_label - m): m + log(sum) would lose the log beside the lowest float
+    d = x.astype(np.float64) - x.astype(np.float64).max(1, keepdims=True)
+    terms = np.log(np.exp(d).sum(1)) - d[np.arange(rows), lab]
+    assert_close64(loss.to_numpy(np.float32, 1)[0], terms.mean(), np.abs(terms).sum() / rows ** 1.5, "loss")
+    prob = ce_prob(x, S.to_numpy(np.float32, (rows, 2)))
+    _, prob_o = O.cross_entropy_fwd(x, lab)
+    assert np.allclose(prob, prob_o, rtol=1e-5, atol=1e-30), "row statistics"
+    gout = np.float32(0.7)
+    GO = hipmem.DeviceBuffer.from_numpy(np.array([gout]))
+    for acc in (False, True):
+        old = rng.standard_normal((rows, C)).astype(np.float32)
+        for o2 in (off, 0):
+            GI = Off(old, o2)
+            K.cross_entropy_bwd(rows, C, X.ptr, S.ptr, L.ptr, GO.ptr, GI.ptr, accumulate=acc)
+            hipmem.synchronize()
+            assert_bits(GI.read(), O.cross_entropy_bwd(prob, lab, float(gout), old if acc else None), f"bwd acc={acc}")
+    lab[5] = C  # out of range: reported, and contributes nothing
+    L2 = hipmem.DeviceBuffer.from_numpy(lab)
+    K.cross_entropy_fwd(rows, C, X.ptr, L2.ptr, S.ptr, loss.ptr, bad.ptr, ws.ptr, nws)
+    hipmem.synchronize()
+    assert bad.to_numpy(np.uint64, 1)[0] == np.uint64((5 << 32) | C)
