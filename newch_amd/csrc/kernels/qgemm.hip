@@ -15,12 +15,14 @@
 // 0-31 with k 0-15, lanes 32-63 the same rows with k 16-31) for A and for B alike, so whatever order
 // the instruction sums a lane's bytes in, A and B pair the same k.  Large problems run 256 x 256
 // tiles (8 waves of 4 x 2 MFMA tiles, BK 128, 147 KiB of LDS), smaller ones 128 x 128 (4 waves of
-// 2 x 2, BK 64).  Large problems with K a multiple of 128 and 16-byte aligned rows take k_qgemm_dma
-// instead: the same tile over 16 waves, its panels loaded straight into LDS one 128-byte k step ahead.
-// When K is also a multiple of 256, k_qgemm_pipe runs that tile over 8 waves with the k loop written
-// as one software-pipelined assembly block (below).  Blocks are remapped so each XCD (blocks b with
-// b % 8 equal) works a contiguous run of tiles, and tiles run in groups of 8 tile-rows so neighbouring
-// blocks share panels in L2.
+// 2 x 2, BK 64), and problems too small to fill the chip with those split K over a workgroup's waves instead
+// (k_qgemm_ks).  Rows that are not 16-byte aligned are loaded with 16-byte loads all the same
+// (2500^3: 400 us byte by byte, 60 so).  Large problems with K a multiple of 128 and 16-byte
+// aligned rows take k_qgemm_dma instead: the same tile over 16 waves, its panels loaded straight
+// into LDS one 128-byte k step ahead. When K is also a multiple of 256, k_qgemm_pipe runs that tile
+// over 8 waves with the k loop written as one software-pipelined assembly block (below).  Blocks
+// are remapped so each XCD (blocks b with b % 8 equal) works a contiguous run of tiles, and tiles
+// run in groups of 8 tile-rows so neighbouring blocks share panels in L2.
 //
 // linear_int8 epilogue (ops_quant.c:75-79): y = (float)acc * xs[m] * ws[n] + (bias ? bias[n] : 0),
 // evaluated left to right in fp32 without contraction (the reference's scalar glue), so the fused
@@ -67,6 +69,18 @@ struct QgArgs {
     const float *bias; // [N] or null
 };
 
+typedef int i4u __attribute__((ext_vector_type(4), aligned(1)));
+
+// 16 bytes of a row from r, column k; those from column K on are zeros and not read
+__device__ __forceinline__ i4 row16(const int8_t *r, int k, int K) {
+    if (k + 16 <= K) return (i4) * (const i4u *)r;
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int b = 0; b < 16; b++)
+        if (k + b < K) w[b >> 2] |= (uint32_t)(uint8_t)r[b] << (8 * (b & 3));
+    return i4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+
 // 16 k-bytes of row `row` starting at column k (zeros past the matrix)
 template <bool ALIGNED>
 __device__ __forceinline__ i4 load16(const int8_t *p, int64_t ld, int row, int rows, int k, int K) {
@@ -76,11 +90,7 @@ __device__ __forceinline__ i4 load16(const int8_t *p, int64_t ld, int row, int r
     if (ALIGNED) {
         if (k < K) v = *(const i4 *)r;
     } else {
-        uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int b = 0; b < 16; b++)
-            if (k + b < K) w[b >> 2] |= (uint32_t)(uint8_t)r[b] << (8 * (b & 3));
-        v = i4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        v = row16(r, k, K);
     }
     return v;
 }
@@ -638,12 +648,187 @@ static int launch_qgemm_cfg(QgArgs p, bool out_f32, hipStream_t st, const char *
     return check_launch(what);
 }
 
+// ------------------------------------------------------------------------------------------------
+// Problems with few tiles: a workgroup owns a (16 TM) x (16 TN) tile and its KS waves split K, each wave's part
+// straight from global memory into registers (no LDS, no barrier in the k loop); the waves' int32 sums meet in LDS
+// once, exact in any order.  K advances 128 bytes a wave and step (wave w: steps w, w + KS, ...), two
+// v_mfma_i32_16x16x64_i8 per tile, the next step's rows loaded before the current one is multiplied.  Lane l of a
+// 16-row fragment holds 16 k bytes of row l % 16 at 16 (l / 16), for A and B alike; the B fragment goes first, so
+// the tiles are C^T and a lane holds 4 consecutive columns of row l % 16.  Rows may start at any byte: 16-byte loads
+// at any alignment, byte by byte only where K ends inside them.  With few rows the weight's bytes are the bound, and
+// what decides is how many of them are in flight on all CUs: 16 x 4096 x 4096 went from 39.4 us (32 tiles of 128 x 128,
+// K a serial chain) to 6.3, 6 x 2384 x 6243 (no row aligned, bytes loaded one by one) from 492 to 14.
+// ------------------------------------------------------------------------------------------------
+template <int TM_, int TN_, int KS_>
+struct QkCfg {
+    static constexpr int TM = TM_, TN = TN_, KS = KS_, NT = 64 * KS_, BM = 16 * TM_, BN = 16 * TN_;
+};
+
+template <class C, bool OUT_F32>
+__global__ __launch_bounds__(C::NT) void k_qgemm_ks(QgArgs p) {
+    constexpr int TM = C::TM, TN = C::TN, KS = C::KS;
+    __shared__ i4 red[KS > 1 ? KS * TM * TN * kWave : 1];
+    const uint32_t nblk = gridDim.x, x = blockIdx.x & 7, per = nblk >> 3, rem = nblk & 7;
+    const int id = (int)(x * per + min(x, rem) + (blockIdx.x >> 3));  // XCD x: the x-th of 8 runs of tiles
+    const int m0 = (id % p.tiles_m) * C::BM, n0 = (id / p.tiles_m) * C::BN;
+    const int lane = threadIdx.x & (kWave - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int fr = lane & 15, fq = lane >> 4;
+
+    const int8_t *pa[TM], *pb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++) pa[i] = p.A + (int64_t)min(m0 + 16 * i + fr, p.M - 1) * p.lda + 16 * fq;
+#pragma unroll
+    for (int j = 0; j < TN; j++) pb[j] = p.B + (int64_t)min(n0 + 16 * j + fr, p.N - 1) * p.ldb + 16 * fq;
+    struct Step {
+        i4 a[TM][2], b[TN][2];
+    };
+    auto load = [&](int k, Step &s) {  // k: the step's first byte, a whole step inside K
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) s.a[i][h] = *(const i4u *)(pa[i] + k + 64 * h);
+#pragma unroll
+            for (int j = 0; j < TN; j++) s.b[j][h] = *(const i4u *)(pb[j] + k + 64 * h);
+        }
+    };
+    i4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = i4{0, 0, 0, 0};
+    auto work = [&](const Step &s) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(s.b[j][h], s.a[i][h], acc[i][j], 0, 0, 0);
+    };
+    const int whole = p.K / 128 * 128;
+    int k = wid * 128;
+    Step u, v;
+    if (k < whole) load(k, u);
+    while (k < whole) {
+        if (k + 128 * KS < whole) load(k + 128 * KS, v);
+        work(u);
+        k += 128 * KS;
+        if (k >= whole) break;
+        if (k + 128 * KS < whole) load(k + 128 * KS, u);
+        work(v);
+        k += 128 * KS;
+    }
+    if (whole < p.K && wid == whole / 128 % KS) {  // the step K ends inside, by the wave whose turn it is
+        Step s;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) s.a[i][h] = row16(pa[i] + whole + 64 * h, whole + 64 * h + 16 * fq, p.K);
+#pragma unroll
+            for (int j = 0; j < TN; j++) s.b[j][h] = row16(pb[j] + whole + 64 * h, whole + 64 * h + 16 * fq, p.K);
+        }
+        work(s);
+    }
+    auto put = [&](int i, int j, i4 c) {
+        const int m = m0 + 16 * i + fr, n = n0 + 16 * j + 4 * fq;
+        if (m >= p.M) return;
+        const int64_t at = (int64_t)m * p.ldc + n;
+        if (OUT_F32) {
+            const float xs = p.xs[m];
+            f4 y;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int ne = min(n + e, p.N - 1);
+                y[e] = (float)c[e] * xs * p.ws[ne] + (p.bias ? p.bias[ne] : 0.0f);
+            }
+            if (n + 4 <= p.N) {
+                *(f4u *)(p.Y + at) = y;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 3; e++)
+                    if (n + e < p.N) p.Y[at + e] = y[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (n + e < p.N) p.C[at + e] = c[e];
+        }
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) put(i, j, acc[i][j]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) red[(wid * TM * TN + i * TN + j) * kWave + lane] = acc[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if ((i * TN + j) % KS != wid) continue;  // the waves share out the tiles
+                i4 c = red[(i * TN + j) * kWave + lane];
+#pragma unroll
+                for (int w = 1; w < KS; w++) c = c + red[(w * TM * TN + i * TN + j) * kWave + lane];
+                put(i, j, c);
+            }
+    }
+}
+
+template <class C>
+static int launch_qgemm_ks(QgArgs p, bool out_f32, hipStream_t st, const char *what) {
+    p.tiles_m = (p.M + C::BM - 1) / C::BM;
+    p.tiles_n = (p.N + C::BN - 1) / C::BN;
+    const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
+    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
+    if (out_f32) hipLaunchKernelGGL((k_qgemm_ks<C, true>), dim3((unsigned)blocks), dim3(C::NT), 0, st, p);
+    else hipLaunchKernelGGL((k_qgemm_ks<C, false>), dim3((unsigned)blocks), dim3(C::NT), 0, st, p);
+    return check_launch(what);
+}
+
+// Which kernel: the one that the costs below call the cheapest, in ns over K bytes for a CU's share of the tiles.
+// The sums are exact in any order, so the choice may follow the device's CU count.  Measured, us (one box):
+//   M x N x K          16x16  16x32  32x32  64x32  64x64  128x128
+//   16 x 4096 x 4096     6.3    8.1    8.5    9.7   13.4    39.4
+//   16 x 8192 x 8192    17.7   14.4   15.2   17.0   23.8    79.9
+//   64 x 4096 x 4096    17.3   14.3   10.3   14.4   18.6    40.1
+//   128 x 4096 x 4096   31.9   26.8   18.3   15.0   19.2    41.6
+//   512 x 4096 x 4096    113     98     61     50     37      46
+//   1024 x 4096 x 4096   224    195    120    100     71      50
+// The split-K tiles go by what they load: (BM + BN) K bytes a tile at about 36 bytes a ns and CU, and the two
+// largest, of which a CU holds one workgroup, by each tile's start and end (1024 x 4096 x 1024: 28.4 against 17.0).
+// The 128 x 128 tile waits for its panels while a CU has one (10 ns a byte of K) and takes 6.2 when two share it; a
+// 256 x 256 tile 17.
 static int launch_qgemm(QgArgs p, bool out_f32, hipStream_t st, const char *what) {
+    const auto rounds = [&](int bm, int bn) {
+        const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+        return (double)((tiles + num_cus() - 1) / num_cus());
+    };
+    const auto ks = [&](int bm, int bn, int tile) {
+        return 4000 + rounds(bm, bn) * (tile + (double)(bm + bn) * p.K / 36);
+    };
     const int64_t big_tiles = (int64_t)((p.M + QgBig::BM - 1) / QgBig::BM) * ((p.N + QgBig::BN - 1) / QgBig::BN);
+    const bool big = big_tiles >= num_cus();
+    const double r128 = rounds(QgSmall::BM, QgSmall::BN);
+    const double wide = 5000 + (double)p.K * (big ? 17 * rounds(QgBig::BM, QgBig::BN) : r128 > 1 ? 6.2 * r128 : 10);
+    const double c[5] = {ks(16, 16, 0), ks(16, 32, 0), ks(32, 32, 0), ks(64, 32, 800), ks(64, 64, 2000)};
+    int best = 0;
+    for (int i = 1; i < 5; i++)
+        if (c[i] < c[best]) best = i;
+    if (c[best] < wide) switch (best) {
+        case 0: return launch_qgemm_ks<QkCfg<1, 1, 16>>(p, out_f32, st, what);
+        case 1: return launch_qgemm_ks<QkCfg<1, 2, 16>>(p, out_f32, st, what);
+        case 2: return launch_qgemm_ks<QkCfg<2, 2, 8>>(p, out_f32, st, what);
+        case 3: return launch_qgemm_ks<QkCfg<4, 2, 8>>(p, out_f32, st, what);
+        default: return launch_qgemm_ks<QkCfg<4, 4, 4>>(p, out_f32, st, what);
+        }
     const bool dma_ok = p.K > 0 && p.K % kDmaBK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) &&
                         aligned16(p.B);
-    if (big_tiles >= num_cus() && dma_ok) return launch_qgemm_dma(p, out_f32, st, what);
-    if (big_tiles >= num_cus()) return launch_qgemm_cfg<QgBig>(p, out_f32, st, what);
+    if (big && dma_ok) return launch_qgemm_dma(p, out_f32, st, what);
+    if (big) return launch_qgemm_cfg<QgBig>(p, out_f32, st, what);
     return launch_qgemm_cfg<QgSmall>(p, out_f32, st, what);
 }
 

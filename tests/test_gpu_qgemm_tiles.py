@@ -1,0 +1,73 @@
+"""The int8 product at the edges of its tiles, K splits and alignments: whole numbers, so equal to the 64-bit product
+bit for bit; the fused linear equal to its own steps in fp32."""
+import numpy as np
+import pytest
+
+from newch_amd import hip, hipmem
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): every tile (16x16, 16x32, 32x32, 64x32, 64x64 with K over the waves, 128x128, 256x256), one past and one
+# short of it; K within a step, a whole number of steps, short of and past a wave's turn, unaligned rows
+SHAPES = [(1, 1, 1), (1, 17, 15), (15, 16, 16), (16, 16, 127), (17, 15, 128), (3, 100, 129), (16, 4096, 2048),
+          (1, 4100, 2049), (16, 8200, 1031), (33, 4090, 260), (64, 4096, 1000), (127, 4096, 520), (129, 4099, 333),
+          (257, 4097, 640), (512, 4096, 250), (1000, 4000, 384), (1030, 4100, 77), (4100, 4090, 65),
+          (4097, 4096, 128), (5, 70000, 129), (31, 33, 6243), (16, 64, 0)]
+
+
+GUARD = -7
+
+
+@pytest.fixture(scope="module")
+def K():
+    return hip.Kernels()
+
+
+def ints(rng, rows, cols):
+    return rng.integers(-127, 128, (rows, cols), dtype=np.int8)
+
+
+def placed(a, ld, off):
+    """`a` on the device, rows `ld` bytes apart from byte `off` of its buffer."""
+    flat = np.full(off + a.shape[0] * ld + 1, 99, np.int8)
+    flat[off:off + a.shape[0] * ld].reshape(a.shape[0], ld)[:, :a.shape[1]] = a
+    return hipmem.DeviceBuffer.from_numpy(flat)
+
+
+def product(a, b):
+    return (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.int32)
+
+
+@pytest.mark.parametrize("M,N,Kd", SHAPES)
+@pytest.mark.parametrize("pad,off", [(0, 0), (5, 3)])
+def test_gemm_s8_exact(K, M, N, Kd, pad, off):
+    rng = np.random.default_rng(M + N + Kd)
+    a, b = ints(rng, M, Kd), ints(rng, N, Kd)
+    lda, ldb, ldc = Kd + pad, Kd + 2 * pad, N + pad
+    da, db = placed(a, lda, off), placed(b, ldb, off)
+    dc = hipmem.DeviceBuffer.from_numpy(np.full(M * ldc + 4, GUARD, np.int32))
+    K.gemm_s8_nt(M, N, Kd, da.ptr + off, lda, db.ptr + off, ldb, dc.ptr, ldc)
+    flat = dc.to_numpy(np.int32, M * ldc + 4)
+    c = flat[:M * ldc].reshape(M, ldc)
+    np.testing.assert_array_equal(c[:, :N], product(a, b))
+    assert (c[:, N:] == GUARD).all() and (flat[M * ldc:] == GUARD).all(), "wrote outside"
+
+
+@pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (7, 515, 130), (16, 4096, 512), (40, 4097, 257), (130, 4098, 129),
+                                    (300, 4095, 384)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_linear_int8_equals_its_steps(K, M, N, Kd, bias):
+    rng = np.random.default_rng(M + N + Kd)
+    x = rng.standard_normal((M, Kd)).astype(np.float32)
+    w, ws = ints(rng, N, Kd), (rng.random(N) + 0.5).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32) if bias else np.zeros(N, np.float32)
+    dx, dw, dws, db = (hipmem.DeviceBuffer.from_numpy(v) for v in (x, w, ws, b))
+    dy = hipmem.DeviceBuffer.from_numpy(np.zeros((M, N), np.float32))
+    n = K.linear_int8_workspace(M, Kd)
+    scratch = hipmem.DeviceBuffer.from_numpy(np.zeros(n, np.int8))
+    K.linear_int8(M, Kd, N, dx.ptr, dw.ptr, dws.ptr, db.ptr if bias else None, dy.ptr, scratch.ptr, n)
+    dq, ds = (hipmem.DeviceBuffer.from_numpy(v) for v in (np.zeros((M, Kd), np.int8), np.zeros(M, np.float32)))
+    K.quantize_rows(M, Kd, dx.ptr, dq.ptr, ds.ptr)
+    q, s = dq.to_numpy(np.int8, M * Kd).reshape(M, Kd), ds.to_numpy(np.float32, M)
+    want = product(q, w).astype(np.float32) * s[:, None] * ws + b
+    np.testing.assert_array_equal(dy.to_numpy(np.float32, M * N).reshape(M, N), want)
