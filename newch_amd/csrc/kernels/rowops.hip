@@ -352,27 +352,48 @@ constexpr int64_t kWgRowMaxBwd = 32768;  // two rows in registers
 // ------------------------------------------------------------------------------------------------
 // LayerNorm
 // ------------------------------------------------------------------------------------------------
+// piece j of gamma / beta, kept in the caches (every row reads it); zeros past the end
+template <bool AL>
+__device__ __forceinline__ f4 vec_load(const float *p, int D, int j) {
+    if constexpr (AL) return ((const f4 *)p)[j];
+    if (4 * j + 4 <= D) return *(const f4u *)(p + 4 * j);
+    f4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+        if (4 * j + e < D) v[e] = p[4 * j + e];
+    return v;
+}
+
+// the squared deviations of a piece, of its first `left` elements where the row ends in it
+template <bool AL>
+__device__ __forceinline__ double ln_sq_dev(f4 v, double mean, int left) {
+    double d[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) d[c] = AL || c < left ? (double)v[c] - mean : 0.0;
+    return (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
+}
+
 // One wave per row; gamma / beta are held in registers and the next row's loads are issued before
-// the current row is reduced.
-template <int VPL>
+// the current row is reduced.  AL: every pointer 16-byte aligned and rows of whole pieces.
+template <int VPL, bool AL>
 __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ x, const float *__restrict__ w,
                                                       const float *__restrict__ b, float eps, float *__restrict__ y,
                                                       float *__restrict__ stats, int64_t rows, int D) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int nv = D / 4;
+    const int nv = (D + 3) / 4;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
     f4 ww[VPL], bv[VPL];
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
         const int j = lane + k * kWave;
-        ww[k] = (w && j < nv) ? ((const f4 *)w)[j] : f4{0.f, 0.f, 0.f, 0.f};
-        bv[k] = (b && j < nv) ? ((const f4 *)b)[j] : f4{0.f, 0.f, 0.f, 0.f};
+        ww[k] = (w && j < nv) ? vec_load<AL>(w, D, j) : f4{0.f, 0.f, 0.f, 0.f};
+        bv[k] = (b && j < nv) ? vec_load<AL>(b, D, j) : f4{0.f, 0.f, 0.f, 0.f};
     }
     auto load = [&](int64_t r, f4 *v) {
-        const f4 *xr = (const f4 *)(x + r * D);
+        const float *xr = x + r * D;
 #pragma unroll
         for (int k = 0; k < VPL; k++)
-            if (lane + k * kWave < nv) v[k] = __builtin_nontemporal_load(xr + lane + k * kWave);
+            if (lane + k * kWave < nv) v[k] = row_load<AL>(xr, D, lane + k * kWave, 0.0f);
     };
     const int64_t r0 = ((int64_t)blockIdx.x * kRowB + threadIdx.x) / kWave;
     f4 v[VPL], vn[VPL];
@@ -388,11 +409,7 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
         double ss = 0.0;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
-            if (lane + k * kWave < nv) {
-                const double a = (double)v[k].x - mean, bb = (double)v[k].y - mean, c = (double)v[k].z - mean,
-                             d = (double)v[k].w - mean;
-                ss += (a * a + bb * bb) + (c * c + d * d);
-            }
+            if (lane + k * kWave < nv) ss += ln_sq_dev<AL>(v[k], mean, D - 4 * (lane + k * kWave));
         }
         ss = wave_sum(ss);
         const float rstd = (float)(1.0 / sqrt(ss / (double)D + (double)eps));
@@ -401,7 +418,7 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
             stats[2 * r] = mf;
             stats[2 * r + 1] = rstd;
         }
-        f4 *yr = (f4 *)(y + r * D);
+        float *yr = y + r * D;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
             const int j = lane + k * kWave;
@@ -412,7 +429,7 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
                 t = (v[k].y - mf) * rstd; o.y = (w ? t * ww[k].y : t) + bv[k].y;
                 t = (v[k].z - mf) * rstd; o.z = (w ? t * ww[k].z : t) + bv[k].z;
                 t = (v[k].w - mf) * rstd; o.w = (w ? t * ww[k].w : t) + bv[k].w;
-                __builtin_nontemporal_store(o, yr + j);
+                row_store<AL>(o, yr, D, j);
             }
         }
 #pragma unroll
@@ -420,6 +437,51 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
     }
 }
 
+// Rows of more than 1024 floats (up to 65536), any length and alignment: a workgroup of NT threads per row, the row in
+// its registers, so x is read once where k_ln_fwd_blk reads it three times.  HBM-bound: [16384, 3001] 223 ->
+// 73 us, [16384, 8192] 574 -> 192 (5.6 TB/s); [16384, 4096] 102 -> 90 against a wave per row.
+template <int VPT, int NT>
+__global__ __launch_bounds__(NT) void k_ln_fwd_wg(const float *__restrict__ x, const float *__restrict__ w,
+                                                  const float *__restrict__ b, float eps, float *__restrict__ y,
+                                                  float *__restrict__ stats, int D) {
+    __shared__ double sh[2][NT / kWave];
+    const int t = threadIdx.x;
+    const float *xr = x + (int64_t)blockIdx.x * D;
+    float *yr = y + (int64_t)blockIdx.x * D;
+    f4 v[VPT];
+#pragma unroll
+    for (int k = 0; k < VPT; k++) v[k] = row_load_or(xr, D, t + k * NT, 0.0f);
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) s += ((double)v[k].x + (double)v[k].y) + ((double)v[k].z + (double)v[k].w);
+    const double mean = wg_sum<NT>(s, sh[0]) / (double)D;
+    double ss = 0.0;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) ss += ln_sq_dev<false>(v[k], mean, D - 4 * (t + k * NT));
+    ss = wg_sum<NT>(ss, sh[1]);
+    const float rstd = (float)(1.0 / sqrt(ss / (double)D + (double)eps));
+    const float mf = (float)mean;
+    if (t == 0) {
+        stats[2 * (int64_t)blockIdx.x] = mf;
+        stats[2 * (int64_t)blockIdx.x + 1] = rstd;
+    }
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        const int j = t + k * NT;
+        if (4 * j >= D) break;
+        const f4 ww = w ? vec_load<false>(w, D, j) : f4{1.f, 1.f, 1.f, 1.f};
+        const f4 bv = b ? vec_load<false>(b, D, j) : f4{0.f, 0.f, 0.f, 0.f};
+        f4 o;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float u = (v[k][c] - mf) * rstd;
+            o[c] = (w ? u * ww[c] : u) + bv[c];
+        }
+        row_store<false>(o, yr, D, j);
+    }
+}
+
+// rows past 65536 floats
 __global__ __launch_bounds__(kRowB) void k_ln_fwd_blk(const float *__restrict__ x, const float *__restrict__ w,
                                                       const float *__restrict__ b, float eps, float *__restrict__ y,
                                                       float *__restrict__ stats, int64_t rows, int64_t D) {
@@ -452,31 +514,24 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_blk(const float *__restrict__ 
 // Backward, register rows.  Each workgroup (8 waves) owns a contiguous range of rows; its waves take
 // rows round-robin.  Per row, the gx loads (when accumulating) and then the next row's x and g are
 // requested before the row is reduced.  The gw / gb column partials of a wave's rows accumulate in
-// fp32 in that wave's own LDS slice (rows up to 1024 floats; registers for longer rows), in row
+// fp32 in that wave's own LDS slice, in row
 // order; at the end each column's 8 wave partials are added in wave order in fp64 and written as
 // the workgroup's partial, which k_ln_cols_combine adds up in a fixed order.
 constexpr int kLnB = 512;
 constexpr int kLnWaves = kLnB / kWave;
 
-template <int VPL>
-constexpr bool ln_cols_in_lds() { return VPL <= 4; }
-
 // bytes of dynamic LDS k_ln_bwd_reg needs for gw / gb
-static size_t ln_bwd_lds(int vpl, int64_t D, bool cols) {
-    if (!cols) return 0;
-    return vpl <= 4 ? (size_t)kLnWaves * 2 * D * sizeof(float) : (size_t)2 * D * sizeof(double);
-}
+static size_t ln_bwd_lds(int64_t D, bool cols) { return cols ? (size_t)kLnWaves * 2 * D * sizeof(float) : 0; }
 
-// rows up to 1024 floats: two workgroups per CU (at most 128 VGPRs); longer rows: one
+// two workgroups per CU: at most 128 VGPRs
 template <int VPL, bool ACC>
-__global__ __launch_bounds__(kLnB, VPL <= 4 ? 4 : 2) void k_ln_bwd_reg(const float *__restrict__ x, const float *__restrict__ w,
+__global__ __launch_bounds__(kLnB, 4) void k_ln_bwd_reg(const float *__restrict__ x, const float *__restrict__ w,
                                                      const float *__restrict__ stats, const float *__restrict__ g,
                                                      float *__restrict__ gx, double *__restrict__ part, int64_t rows,
                                                      int D, int64_t rows_per_block) {
     extern __shared__ char ln_lds[];
     // gamma staged in LDS: its reads then wait on the LDS counter, not behind the prefetched row
     __shared__ f4 wsh[VPL * kWave];
-    constexpr bool kLdsCols = ln_cols_in_lds<VPL>();
     const int lane = threadIdx.x & (kWave - 1);
     const int wv = threadIdx.x / kWave;
     const int nv = D / 4;
@@ -487,20 +542,14 @@ __global__ __launch_bounds__(kLnB, VPL <= 4 ? 4 : 2) void k_ln_bwd_reg(const flo
         for (int j = threadIdx.x; j < nv; j += kLnB) wsh[j] = ((const f4 *)w)[j];
         __syncthreads();
     }
-    // column accumulators: this wave's LDS slice [2][D] floats, or registers
+    // column accumulators: this wave's LDS slice [2][D] floats
     f4 *accw = (f4 *)ln_lds + (size_t)wv * 2 * nv, *accb = accw + nv;
-    f4 aw[kLdsCols ? 1 : VPL], ab[kLdsCols ? 1 : VPL];
-    if constexpr (kLdsCols) {
-        if (cols) {
+    if (cols) {
 #pragma unroll
-            for (int k = 0; k < VPL; k++) {
-                const int j = lane + k * kWave;
-                if (j < nv) accw[j] = accb[j] = f4{0.f, 0.f, 0.f, 0.f};
-            }
+        for (int k = 0; k < VPL; k++) {
+            const int j = lane + k * kWave;
+            if (j < nv) accw[j] = accb[j] = f4{0.f, 0.f, 0.f, 0.f};
         }
-    } else {
-#pragma unroll
-        for (int k = 0; k < VPL; k++) aw[k] = ab[k] = f4{0.f, 0.f, 0.f, 0.f};
     }
     auto load = [&](int64_t r, f4 *xv, f4 *gv) {
         const f4 *xr = (const f4 *)(x + r * D), *gr = (const f4 *)(g + r * D);
@@ -513,22 +562,20 @@ __global__ __launch_bounds__(kLnB, VPL <= 4 ? 4 : 2) void k_ln_bwd_reg(const flo
             }
         }
     };
-    constexpr bool kPrefetch = VPL <= 4;  // longer rows have no registers for the next row
-    f4 xv4[VPL], gg[VPL], xn[kPrefetch ? VPL : 1], gn[kPrefetch ? VPL : 1];
-    if (kPrefetch && r0 + wv < r1) load(r0 + wv, xv4, gg);
+    f4 xv4[VPL], gg[VPL], xn[VPL], gn[VPL];
+    if (r0 + wv < r1) load(r0 + wv, xv4, gg);
     for (int64_t r = r0 + wv; r < r1; r += kLnWaves) {
         f4 *dx = gx ? (f4 *)(gx + r * D) : nullptr;
         // the row's statistics, then its gx, then the next row: waits for the first two do not
         // wait for the prefetch
         const float mean = stats[2 * r], rstd = stats[2 * r + 1];
-        if (!kPrefetch) load(r, xv4, gg);
         f4 go[VPL];
         if (ACC && dx) {
 #pragma unroll
             for (int k = 0; k < VPL; k++)
                 if (lane + k * kWave < nv) go[k] = __builtin_nontemporal_load(dx + lane + k * kWave);
         }
-        if (kPrefetch && r + kLnWaves < r1) load(r + kLnWaves, xn, gn);
+        if (r + kLnWaves < r1) load(r + kLnWaves, xn, gn);
         // xhat = (x - mean) * rstd and gw = g * w, recomputed (same fp32 operations) in the second
         // pass rather than held live across the row reductions
         auto terms = [&](int k, int j, f4 &xh, f4 &gw) {
@@ -553,19 +600,14 @@ __global__ __launch_bounds__(kLnB, VPL <= 4 ? 4 : 2) void k_ln_bwd_reg(const flo
                 sgx += ((double)(gw4.x * xh.x) + (double)(gw4.y * xh.y)) +
                        ((double)(gw4.z * xh.z) + (double)(gw4.w * xh.w));
                 if (cols) {
-                    f4 t = kLdsCols ? accw[j] : aw[k], u = kLdsCols ? accb[j] : ab[k];
+                    f4 t = accw[j], u = accb[j];
                     t.x += gg[k].x * xh.x;
                     t.y += gg[k].y * xh.y;
                     t.z += gg[k].z * xh.z;
                     t.w += gg[k].w * xh.w;
                     u += gg[k];
-                    if constexpr (kLdsCols) {
-                        accw[j] = t;
-                        accb[j] = u;
-                    } else {
-                        aw[k] = t;
-                        ab[k] = u;
-                    }
+                    accw[j] = t;
+                    accb[j] = u;
                 }
             }
         }
@@ -588,51 +630,22 @@ __global__ __launch_bounds__(kLnB, VPL <= 4 ? 4 : 2) void k_ln_bwd_reg(const flo
                 }
             }
         }
-        if constexpr (kPrefetch) {
 #pragma unroll
-            for (int k = 0; k < VPL; k++) {
-                xv4[k] = xn[k];
-                gg[k] = gn[k];
-            }
+        for (int k = 0; k < VPL; k++) {
+            xv4[k] = xn[k];
+            gg[k] = gn[k];
         }
     }
     if (!cols) return;
     double *out = part + (size_t)blockIdx.x * 2 * D;
-    if constexpr (kLdsCols) {
-        // column i of [gw | gb]: the 8 wave slices added in wave order
-        __syncthreads();
-        const float *acc = (const float *)ln_lds;
-        for (int i = threadIdx.x; i < 2 * D; i += kLnB) {
-            double t = 0.0;
+    // column i of [gw | gb]: the 8 wave slices added in wave order
+    __syncthreads();
+    const float *acc = (const float *)ln_lds;
+    for (int i = threadIdx.x; i < 2 * D; i += kLnB) {
+        double t = 0.0;
 #pragma unroll
-            for (int w8 = 0; w8 < kLnWaves; w8++) t += (double)acc[(size_t)w8 * 2 * D + i];
-            out[i] = t;
-        }
-    } else {
-        // combine the waves' register partials in LDS (wave order)
-        double *lds = (double *)ln_lds;  // [2][D]
-        for (int i = threadIdx.x; i < 2 * D; i += kLnB) lds[i] = 0.0;
-        __syncthreads();
-        for (int wsel = 0; wsel < kLnWaves; wsel++) {
-            if (wv == wsel) {
-#pragma unroll
-                for (int k = 0; k < VPL; k++) {
-                    const int j = lane + k * kWave;
-                    if (j < nv) {
-                        lds[4 * j + 0] += aw[k].x;
-                        lds[4 * j + 1] += aw[k].y;
-                        lds[4 * j + 2] += aw[k].z;
-                        lds[4 * j + 3] += aw[k].w;
-                        lds[D + 4 * j + 0] += ab[k].x;
-                        lds[D + 4 * j + 1] += ab[k].y;
-                        lds[D + 4 * j + 2] += ab[k].z;
-                        lds[D + 4 * j + 3] += ab[k].w;
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        for (int i = threadIdx.x; i < 2 * D; i += kLnB) out[i] = lds[i];
+        for (int w8 = 0; w8 < kLnWaves; w8++) t += (double)acc[(size_t)w8 * 2 * D + i];
+        out[i] = t;
     }
 }
 
@@ -910,6 +923,155 @@ __global__ __launch_bounds__(kLnPairWaves *kWave, 4) void k_ln_bwd_pair(const fl
     }
 }
 
+// Backward of rows that are not whole aligned float4s, and of any row past 1024 floats (up to 12288): a row is held by a
+// team of TW waves, VPT 16-byte pieces of x and of g a lane, the next row's pieces on the way while it is reduced.
+// TW = 1: eight waves a workgroup, each with its own rows; else the workgroup is the team, the waves' fp64 sums meet in
+// LDS (two sets of slots in turn, so one barrier a row) and are added in wave order.  A lane keeps the gw / gb
+// partials of its columns over the workgroup's rows in fp64 registers, as the element-by-element kernels do;
+// k_ln_cols_combine adds the workgroups'.  HBM-bound: [16384, 767] 57 -> 44 us, [16384, 3001]
+// 270 -> 136, [16384, 8192] 735 -> 341 (4.7 TB/s) against those; [16384, 2048] 113 -> 80 against a wave per row.
+constexpr int ln_team_threads(int tw) { return tw == 1 ? kLnB : tw * kWave; }
+
+template <int VPT, int TW, bool ACC>
+__global__ __launch_bounds__(ln_team_threads(TW), 4) void k_ln_bwd_team(const float *__restrict__ x,
+                                                                        const float *__restrict__ w,
+                                                                        const float *__restrict__ stats,
+                                                                        const float *__restrict__ g,
+                                                                        float *__restrict__ gx,
+                                                                        double *__restrict__ part, int64_t rows, int D) {
+    constexpr int NT = ln_team_threads(TW), NL = TW * kWave, kTeams = NT / NL;
+    __shared__ double slot[2][TW == 1 ? 1 : TW][2];
+    const int t = TW == 1 ? (int)threadIdx.x % kWave : (int)threadIdx.x;  // lane of the team
+    const int wv = threadIdx.x / kWave;
+    const bool cols = part != nullptr;
+    double aw[VPT][4], ab[VPT][4];
+#pragma unroll
+    for (int k = 0; k < VPT; k++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) aw[k][c] = ab[k][c] = 0.0;
+    f4 xv[VPT], gv[VPT], xn[VPT], gn[VPT];
+    auto load = [&](int64_t r, f4 *xs, f4 *gs) {
+#pragma unroll
+        for (int k = 0; k < VPT; k++) {
+            xs[k] = row_load_or(x + r * D, D, t + k * NL, 0.0f);
+            gs[k] = row_load_or(g + r * D, D, t + k * NL, 0.0f);
+        }
+    };
+    int64_t r = (int64_t)blockIdx.x * kTeams + (TW == 1 ? wv : 0);
+    const int64_t step = (int64_t)gridDim.x * kTeams;
+    if (r < rows) load(r, xv, gv);
+    for (int par = 0; r < rows; r += step, par ^= 1) {
+        const float mean = stats[2 * r], rstd = stats[2 * r + 1];
+        f4 old[VPT];
+        if (ACC && gx) {
+#pragma unroll
+            for (int k = 0; k < VPT; k++) old[k] = row_load_or(gx + r * D, D, t + k * NL, 0.0f);
+        }
+        if (r + step < rows) load(r + step, xn, gn);
+        f4 ww[VPT];
+        double sg = 0.0, sgx = 0.0;
+#pragma unroll
+        for (int k = 0; k < VPT; k++) {
+            const int j = t + k * NL;
+            ww[k] = w && 4 * j < D ? vec_load<false>(w, D, j) : f4{1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float xh = (xv[k][c] - mean) * rstd, gw = gv[k][c] * ww[k][c];
+                sg += (double)gw;
+                sgx += (double)(gw * xh);
+                if (cols) {
+                    aw[k][c] += (double)(gv[k][c] * xh);
+                    ab[k][c] += (double)gv[k][c];
+                }
+            }
+        }
+        if (gx) {
+            sg = wave_sum(sg);
+            sgx = wave_sum(sgx);
+            if constexpr (TW > 1) {
+                if (t % kWave == 0) {
+                    slot[par][wv][0] = sg;
+                    slot[par][wv][1] = sgx;
+                }
+                __syncthreads();
+                sg = sgx = 0.0;
+#pragma unroll
+                for (int i = 0; i < TW; i++) {
+                    sg += slot[par][i][0];
+                    sgx += slot[par][i][1];
+                }
+            }
+            const float mg = (float)(sg / (double)D), mgx = (float)(sgx / (double)D);
+#pragma unroll
+            for (int k = 0; k < VPT; k++) {
+                const int j = t + k * NL;
+                if (4 * j >= D) break;
+                f4 o;
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const float xh = (xv[k][c] - mean) * rstd, gw = gv[k][c] * ww[k][c];
+                    o[c] = (ACC ? old[k][c] : 0.0f) + rstd * ((gw - mg) - xh * mgx);
+                }
+                row_store<false>(o, gx + r * D, D, j);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < VPT; k++) {
+            xv[k] = xn[k];
+            gv[k] = gn[k];
+        }
+    }
+    if (!cols) return;
+    double *out = part + (size_t)blockIdx.x * 2 * D;
+    if constexpr (TW > 1) {
+#pragma unroll
+        for (int k = 0; k < VPT; k++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int i = 4 * (t + k * NL) + c;
+                if (i < D) {
+                    out[i] = aw[k][c];
+                    out[D + i] = ab[k][c];
+                }
+            }
+    } else {  // the waves' partials, added in wave order
+        __shared__ double sums[2][TW == 1 ? 4 * VPT * kWave : 1];
+        for (int sel = 0; sel < kTeams; sel++) {
+            if (wv == sel) {
+#pragma unroll
+                for (int k = 0; k < VPT; k++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const int i = c * VPT * kWave + t + k * kWave;  // lanes on neighbouring banks
+                        sums[0][i] = sel ? sums[0][i] + aw[k][c] : aw[k][c];
+                        sums[1][i] = sel ? sums[1][i] + ab[k][c] : ab[k][c];
+                    }
+            }
+            __syncthreads();
+        }
+        for (int i = threadIdx.x; i < D; i += NT) {
+            const int at = (i % 4) * VPT * kWave + i / 4;
+            out[i] = sums[0][at];
+            out[D + i] = sums[1][at];
+        }
+    }
+}
+
+// (pieces a lane, waves) of the team for a row length.  Wider teams with fewer pieces a lane wait more at their barriers:
+// one piece a lane took 146 us at [16384, 3072] where three take 120, though 29 where they take 32 at 2000 rows.
+#define NC_LN_TEAM_SWITCH(D, CALL)                                  \
+    if ((D) <= 256) { constexpr int VP = 1, TW = 1; CALL; }         \
+    else if ((D) <= 512) { constexpr int VP = 2, TW = 1; CALL; }    \
+    else if ((D) <= 768) { constexpr int VP = 3, TW = 1; CALL; }    \
+    else if ((D) <= 1024) { constexpr int VP = 4, TW = 1; CALL; }   \
+    else if ((D) <= 2048) { constexpr int VP = 2, TW = 4; CALL; }   \
+    else if ((D) <= 3072) { constexpr int VP = 3, TW = 4; CALL; }   \
+    else if ((D) <= 4096) { constexpr int VP = 2, TW = 8; CALL; }   \
+    else if ((D) <= 6144) { constexpr int VP = 3, TW = 8; CALL; }   \
+    else if ((D) <= 8192) { constexpr int VP = 2, TW = 16; CALL; }  \
+    else { constexpr int VP = 3, TW = 16; CALL; }
+constexpr int64_t kLnTeamMax = 12288;
+
 // Generic backward: one workgroup per row for gx, and column partials for gw/gb.
 template <bool ACC>
 __global__ __launch_bounds__(kRowB) void k_ln_bwd_blk(const float *__restrict__ x, const float *__restrict__ w,
@@ -1019,15 +1181,6 @@ static unsigned rows_grid(int64_t rows) {
     return (unsigned)(blocks < cap ? blocks : cap);
 }
 
-#define NC_VPL_SWITCH(V, CALL)                      \
-    switch (V) {                                    \
-    case 1: { constexpr int VP = 1; CALL; } break;  \
-    case 2: { constexpr int VP = 2; CALL; } break;  \
-    case 4: { constexpr int VP = 4; CALL; } break;  \
-    case 8: { constexpr int VP = 8; CALL; } break;  \
-    default: { constexpr int VP = 16; CALL; } break; \
-    }
-
 #define NC_VPL_SWITCH4(V, CALL)                     \
     switch (V) {                                    \
     case 1: { constexpr int VP = 1; CALL; } break;  \
@@ -1035,17 +1188,10 @@ static unsigned rows_grid(int64_t rows) {
     default: { constexpr int VP = 4; CALL; } break; \
     }
 
-#define NC_VPL_SWITCH8(V, CALL)                     \
-    switch (V) {                                    \
-    case 1: { constexpr int VP = 1; CALL; } break;  \
-    case 2: { constexpr int VP = 2; CALL; } break;  \
-    case 4: { constexpr int VP = 4; CALL; } break;  \
-    default: { constexpr int VP = 8; CALL; } break; \
-    }
-
 // LayerNorm backward plan (shared by the workspace query and the launch)
 struct LnPlan {
     bool reg;
+    bool team;                       // k_ln_bwd_team
     int vpl;
     bool full;                       // k_ln_bwd_pp (full rows of up to 1024 floats, gx written)
     bool pair;                       // k_ln_bwd_pair (rows of 512 or 1024 floats, gx written)
@@ -1058,9 +1204,20 @@ struct LnPlan {
 static LnPlan ln_plan(int64_t rows, int64_t D, bool aligned, bool has_gx) {
     LnPlan p{};
     p.vpl = (D % 4 == 0 && aligned) ? vpl_for(D) : 0;
-    if (p.vpl > 8) p.vpl = 0;  // rows beyond 2048 floats would spill registers: generic path
+    if (p.vpl > 4) p.vpl = 0;  // rows past 1024 floats go to teams of waves
     p.reg = p.vpl != 0;
-    if (p.reg) {
+    p.team = !p.reg && D <= kLnTeamMax;
+    if (p.team) {
+        // Up to 16 waves a CU of a 256-CU part, with two rows a wave or four a team at least, so that the partials stay
+        // small beside the rows; fewer rows than fill the CUs that way go to a workgroup each CU.
+        int tw = 1;
+        NC_LN_TEAM_SWITCH(D, (void)VP; tw = TW)
+        const int64_t teams = tw == 1 ? kLnWaves : 1, most = (rows + teams - 1) / teams;
+        const int64_t per = tw == 1 ? 2 : 4, cap = tw == 1 ? 2 * kPlanCUs : 16 * kPlanCUs / tw;
+        p.blocks = std::min<int64_t>(cap, std::max<int64_t>((most + per - 1) / per, std::min<int64_t>(most, kPlanCUs)));
+        if (p.blocks < 1) p.blocks = 1;
+        p.ws = (size_t)p.blocks * 2 * D * sizeof(double);
+    } else if (p.reg) {
         p.full = has_gx && p.vpl <= 4 && D == (int64_t)p.vpl * 4 * kWave;
         p.pair = NC_LN_BWD_PAIR && p.full && (p.vpl == 2 || p.vpl == 4);
         if (p.pair) {  // one workgroup per CU of a 256-CU part, rows dealt to its pairs in turn
@@ -1160,10 +1317,13 @@ extern "C" NC_HIP_API int nc_hip_layer_norm_fwd(int64_t rows, int64_t D, const f
     if (rows < 0 || D <= 0) return set_error(NC_HIP_ERR_ARG, "nc_hip_layer_norm_fwd: bad size");
     if (rows == 0) return NC_HIP_OK;
     hipStream_t st = as_stream(stream);
-    const bool al = aligned16(x) && aligned16(y) && (!w || aligned16(w)) && (!b || aligned16(b));
-    const int v = (D % 4 == 0 && al) ? vpl_for(D) : 0;
-    if (v) {
-        NC_VPL_SWITCH(v, hipLaunchKernelGGL(k_ln_fwd_reg<VP>, rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
+    const bool al = D % 4 == 0 && aligned16(x) && aligned16(y) && (!w || aligned16(w)) && (!b || aligned16(b));
+    if (D <= kWaveRowMax) {  // a wave per row
+        const int v = vpl_for(D);
+        if (al) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, true>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
+        else NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, false>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
+    } else if (D <= kWgRowMax && rows <= INT32_MAX) {  // a workgroup per row
+        NC_WG_SWITCH(D, hipLaunchKernelGGL((k_ln_fwd_wg<VP, NT>), dim3((unsigned)rows), NT, 0, st, x, w, b, eps, y, stats, (int)D))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         hipLaunchKernelGGL(k_ln_fwd_blk, grid, kRowB, 0, st, x, w, b, eps, y, stats, rows, D);
@@ -1205,17 +1365,23 @@ extern "C" NC_HIP_API int nc_hip_layer_norm_bwd(int64_t rows, int64_t D, const f
         if (cols)
             hipLaunchKernelGGL(k_ln_cols_combine, dim3((unsigned)((D + kCombCols - 1) / kCombCols), 2), kCombCols * kCombSlices, 0, st, part, gw, gb, D, (int)p.blocks);
     } else if (p.reg) {
-        const size_t lds = ln_bwd_lds(p.vpl, D, cols);
-        if (lds > 65536) return set_error(NC_HIP_ERR_ARG, "nc_hip_layer_norm_bwd: D too large for LDS combine");
+        const size_t lds = ln_bwd_lds(D, cols);
         const bool full = p.full;
         if (full && accumulate)
             NC_VPL_SWITCH4(p.vpl, if (w) hipLaunchKernelGGL((k_ln_bwd_pp<VP, true, true>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block); else hipLaunchKernelGGL((k_ln_bwd_pp<VP, true, false>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
         else if (full)
             NC_VPL_SWITCH4(p.vpl, if (w) hipLaunchKernelGGL((k_ln_bwd_pp<VP, false, true>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block); else hipLaunchKernelGGL((k_ln_bwd_pp<VP, false, false>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
         else if (accumulate)
-            NC_VPL_SWITCH8(p.vpl, hipLaunchKernelGGL((k_ln_bwd_reg<VP, true>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
+            NC_VPL_SWITCH4(p.vpl, hipLaunchKernelGGL((k_ln_bwd_reg<VP, true>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
         else
-            NC_VPL_SWITCH8(p.vpl, hipLaunchKernelGGL((k_ln_bwd_reg<VP, false>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
+            NC_VPL_SWITCH4(p.vpl, hipLaunchKernelGGL((k_ln_bwd_reg<VP, false>), dim3(p.blocks), kLnB, lds, st, x, w, stats, g, gx, part, rows, (int)D, p.rows_per_block))
+        if (cols)
+            hipLaunchKernelGGL(k_ln_cols_combine, dim3((unsigned)((D + kCombCols - 1) / kCombCols), 2), kCombCols * kCombSlices, 0, st, part, gw, gb, D, (int)p.blocks);
+    } else if (p.team) {
+        if (accumulate)
+            NC_LN_TEAM_SWITCH(D, hipLaunchKernelGGL((k_ln_bwd_team<VP, TW, true>), dim3((unsigned)p.blocks), ln_team_threads(TW), 0, st, x, w, stats, g, gx, part, rows, (int)D))
+        else
+            NC_LN_TEAM_SWITCH(D, hipLaunchKernelGGL((k_ln_bwd_team<VP, TW, false>), dim3((unsigned)p.blocks), ln_team_threads(TW), 0, st, x, w, stats, g, gx, part, rows, (int)D))
         if (cols)
             hipLaunchKernelGGL(k_ln_cols_combine, dim3((unsigned)((D + kCombCols - 1) / kCombCols), 2), kCombCols * kCombSlices, 0, st, part, gw, gb, D, (int)p.blocks);
     } else {
