@@ -755,6 +755,117 @@ static bool plan_reduce(const Prepared &p, RedPlan &pl, size_t *ws_need) {
     return true;
 }
 
+// Column sums of one kept and one reduced dim, g[k gr + m] (a bias gradient): a workgroup takes 32 columns and up to
+// `chunk` rows, 16 lanes (two columns, 8 bytes each) by 64 row slices, eight rows of loads in flight a lane; the
+// slices meet by wave shuffles and in LDS, in a fixed order.  With one chunk it writes the gradient itself.  Bound by
+// latency at these sizes: with a lane a column walking 64 rows one after another, and a launch to combine, [2048, 768] took
+// 24 us and takes 7, [2048, 3072] 26 and 7, [4096, 1000] 26 and 10 (in chunks).
+// Divisors that are the same for every row are inverted once in fp64, where terms like 0 / 0 stay what they are.
+constexpr int kColLanes = 16, kColSlices = 64, kColB = kColLanes * kColSlices, kColU = 8;
+constexpr uint32_t kColW = 2 * kColLanes;
+struct ColArgs {
+    uint32_t M, K, chunk, P;
+    int64_t gr, p1k, p1r, p2k, p2r, gxk;  // strides along the rows (r) and the columns (k)
+};
+
+template <int MODE, bool ACC>
+__global__ __launch_bounds__(kColB) void k_grad_cols(const float *__restrict__ g, const float *__restrict__ p1,
+                                                     const float *__restrict__ p2, float *__restrict__ gx,
+                                                     double *__restrict__ part, ColArgs c, double alpha) {
+    typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+    __shared__ double sh[kColB / kWave][kColW];
+    const int x = threadIdx.x % kColLanes, y = threadIdx.x / kColLanes;
+    const uint32_t groups = (c.M + kColW - 1) / kColW, p = blockIdx.x / groups;
+    const uint32_t m0 = (blockIdx.x - p * groups) * kColW, m = m0 + 2 * x;
+    const uint32_t k0 = p * c.chunk, k1 = min(c.K, k0 + c.chunk);
+    // the last column of an odd number is the second of the pair before it
+    const bool two = m + 1 < c.M;
+    const uint32_t mb = two ? m : c.M - 2;
+    const bool inv1 = MODE == 2 && c.p1r == 0, inv2 = MODE == 3 && c.p2r == 0;
+    auto at = [&](const float *q, int64_t ks, int64_t rs, uint32_t k) {
+        const float *e = q + (int64_t)k * rs;
+        if (ks == 0) return f2{*e, *e};
+        const f2u v = *(const f2u *)(e + mb);
+        return f2{v.x, v.y};
+    };
+    double acc[2] = {0.0, 0.0}, r1[2] = {1.0, 1.0}, r2[2] = {1.0, 1.0};
+    auto add = [&](f2 gv, f2 v1, f2 v2) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            if (inv1) acc[i] += (double)gv[i] * r1[i];
+            else if (inv2) acc[i] += -((double)gv[i] * (double)v1[i]) * r2[i];
+            else acc[i] += grad_d<MODE>((double)gv[i], (double)v1[i], (double)v2[i], alpha);
+        }
+    };
+    if (m < c.M) {
+        const f2 one = {1.f, 1.f};
+        if (inv1) {
+            const f2 v = at(p1, c.p1k, 0, 0);
+            r1[0] = 1.0 / (double)v.x;
+            r1[1] = 1.0 / (double)v.y;
+        }
+        if (inv2) {
+            const f2 v = at(p2, c.p2k, 0, 0);
+            r2[0] = 1.0 / ((double)v.x * (double)v.x);
+            r2[1] = 1.0 / ((double)v.y * (double)v.y);
+        }
+        uint32_t k = k0 + y;
+        for (; k + (kColU - 1) * kColSlices < k1; k += kColU * kColSlices) {
+            f2 gv[kColU], v1[kColU], v2[kColU];
+#pragma unroll
+            for (int u = 0; u < kColU; u++) {
+                gv[u] = at(g, 1, c.gr, k + u * kColSlices);
+                v1[u] = MODE != 0 && !inv1 ? at(p1, c.p1k, c.p1r, k + u * kColSlices) : one;
+                v2[u] = MODE == 3 && !inv2 ? at(p2, c.p2k, c.p2r, k + u * kColSlices) : one;
+            }
+#pragma unroll
+            for (int u = 0; u < kColU; u++) add(gv[u], v1[u], v2[u]);
+        }
+        for (; k < k1; k += kColSlices)
+            add(at(g, 1, c.gr, k), MODE != 0 && !inv1 ? at(p1, c.p1k, c.p1r, k) : one,
+                MODE == 3 && !inv2 ? at(p2, c.p2k, c.p2r, k) : one);
+        if (!two) acc[0] = acc[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        acc[i] += __shfl_xor(acc[i], 16);
+        acc[i] += __shfl_xor(acc[i], 32);
+        if (threadIdx.x % kWave < kColLanes) sh[threadIdx.x / kWave][2 * x + i] = acc[i];
+    }
+    __syncthreads();
+    const uint32_t o = m0 + threadIdx.x;
+    if (threadIdx.x >= kColW || o >= c.M) return;
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < kColB / kWave; i++) t += sh[i][threadIdx.x];
+    if (c.P == 1) {
+        float *q = gx + (int64_t)o * c.gxk;
+        *q = (float)((ACC ? (double)*q : 0.0) + t);
+    } else {
+        part[(size_t)p * c.M + o] = t;
+    }
+}
+
+// The plan's column sums as k_grad_cols takes them.  One chunk up to 2048 rows (32 a lane): splitting further costs the
+// combining launch, about 4 us.  Past that chunks of 512 to 2048 rows, the shorter the fewer column groups there
+// are to fill the CUs; never more partials than the general plan's, which sizes the workspace.
+static bool plan_cols(const RedPlan &pl, int mode, ColArgs &c) {
+    if (!pl.inner_kept || pl.kept.nd != 1 || pl.red.nd != 1 || pl.M < 2 || pl.kept.st[0][0] != 1) return false;
+    if (pl.K < 32 && pl.M > 4096) return false;  // most slices idle, and columns enough for a lane each
+    const auto k01 = [&](int o) { return pl.kept.st[o][0] == 0 || pl.kept.st[o][0] == 1; };
+    if ((mode != 0 && !k01(1)) || (mode == 3 && !k01(2))) return false;
+    c = ColArgs{pl.M, pl.K, pl.K, 1, pl.red.st[0][0], pl.kept.st[1][0], pl.red.st[1][0], pl.kept.st[2][0],
+                pl.red.st[2][0], pl.kept.st[3][0]};
+    if (pl.K > 2048) {
+        const uint32_t groups = (pl.M + kColW - 1) / kColW;
+        uint32_t P = std::max((pl.K + 2047) / 2048, (kPlanCUs + groups - 1) / groups);
+        P = std::min({P, (pl.K + 511) / 512, pl.P});
+        c.chunk = (pl.K + P - 1) / P;
+        c.P = (pl.K + c.chunk - 1) / c.chunk;
+    }
+    return true;
+}
+
 template <int MODE>
 static int launch_grad(const float *g, const float *p1, const float *p2, float *gx, const Prepared &p, float alpha,
                        int acc, void *ws, size_t ws_bytes, hipStream_t st) {
@@ -800,7 +911,18 @@ static int launch_grad(const float *g, const float *p1, const float *p2, float *
         return set_error(NC_HIP_ERR_WORKSPACE, "grad: workspace of %zu bytes needed, %zu given", need, ws_bytes);
     double *part = (double *)ws;
     const uint64_t items = (uint64_t)pl.M * pl.P;
-    if (pl.inner_kept) {
+    ColArgs cols;
+    if (plan_cols(pl, MODE, cols)) {
+        const dim3 grid((cols.M + kColW - 1) / kColW * cols.P);
+        if (acc)
+            hipLaunchKernelGGL((k_grad_cols<MODE, true>), grid, dim3(kColB), 0, st, g, p1, p2, gx, part, cols,
+                               (double)alpha);
+        else
+            hipLaunchKernelGGL((k_grad_cols<MODE, false>), grid, dim3(kColB), 0, st, g, p1, p2, gx, part, cols,
+                               (double)alpha);
+        if (cols.P == 1) return check_launch("nc_hip_binary_bwd");
+        pl.P = cols.P;
+    } else if (pl.inner_kept) {
         const uint64_t blocks = (items + kB - 1) / kB;
         const unsigned grid = (unsigned)(blocks < 1048576 ? blocks : 1048576);
         hipLaunchKernelGGL(k_grad_reduce_col<MODE>, dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
