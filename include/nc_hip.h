@@ -105,6 +105,10 @@ NC_HIP_API int nc_hip_copy_strided(int elem_bytes, int nd, const int64_t *shape,
 NC_HIP_API int nc_hip_accumulate_strided(int nd, const int64_t *shape, const float *src, float *dst,
                                          const int64_t *sd, void *stream);
 
+/* the same into memory whose old values do not count: dst[...] = 0 + src */
+NC_HIP_API int nc_hip_store_strided(int nd, const int64_t *shape, const float *src, float *dst,
+                                    const int64_t *sd, void *stream);
+
 /* y[i] += alpha * x[i] (fused, as axpy_f32 kernels_avx2.c:39-45). */
 NC_HIP_API int nc_hip_axpy(int64_t n, float alpha, const float *x, float *y, void *stream);
 /* Fill n elements of elem_bytes (1, 2, 4, 8) with the low bytes of `pattern`. */

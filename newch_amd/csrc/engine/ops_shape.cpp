@@ -198,15 +198,18 @@ static bool slice_alias(nc_node *n, const OutSpec &) { return view_of(n, sliced(
 static nc_status slice_fwd(nc_node *n) { return gather(n, sliced(n)); }
 
 // transpose / slice backward: the output gradient (contiguous) is added into x's contiguous gradient
-// at the places the layout picked, i.e. through the layout rebuilt over x's contiguous strides
-static void layout_bwd(nc_node *n, const Layout &over_grad) {
+// at the places the layout picked, i.e. through the layout rebuilt over x's contiguous strides.
+// covers: the layout picks every element of x, so a fresh gradient is stored, with no zeros first
+static void layout_bwd(nc_node *n, const Layout &over_grad, bool covers) {
     nc_tensor *x = n->in[0], *o = n->out;
     if (!grad_buf(x) || nc_numel(o) == 0) return;  // an empty output adds nothing to x's (zero) gradient
     const float *g = fptr(o->grad);
-    float *gx = g ? fptr(x->grad) : nullptr;
+    if (!g) return;
+    const int acc = covers ? grad_acc(x) : 1;
+    float *gx = fptr(x->grad);
+    const auto put = acc ? nc_hip_accumulate_strided : nc_hip_store_strided;
     if (!gx || !hip_layer_ok(x->ctx,
-                             nc_hip_accumulate_strided(o->ndim, o->shape, g, gx + over_grad.offset, over_grad.st,
-                                                       stream(x->ctx)),
+                             put(o->ndim, o->shape, g, gx + over_grad.offset, over_grad.st, stream(x->ctx)),
                              n->op->name))
         return;
     wrote_dev(x->grad);
@@ -224,7 +227,7 @@ static void transpose_bwd(nc_node *n) {
     Layout L = dense_of(n->in[0]);
     const int a = (int)n->p.i[0], b = (int)n->p.i[1];
     std::swap(L.st[a], L.st[b]);
-    layout_bwd(n, L);
+    layout_bwd(n, L, true);
 }
 
 static void slice_bwd(nc_node *n) {
@@ -232,7 +235,7 @@ static void slice_bwd(nc_node *n) {
     const int a = (int)n->p.i[0];
     if (n->p.i[2] > 0) L.offset = n->p.i[1] * L.st[a];
     L.st[a] *= n->p.i[3];
-    layout_bwd(n, L);
+    layout_bwd(n, L, false);
 }
 
 const OpDef op_transpose = {"transpose", OPF_VIEW, 0, transpose_shape, transpose_alias, transpose_fwd, transpose_bwd};

@@ -1651,13 +1651,67 @@ __global__ __launch_bounds__(kB) void k_gather(const T *__restrict__ src, T *__r
     }
 }
 
+// dst[map(w)] = (ACC ? dst[map(w)] : 0) + src[w]
+template <bool ACC>
 __global__ __launch_bounds__(kB) void k_scatter_add(const float *__restrict__ src, float *__restrict__ dst,
                                                     IdxMap<1> m, uint32_t n) {
     const uint32_t step = gridDim.x * kB;
     for (uint32_t w = blockIdx.x * kB + threadIdx.x; w < n; w += step) {
         int64_t off[1];
         offsets<1>(m, w, off);
-        dst[off[0]] = dst[off[0]] + src[w];
+        dst[off[0]] = (ACC ? dst[off[0]] : 0.0f) + src[w];
+    }
+}
+
+// Copies between two layouts whose unit-stride dims differ (a transposed view gathered, or its gradient scattered
+// back): 64 x 64 tiles of the two dims turned in LDS, so both sides move whole cache lines where the maps above touch one
+// per element on the strided side.  HBM-bound; the gradient of
+// keys [96, 197, 64] seen transposed took 25 us to clear and scatter into, and is stored in 8 (10 MB each way).
+// MODE: 0 copy, 1 dst = 0 + src, 2 dst += src.
+enum { TR_COPY = 0, TR_STORE = 1, TR_ADD = 2 };
+constexpr uint32_t kTr = 64;
+struct TrPlan {
+    uint32_t A, B;    // extents: A along the source's unit stride, B along the destination's
+    int64_t sB, dA;   // the source's stride along B, the destination's along A
+    IntDiv ta, tb;    // tiles along each
+    IdxMap<2> batch;  // the other dims: 0 source, 1 destination
+    uint32_t blocks;
+};
+
+template <int MODE, typename T>
+__global__ __launch_bounds__(kB) void k_turn(const T *__restrict__ src, T *__restrict__ dst, TrPlan pl) {
+    __shared__ T tile[kTr][kTr + 1];
+    uint32_t q = pl.ta.div(blockIdx.x);
+    const uint32_t a0 = (blockIdx.x - q * pl.ta.d) * kTr;
+    const uint32_t bi = pl.tb.div(q), b0 = (q - bi * pl.tb.d) * kTr;
+    int64_t off[2];
+    offsets<2>(pl.batch, bi, off);
+    src += off[0];
+    dst += off[1];
+    const uint32_t x = threadIdx.x % kTr, y = threadIdx.x / kTr;
+    constexpr uint32_t kStep = kB / kTr;
+    T old[kTr / kStep];
+    if constexpr (MODE == TR_ADD) {
+#pragma unroll
+        for (uint32_t i = 0; i < kTr / kStep; i++) {
+            const uint32_t a = a0 + y + i * kStep, b = b0 + x;
+            if (a < pl.A && b < pl.B) old[i] = dst[(int64_t)a * pl.dA + b];
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kTr / kStep; i++) {
+        const uint32_t a = a0 + x, b = b0 + y + i * kStep;
+        if (a < pl.A && b < pl.B) tile[y + i * kStep][x] = src[(int64_t)b * pl.sB + a];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kTr / kStep; i++) {
+        const uint32_t a = a0 + y + i * kStep, b = b0 + x;
+        if (a < pl.A && b < pl.B) {
+            const T v = tile[x][y + i * kStep];
+            if constexpr (MODE == TR_COPY) dst[(int64_t)a * pl.dA + b] = v;
+            else dst[(int64_t)a * pl.dA + b] = (MODE == TR_ADD ? old[i] : T(0)) + v;
+        }
     }
 }
 
@@ -1713,6 +1767,45 @@ static void contiguous_strides(int nd, const int64_t *shape, int64_t *cs) {
     }
 }
 
+// The tiles for a strided operand (p.st[0]) against the contiguous one of p's shape, where the two have different unit
+// dims of at least 16 elements: shorter ones leave most of a tile empty, and the plain maps stay.
+static bool plan_turn(const Prepared &p, bool strided_src, TrPlan &pl) {
+    const int in = p.nd - 1;
+    if (p.nd < 2 || p.st[0][in] == 1) return false;
+    int j = -1;
+    for (int d = 0; d < in; d++)
+        if (p.st[0][d] == 1) j = d;
+    if (j < 0 || p.shape[j] < 16 || p.shape[in] < 16) return false;
+    int64_t cs[NC_HIP_MAX_DIMS];
+    contiguous_strides(p.nd, p.shape, cs);
+    const int a = strided_src ? j : in, b = strided_src ? in : j;
+    pl.A = (uint32_t)p.shape[a];
+    pl.B = (uint32_t)p.shape[b];
+    pl.sB = strided_src ? p.st[0][b] : cs[b];
+    pl.dA = strided_src ? cs[a] : p.st[0][a];
+    Prepared o{};
+    uint64_t n = 1;
+    for (int d = 0; d < p.nd; d++) {
+        if (d == a || d == b) continue;
+        o.shape[o.nd] = p.shape[d];
+        o.st[0][o.nd] = strided_src ? p.st[0][d] : cs[d];
+        o.st[1][o.nd++] = strided_src ? cs[d] : p.st[0][d];
+        n *= (uint64_t)p.shape[d];
+    }
+    if (o.nd == 0) {
+        o.nd = 1;
+        o.shape[0] = 1;
+    }
+    make_map<2>(o, 1, pl.batch);
+    const uint32_t ta = (pl.A + kTr - 1) / kTr, tb = (pl.B + kTr - 1) / kTr;
+    n *= (uint64_t)ta * tb;
+    if (n > INT32_MAX) return false;
+    pl.ta = IntDiv(ta);
+    pl.tb = IntDiv(tb);
+    pl.blocks = (uint32_t)n;
+    return true;
+}
+
 // Gathers of 2^32 elements or more: runs of at most 2^30 elements (for_each_run), each a launch of
 // its own; the destination is the contiguous tensor of the whole shape.
 extern "C" NC_HIP_API int nc_hip_copy_strided(int elem_bytes, int nd, const int64_t *shape, const void *src,
@@ -1740,6 +1833,12 @@ extern "C" NC_HIP_API int nc_hip_copy_strided(int elem_bytes, int nd, const int6
                                        (char *)dst + off[1] * elem_bytes, stream);
         });
     }
+    TrPlan tr;
+    if (elem_bytes == 4 && plan_turn(p, true, tr)) {
+        hipLaunchKernelGGL((k_turn<TR_COPY, uint32_t>), dim3(tr.blocks), kB, 0, st, (const uint32_t *)src,
+                           (uint32_t *)dst, tr);
+        return check_launch("nc_hip_copy_strided");
+    }
     IdxMap<1> m;
     make_map<1>(p, 1, m);
     const unsigned grid = stream_grid(p.numel, kB, 16);
@@ -1754,11 +1853,11 @@ extern "C" NC_HIP_API int nc_hip_copy_strided(int elem_bytes, int nd, const int6
     return check_launch("nc_hip_copy_strided");
 }
 
-extern "C" NC_HIP_API int nc_hip_accumulate_strided(int nd, const int64_t *shape, const float *src, float *dst,
-                                                    const int64_t *sd, void *stream) {
+static int scatter(bool acc, int nd, const int64_t *shape, const float *src, float *dst, const int64_t *sd, void *stream,
+                   const char *who) {
     Prepared p;
     const int64_t *strides[1] = {sd};
-    int rc = prepare(nd, shape, 1, strides, p, "nc_hip_accumulate_strided");
+    int rc = prepare(nd, shape, 1, strides, p, who);
     if (rc) return rc;
     if (p.numel == 0) return NC_HIP_OK;
     const RunSplit rsp = run_split();
@@ -1767,7 +1866,7 @@ extern "C" NC_HIP_API int nc_hip_accumulate_strided(int nd, const int64_t *shape
         contiguous_strides(nd, shape, cs);
         const int64_t *st2[2] = {cs, sd};
         return for_each_run(nd, shape, 2, st2, rsp.limit, [&](const int64_t *rs, const int64_t *off, const bool *) {
-            return nc_hip_accumulate_strided(nd, rs, src + off[0], dst + off[1], sd, stream);
+            return scatter(acc, nd, rs, src + off[0], dst + off[1], sd, stream, who);
         });
     }
     if (p.nd == 0) {
@@ -1775,11 +1874,29 @@ extern "C" NC_HIP_API int nc_hip_accumulate_strided(int nd, const int64_t *shape
         p.shape[0] = 1;
         p.st[0][0] = 0;
     }
+    hipStream_t st = as_stream(stream);
+    TrPlan tr;
+    if (plan_turn(p, false, tr)) {
+        if (acc) hipLaunchKernelGGL((k_turn<TR_ADD, float>), dim3(tr.blocks), kB, 0, st, src, dst, tr);
+        else hipLaunchKernelGGL((k_turn<TR_STORE, float>), dim3(tr.blocks), kB, 0, st, src, dst, tr);
+        return check_launch(who);
+    }
     IdxMap<1> m;
     make_map<1>(p, 1, m);
-    hipLaunchKernelGGL(k_scatter_add, stream_grid(p.numel, kB, 16), kB, 0, as_stream(stream), src, dst, m,
-                       (uint32_t)p.numel);
-    return check_launch("nc_hip_accumulate_strided");
+    const unsigned grid = stream_grid(p.numel, kB, 16);
+    if (acc) hipLaunchKernelGGL(k_scatter_add<true>, grid, kB, 0, st, src, dst, m, (uint32_t)p.numel);
+    else hipLaunchKernelGGL(k_scatter_add<false>, grid, kB, 0, st, src, dst, m, (uint32_t)p.numel);
+    return check_launch(who);
+}
+
+extern "C" NC_HIP_API int nc_hip_accumulate_strided(int nd, const int64_t *shape, const float *src, float *dst,
+                                                    const int64_t *sd, void *stream) {
+    return scatter(true, nd, shape, src, dst, sd, stream, "nc_hip_accumulate_strided");
+}
+
+extern "C" NC_HIP_API int nc_hip_store_strided(int nd, const int64_t *shape, const float *src, float *dst,
+                                               const int64_t *sd, void *stream) {
+    return scatter(false, nd, shape, src, dst, sd, stream, "nc_hip_store_strided");
 }
 
 extern "C" NC_HIP_API int nc_hip_axpy(int64_t n, float alpha, const float *x, float *y, void *stream) {

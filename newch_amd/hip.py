@@ -47,6 +47,7 @@ SIGNATURES = {
                                    c_size_t, P]),
     "nc_hip_copy_strided": (c_int, [c_int, c_int, I64P, P, I64P, P, P]),
     "nc_hip_accumulate_strided": (c_int, [c_int, I64P, P, P, I64P, P]),
+    "nc_hip_store_strided": (c_int, [c_int, I64P, P, P, I64P, P]),
     "nc_hip_axpy": (c_int, [c_int64, c_float, P, P, P]),
     "nc_hip_fill": (c_int, [P, c_int, c_uint64, c_int64, P]),
     "nc_hip_convert": (c_int, [c_int, c_int, c_int64, P, P, P]),
