@@ -193,6 +193,14 @@ NC_HIP_API int nc_hip_nll_loss_fwd(int64_t N, int64_t C, const float *x, const i
 /* gi[i, lab_i] -= s, s = gout (sum) or gout / N; gi is read and written: nll_bwd, ops_nn.c:412-420. */
 NC_HIP_API int nc_hip_nll_loss_bwd(int64_t N, int64_t C, const int32_t *lab, const float *gout, int sum,
                                    float *gi, void *stream);
+/* Mean squared error over n elements: d = a - b (16-byte aligned, kept by the caller for the backward), *loss the mean
+ * of d * d; the gradients 2 (*gout / n) d of a and its negative of b, each stored or added (acc) where its pointer is
+ * set. */
+NC_HIP_API size_t nc_hip_mse_loss_workspace(int64_t n);
+NC_HIP_API int nc_hip_mse_loss_fwd(int64_t n, const float *a, const float *b, float *d, float *loss, void *ws,
+                                   size_t ws_bytes, void *stream);
+NC_HIP_API int nc_hip_mse_loss_bwd(int64_t n, const float *d, const float *gout, float *ga, float *gb, int acc_a,
+                                   int acc_b, void *stream);
 
 /* One optimizer update of a parameter w [n] with gradient g (optim.c:161-216): the reference's fp32
  * expression per element, in its order, without fused multiply-adds.  kind: NC_HIP_OPT_*.  s1 is

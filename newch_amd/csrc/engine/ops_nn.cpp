@@ -1,6 +1,8 @@
 // softmax / log_softmax over the last axis, LayerNorm over the last k axes, and the losses built on
 // the softmax rows.  Reference: engine/src/ops/ops_nn.c (:8-77 softmax, :83-162 cross_entropy and
 // mse_loss, :368-426 nll_loss, :434-538 layer_norm).
+#include <algorithm>
+
 #include "engine.hpp"
 
 namespace nce {
@@ -242,6 +244,44 @@ static void loss_bwd(nc_node *n) {
     wrote_dev(xt->grad);
 }
 
+// mse_loss of two f32 tensors of one shape, in one pass each way; d = pred - target is kept for the backward.
+static nc_status mse_shape(nc_node *, OutSpec &out) {
+    out.dims = Dims{};
+    return NC_OK;
+}
+
+static nc_status mse_fwd(nc_node *n) {
+    nc_ctx *ctx = n->in[0]->ctx;
+    const int64_t N = nc_numel(n->in[0]);
+    const float *a = contig_f32(n->in[0]), *b = contig_f32(n->in[1]);
+    float *loss = fptr(n->out), *d = (float *)save_state(n, (size_t)N * sizeof(float));
+    const size_t ws_bytes = nc_hip_mse_loss_workspace(N);
+    char *ws = arena_alloc(ctx, ws_bytes);
+    if (!a || !b || !loss || !d || !ws) return NC_ERR_STATE;
+    if (!hip_layer_ok(ctx, nc_hip_mse_loss_fwd(N, a, b, d, loss, ws, ws_bytes, stream(ctx)), "mse_loss"))
+        return NC_ERR_STATE;
+    wrote_dev(n->out);
+    return NC_OK;
+}
+
+static void mse_bwd(nc_node *n) {
+    nc_tensor *a = n->in[0], *b = n->in[1];
+    const bool want_a = needs_grad(a), want_b = needs_grad(b);
+    const float *g = fptr(n->out->grad);
+    if (!g || (want_a && !grad_buf(a)) || (want_b && !grad_buf(b))) return;
+    const int acc_a = want_a ? grad_acc(a) : 1, acc_b = want_b ? grad_acc(b) : 1;
+    float *ga = want_a ? fptr(a->grad) : nullptr, *gb = want_b ? fptr(b->grad) : nullptr;
+    if ((want_a && !ga) || (want_b && !gb)) return;
+    if (!hip_layer_ok(a->ctx,
+                      nc_hip_mse_loss_bwd(nc_numel(a), (const float *)n->saved, g, ga, gb, acc_a, acc_b, stream(a->ctx)),
+                      "mse_loss"))
+        return;
+    if (want_a) wrote_dev(a->grad);
+    if (want_b) wrote_dev(b->grad);
+}
+
+const OpDef op_mse_loss = {"mse_loss", 0, 0, mse_shape, nullptr, mse_fwd, mse_bwd};
+
 const OpDef op_cross_entropy = {"cross_entropy", 0, LOSS_CE, loss_shape, nullptr, loss_fwd, loss_bwd};
 const OpDef op_nll_loss = {"nll_loss", 0, LOSS_NLL, loss_shape, nullptr, loss_fwd, loss_bwd};
 
@@ -265,8 +305,15 @@ nc_tensor *nc_nll_loss(nc_tensor *logp, nc_tensor *labels, int sum) {
     return apply(&op_nll_loss, in, 2, &p);
 }
 
-// composite, differentiable through the ops it is built from (ops_nn.c:158-162)
+// Two different f32 tensors of one shape run as one op; anything else (broadcasts, empty tensors, a tensor against
+// itself, failures) as the ops it is composed of (ops_nn.c:158-162), with their results and errors.
 nc_tensor *nc_mse_loss(nc_tensor *pred, nc_tensor *target) {
+    if (pred && target && pred != target && pred->ctx == target->ctx && pred->ctx->device >= 0 &&
+        pred->dtype == NC_F32 && target->dtype == NC_F32 && pred->ndim == target->ndim &&
+        std::equal(pred->shape, pred->shape + pred->ndim, target->shape) && nc_numel(pred) > 0) {
+        nc_tensor *in[2] = {pred, target};
+        return apply(&op_mse_loss, in, 2, nullptr);
+    }
     nc_tensor *d = nc_sub(pred, target);
     return nc_mean(nc_mul(d, d), NC_ALL_AXES, 0);
 }

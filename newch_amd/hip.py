@@ -76,6 +76,9 @@ SIGNATURES = {
     "nc_hip_cross_entropy_fwd": (c_int, [c_int64, c_int64, P, P, P, P, P, P, c_size_t, P]),
     "nc_hip_cross_entropy_bwd": (c_int, [c_int64, c_int64, P, P, P, P, P, c_int, P]),
     "nc_hip_nll_loss_fwd": (c_int, [c_int64, c_int64, P, P, c_int, P, P, P, c_size_t, P]),
+    "nc_hip_mse_loss_workspace": (c_size_t, [c_int64]),
+    "nc_hip_mse_loss_fwd": (c_int, [c_int64, P, P, P, P, P, c_size_t, P]),
+    "nc_hip_mse_loss_bwd": (c_int, [c_int64, P, P, P, P, c_int, c_int, P]),
     "nc_hip_nll_loss_bwd": (c_int, [c_int64, c_int64, P, P, c_int, P, P]),
     "nc_hip_gemm_f32": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_float, P, c_int64, P, c_int64, c_float, P,
                                 c_int64, P]),
