@@ -298,6 +298,15 @@ struct Prepared {
     int64_t numel;
 };
 
+// row-major (contiguous) element strides of shape
+static void contiguous_strides(int nd, const int64_t *shape, int64_t *cs) {
+    int64_t s = 1;
+    for (int d = nd - 1; d >= 0; d--) {
+        cs[d] = s;
+        s *= shape[d];
+    }
+}
+
 static int prepare(int nd, const int64_t *shape, int nops, const int64_t *const *strides, Prepared &p,
                    const char *who) {
     if (nd < 0 || nd > NC_HIP_MAX_DIMS) return set_error(NC_HIP_ERR_ARG, "%s: ndim %d out of range", who, nd);
@@ -561,6 +570,60 @@ __global__ __launch_bounds__(64) void k_grad_elementwise4(const f4 *__restrict__
     __builtin_nontemporal_store(r, gx + i);
 }
 
+// The same where g and gx are contiguous over the whole shape and the other operands broadcast or are strided: four
+// consecutive elements a lane, g and gx in 16-byte pieces at any alignment, one division of the index per dim for the
+// four.  A group that reaches past the innermost dim finds its elements one by one.
+typedef float f4any __attribute__((ext_vector_type(4), aligned(4)));
+template <int NOPS>
+__device__ __forceinline__ f4 row4(const float *q, const IdxMap<NOPS> &m, int o, int64_t off, uint32_t e, bool in_row) {
+    const int64_t s = m.st[o][m.nd - 1];
+    if (in_row) {
+        if (s == 0) {
+            const float v = q[off];
+            return f4{v, v, v, v};
+        }
+        if (s == 1) return *(const f4any *)(q + off);
+        return f4{q[off], q[off + s], q[off + 2 * s], q[off + 3 * s]};
+    }
+    f4 v;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        int64_t t[NOPS];
+        offsets<NOPS>(m, e + c, t);
+        v[c] = q[t[o]];
+    }
+    return v;
+}
+
+template <int MODE, bool ACC>
+__global__ __launch_bounds__(kB) void k_grad_rows4(const float *__restrict__ g, const float *__restrict__ p1,
+                                                   const float *__restrict__ p2, float *__restrict__ gx, IdxMap<2> m,
+                                                   uint32_t n, float alpha) {
+    const uint32_t e = (blockIdx.x * kB + threadIdx.x) * 4;
+    if (e >= n) return;
+    if (e + 4 <= n) {
+        int64_t off[2];
+        offsets<2>(m, e, off);
+        const uint32_t w = m.size[m.nd - 1];
+        const bool in_row = e - m.div[m.nd - 1].div(e) * w + 4 <= w;
+        const f4 z = {0.f, 0.f, 0.f, 0.f};
+        const f4 gg = __builtin_nontemporal_load((const f4any *)(g + e));
+        const f4 o = ACC ? __builtin_nontemporal_load((const f4any *)(gx + e)) : z;
+        const f4 a = MODE != 0 ? row4<2>(p1, m, 0, off[0], e, in_row) : z;
+        const f4 b = MODE == 3 ? row4<2>(p2, m, 1, off[1], e, in_row) : z;
+        f4 r;
+#pragma unroll
+        for (int c = 0; c < 4; c++) r[c] = grad_f<MODE>(o[c], gg[c], a[c], b[c], alpha);
+        __builtin_nontemporal_store(r, (f4any *)(gx + e));
+        return;
+    }
+    for (uint32_t c = e; c < n; c++) {
+        int64_t off[2];
+        offsets<2>(m, c, off);
+        gx[c] = grad_f<MODE>(ACC ? gx[c] : 0.0f, g[c], MODE != 0 ? p1[off[0]] : 0.0f, MODE == 3 ? p2[off[1]] : 0.0f, alpha);
+    }
+}
+
 // Reduced grads.  The coalesced dims split into kept dims (gx stride != 0) and reduced dims.
 struct RedPlan {
     IdxMap<4> kept;      // over the M kept indices (gx offsets in operand 3)
@@ -641,13 +704,21 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_col(const float *__restrict_
     }
 }
 
-// row mode: one block per (kept index, chunk of reduced indices); lanes stride over the chunk
+// row mode: one block per (kept index, chunk of reduced indices); lanes take four consecutive indices at a time, in
+// 16-byte pieces where the operand's innermost stride is 1.  The sum over all but the middle dim of
+// [704, 704, 128] with division took 190 us an element a lane, dividing each in fp64, and takes 115.  A divisor that is the same for all reduced indices is
+// inverted once, in fp64, where terms like 0 / 0 stay what they are.
 template <int MODE>
 __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict__ g, const float *__restrict__ p1,
                                                         const float *__restrict__ p2, RedPlan pl, double alpha,
                                                         double *__restrict__ part) {
     __shared__ double sh[kB / kWave];
     const uint64_t total = (uint64_t)pl.M * pl.P;
+    const int in = pl.red.nd - 1;
+    const uint32_t w = pl.red.size[in];
+    const int od = MODE == 2 ? 1 : 2;  // the divisor's operand
+    bool one = MODE == 2 || MODE == 3;
+    for (int d = 0; d <= in; d++) one = one && pl.red.st[od][d] == 0;
     for (uint64_t item = blockIdx.x; item < total; item += gridDim.x) {  // block-uniform loop
         const uint32_t mi = (uint32_t)(item % pl.M);
         const uint32_t p = (uint32_t)(item / pl.M);
@@ -655,13 +726,35 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
         offsets<4>(pl.kept, mi, ko);
         const uint32_t k0 = p * pl.chunk;
         const uint32_t k1 = min(pl.K, k0 + pl.chunk);
+        const float *gk = g + ko[0], *q1 = p1 + ko[1], *q2 = p2 + ko[2];
+        double inv = 1.0;
+        if (one) {
+            const double v = (double)(MODE == 2 ? *q1 : *q2);
+            inv = 1.0 / (MODE == 2 ? v : v * v);
+        }
+        auto term = [&](float gv, float v1, float v2) {
+            if (MODE == 2 && one) return (double)gv * inv;
+            if (MODE == 3 && one) return -((double)gv * (double)v1) * inv;
+            return grad_d<MODE>((double)gv, (double)v1, (double)v2, alpha);
+        };
         double acc = 0.0;
-        for (uint32_t k = k0 + threadIdx.x; k < k1; k += kB) {
+        for (uint32_t k = k0 + 4 * threadIdx.x; k < k1; k += 4 * kB) {
             int64_t ro[3];
             offsets<3>(pl.red, k, ro);
-            const double v1 = (MODE == 1 || MODE == 2 || MODE == 3) ? (double)p1[ko[1] + ro[1]] : 0.0;
-            const double v2 = MODE == 3 ? (double)p2[ko[2] + ro[2]] : 0.0;
-            acc += grad_d<MODE>((double)g[ko[0] + ro[0]], v1, v2, alpha);
+            const f4 z = {0.f, 0.f, 0.f, 0.f};
+            if (k + 4 <= k1) {
+                const bool in_row = k - pl.red.div[in].div(k) * w + 4 <= w;
+                const f4 gv = row4<3>(gk, pl.red, 0, ro[0], k, in_row);
+                const f4 v1 = MODE != 0 && !(MODE == 2 && one) ? row4<3>(q1, pl.red, 1, ro[1], k, in_row) : z;
+                const f4 v2 = MODE == 3 && !one ? row4<3>(q2, pl.red, 2, ro[2], k, in_row) : z;
+#pragma unroll
+                for (int c = 0; c < 4; c++) acc += term(gv[c], v1[c], v2[c]);
+            } else {
+                for (uint32_t c = k; c < k1; c++) {
+                    offsets<3>(pl.red, c, ro);
+                    acc += term(gk[ro[0]], MODE != 0 ? q1[ro[1]] : 0.0f, MODE == 3 ? q2[ro[2]] : 0.0f);
+                }
+            }
         }
         acc = wave_sum(acc);
         if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave] = acc;
@@ -893,9 +986,32 @@ static int launch_grad(const float *g, const float *p1, const float *p2, float *
                                    (const f4 *)p1, (const f4 *)p2, (f4 *)gx, n4, alpha);
             return check_launch("nc_hip_binary_bwd");
         }
+        if (p.numel >= (int64_t)UINT32_MAX) return set_error(NC_HIP_ERR_ARG, "grad: 2^32 or more elements");
+        // g and gx in whole: four elements a lane.  x[704, 704, 128] / b[704, 1] 161 -> 81 us (6.2 TB/s), x[2001, 12939] *
+        // b[12939] 66 -> 36, against the kernel below, which stays for gradients laid out in another order
+        int64_t cs[NC_HIP_MAX_DIMS];
+        contiguous_strides(q.nd, q.shape, cs);
+        bool flat = q.numel < (int64_t)UINT32_MAX - 4 * kB;
+        for (int d = 0; d < q.nd; d++) flat = flat && q.st[0][d] == cs[d] && q.st[3][d] == cs[d];
+        if (flat) {
+            Prepared o = q;
+            for (int d = 0; d < q.nd; d++) {
+                o.st[0][d] = q.st[1][d];
+                o.st[1][d] = q.st[2][d];
+            }
+            IdxMap<2> m2;
+            make_map<2>(o, 1, m2);
+            const dim3 g4((unsigned)((q.numel + 4 * kB - 1) / (4 * kB)));
+            if (acc)
+                hipLaunchKernelGGL((k_grad_rows4<MODE, true>), g4, dim3(kB), 0, st, g, p1, p2, gx, m2, (uint32_t)q.numel,
+                                   alpha);
+            else
+                hipLaunchKernelGGL((k_grad_rows4<MODE, false>), g4, dim3(kB), 0, st, g, p1, p2, gx, m2, (uint32_t)q.numel,
+                                   alpha);
+            return check_launch("nc_hip_binary_bwd");
+        }
         IdxMap<4> m;
         make_map<4>(q, 1, m);
-        if (p.numel >= (int64_t)UINT32_MAX) return set_error(NC_HIP_ERR_ARG, "grad: 2^32 or more elements");
         const unsigned grid = stream_grid(p.numel, kB, 16);
         if (acc)
             hipLaunchKernelGGL((k_grad_elementwise<MODE, true>), dim3(grid), dim3(kB), 0, st, g, p1, p2, gx, m,
@@ -1757,15 +1873,6 @@ __global__ __launch_bounds__(kB) void k_convert(const S *__restrict__ src, D *__
 }
 
 }  // namespace nchip
-
-// row-major (contiguous) element strides of shape
-static void contiguous_strides(int nd, const int64_t *shape, int64_t *cs) {
-    int64_t s = 1;
-    for (int d = nd - 1; d >= 0; d--) {
-        cs[d] = s;
-        s *= shape[d];
-    }
-}
 
 // The tiles for a strided operand (p.st[0]) against the contiguous one of p's shape, where the two have different unit
 // dims of at least 16 elements: shorter ones leave most of a tile empty, and the plain maps stay.

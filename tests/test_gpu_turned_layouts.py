@@ -78,6 +78,7 @@ def test_gaps_and_repeats(K):
     assert K.lib.nc_hip_copy_strided(4, 3, i64((3, 65, 70)), dx.ptr, i64((0, 1, 90)), out.ptr, None) == 0
     np.testing.assert_array_equal(out.to_numpy(np.float32, 3 * 65 * 70).reshape(3, 65, 70), np.stack([view] * 3))
     v = rng.standard_normal((65, 70)).astype(np.float32)
-    assert K.lib.nc_hip_accumulate_strided(2, i64((65, 70)), dev(v).ptr, dx.ptr, i64((1, 90)), None) == 0
+    dv = dev(v)
+    assert K.lib.nc_hip_accumulate_strided(2, i64((65, 70)), dv.ptr, dx.ptr, i64((1, 90)), None) == 0
     x[:, :65] += v.T
     np.testing.assert_array_equal(dx.to_numpy(np.float32, (70, 90)), x)
