@@ -1906,7 +1906,7 @@ static bool plan_turn(const Prepared &p, bool strided_src, TrPlan &pl) {
     make_map<2>(o, 1, pl.batch);
     const uint32_t ta = (pl.A + kTr - 1) / kTr, tb = (pl.B + kTr - 1) / kTr;
     n *= (uint64_t)ta * tb;
-    if (n > INT32_MAX) return false;
+    if (n > (uint64_t)kMaxLanes / kB) return false;  // thin matrices, nearly empty tiles: more lanes than a launch has
     pl.ta = IntDiv(ta);
     pl.tb = IntDiv(tb);
     pl.blocks = (uint32_t)n;

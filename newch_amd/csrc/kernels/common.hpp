@@ -406,4 +406,9 @@ inline unsigned stream_grid(int64_t work_items, int block, int per_cu = 8) {
     return (unsigned)(need < cap ? need : cap);
 }
 
+// A dispatch counts its work-items in 32 bits.  Kernels with a workgroup (of up to 1024 lanes) for every row are launched
+// over at most kWgRowsPerLaunch rows at a time.
+constexpr int64_t kMaxLanes = (int64_t)UINT32_MAX;
+constexpr int64_t kWgRowsPerLaunch = int64_t(1) << 21;
+
 }  // namespace nchip

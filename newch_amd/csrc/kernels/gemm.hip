@@ -310,25 +310,26 @@ static int sg_launch_dma(SgArgs &p, int64_t count, hipStream_t st, const char *w
 // waves).  The choice fixes how K is split, so it depends on the shape and layout alone: planned for kPlanCUs,
 // never for the device.
 struct SgTile {
-    int bm, bn;
+    int bm, bn, lanes;
     float c[3][4];  // a0, a1, s0, s1 by M/N-contiguous operands
 };
 static const SgTile kSgTiles[] = {  // in the order of sg_tile_run
-    {128, 64, {{2.95f, 0.410f, 2.01f, 0.975f}, {3.65f, 0.459f, 1.36f, 1.032f}, {4.24f, 0.316f, 1.11f, 1.267f}}},
-    {96, 96, {{3.45f, 0.049f, 2.35f, 1.346f}, {2.94f, 0.089f, 3.19f, 1.353f}, {3.16f, 0.079f, 3.33f, 1.369f}}},
-    {96, 64, {{2.85f, 0.367f, 1.28f, 0.710f}, {3.25f, 0.330f, 1.25f, 0.810f}, {4.04f, 0.346f, 1.00f, 0.899f}}},
-    {96, 64, {{2.98f, 0.131f, 1.94f, 0.746f}, {2.29f, 0.039f, 2.53f, 0.949f}, {2.43f, 0.048f, 2.73f, 1.015f}}},
-    {64, 96, {{3.10f, 0.118f, 1.94f, 0.753f}, {2.11f, 0.026f, 2.88f, 0.981f}, {2.15f, 0.065f, 2.62f, 1.061f}}},
-    {64, 64, {{2.42f, 0.242f, 1.26f, 0.486f}, {2.90f, 0.227f, 0.95f, 0.561f}, {2.89f, 0.305f, 1.02f, 0.565f}}},
-    {64, 64, {{2.98f, 0.075f, 1.39f, 0.520f}, {2.86f, 0.113f, 1.41f, 0.582f}, {2.83f, 0.142f, 1.35f, 0.601f}}},
-    {64, 32, {{1.73f, 0.004f, 1.99f, 0.332f}, {2.00f, -0.002f, 1.82f, 0.386f}, {1.71f, 0.020f, 2.07f, 0.412f}}},
-    {32, 64, {{1.71f, 0.010f, 2.12f, 0.313f}, {1.82f, 0.012f, 1.96f, 0.390f}, {1.75f, 0.013f, 2.07f, 0.409f}}},
-    {32, 32, {{2.74f, 0.063f, 0.65f, 0.162f}, {2.67f, 0.064f, 0.65f, 0.192f}, {2.75f, 0.062f, 0.71f, 0.195f}}},
-    {32, 32, {{2.82f, -0.014f, 1.40f, 0.188f}, {2.19f, -0.004f, 1.73f, 0.218f}, {1.93f, 0.003f, 1.98f, 0.206f}}},
-    {32, 16, {{3.55f, -0.028f, 1.08f, 0.114f}, {3.12f, -0.024f, 1.30f, 0.137f}, {3.24f, -0.026f, 1.18f, 0.155f}}},
-    {16, 32, {{3.10f, -0.022f, 1.15f, 0.114f}, {3.37f, -0.023f, 1.21f, 0.135f}, {3.06f, -0.025f, 1.35f, 0.156f}}},
-    {16, 16, {{3.61f, -0.031f, 1.37f, 0.063f}, {3.65f, -0.034f, 1.43f, 0.086f}, {3.61f, -0.033f, 1.39f, 0.094f}}},
+    {128, 64, 256, {{2.95f, 0.410f, 2.01f, 0.975f}, {3.65f, 0.459f, 1.36f, 1.032f}, {4.24f, 0.316f, 1.11f, 1.267f}}},
+    {96, 96, 512, {{3.45f, 0.049f, 2.35f, 1.346f}, {2.94f, 0.089f, 3.19f, 1.353f}, {3.16f, 0.079f, 3.33f, 1.369f}}},
+    {96, 64, 256, {{2.85f, 0.367f, 1.28f, 0.710f}, {3.25f, 0.330f, 1.25f, 0.810f}, {4.04f, 0.346f, 1.00f, 0.899f}}},
+    {96, 64, 512, {{2.98f, 0.131f, 1.94f, 0.746f}, {2.29f, 0.039f, 2.53f, 0.949f}, {2.43f, 0.048f, 2.73f, 1.015f}}},
+    {64, 96, 512, {{3.10f, 0.118f, 1.94f, 0.753f}, {2.11f, 0.026f, 2.88f, 0.981f}, {2.15f, 0.065f, 2.62f, 1.061f}}},
+    {64, 64, 256, {{2.42f, 0.242f, 1.26f, 0.486f}, {2.90f, 0.227f, 0.95f, 0.561f}, {2.89f, 0.305f, 1.02f, 0.565f}}},
+    {64, 64, 512, {{2.98f, 0.075f, 1.39f, 0.520f}, {2.86f, 0.113f, 1.41f, 0.582f}, {2.83f, 0.142f, 1.35f, 0.601f}}},
+    {64, 32, 512, {{1.73f, 0.004f, 1.99f, 0.332f}, {2.00f, -0.002f, 1.82f, 0.386f}, {1.71f, 0.020f, 2.07f, 0.412f}}},
+    {32, 64, 512, {{1.71f, 0.010f, 2.12f, 0.313f}, {1.82f, 0.012f, 1.96f, 0.390f}, {1.75f, 0.013f, 2.07f, 0.409f}}},
+    {32, 32, 256, {{2.74f, 0.063f, 0.65f, 0.162f}, {2.67f, 0.064f, 0.65f, 0.192f}, {2.75f, 0.062f, 0.71f, 0.195f}}},
+    {32, 32, 512, {{2.82f, -0.014f, 1.40f, 0.188f}, {2.19f, -0.004f, 1.73f, 0.218f}, {1.93f, 0.003f, 1.98f, 0.206f}}},
+    {32, 16, 512, {{3.55f, -0.028f, 1.08f, 0.114f}, {3.12f, -0.024f, 1.30f, 0.137f}, {3.24f, -0.026f, 1.18f, 0.155f}}},
+    {16, 32, 512, {{3.10f, -0.022f, 1.15f, 0.114f}, {3.37f, -0.023f, 1.21f, 0.135f}, {3.06f, -0.025f, 1.35f, 0.156f}}},
+    {16, 16, 1024, {{3.61f, -0.031f, 1.37f, 0.063f}, {3.65f, -0.034f, 1.43f, 0.086f}, {3.61f, -0.033f, 1.39f, 0.094f}}},
 };
+constexpr int kSgTileCount = (int)(sizeof(kSgTiles) / sizeof(kSgTiles[0]));
 // The 256 x 256 direct-to-LDS kernel, one tile per CU at a time
 static const float kSgDma[4] = {3.0f, 0.0f, 8.3f, 8.05f};
 
@@ -346,11 +347,14 @@ static int sg_pick(const SgArgs &p, bool ak, bool bk, bool dma, int64_t count) {
     const int mc = !ak + !bk;
     int best = -1;
     float least = dma ? sg_cost(kSgDma, tiles_of(p.M, p.N, SgBig::BM, SgBig::BN) * count, panels) : 3e38f;
-    for (int i = 0; i < (int)(sizeof(kSgTiles) / sizeof(kSgTiles[0])); i++) {
+    for (int i = 0; i < kSgTileCount; i++) {
         const SgTile &t = kSgTiles[i];
-        const float c = sg_cost(t.c[mc], tiles_of(p.M, p.N, t.bm, t.bn) * count, panels);
+        const int64_t tiles = tiles_of(p.M, p.N, t.bm, t.bn) * count;
+        const float c = sg_cost(t.c[mc], tiles, panels);
+        if (tiles > kMaxLanes / t.lanes) continue;  // more lanes than a launch has
         if (c < least) least = c, best = i;
     }
+    if (best < 0 && !dma) return 5;  // no tile's launch is small enough: 64 x 64, whose launch then fails
     return best;
 }
 

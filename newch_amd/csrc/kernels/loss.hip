@@ -769,9 +769,9 @@ extern "C" NC_HIP_API int nc_hip_mse_loss_bwd(int64_t n, const float *d, const f
     if (!d || !gout) return set_error(NC_HIP_ERR_ARG, "nc_hip_mse_loss_bwd: NULL pointer");
     if (!ga && !gb) return NC_HIP_OK;
     const bool al = aligned16(d) && (!ga || aligned16(ga)) && (!gb || aligned16(gb));
-    const int64_t items = al ? (n + 3) / 4 : n, per = (int64_t)(INT32_MAX / 2) * kMseB;
+    const int64_t items = al ? (n + 3) / 4 : n, per = int64_t(1) << 31;
     const float inv = 1.0f / (float)n;
-    for (int64_t i0 = 0; i0 < items; i0 += per) {  // launches of less than 2^30 workgroups
+    for (int64_t i0 = 0; i0 < items; i0 += per) {  // launches of at most 2^31 work-items
         const int64_t e0 = al ? 4 * i0 : i0, left = n - e0, k = std::min(items - i0, per), cnt = std::min(left, al ? 4 * k : k);
         const unsigned grid = (unsigned)((k + kMseB - 1) / kMseB);
         float *pa = ga ? ga + e0 : nullptr, *pb = gb ? gb + e0 : nullptr;

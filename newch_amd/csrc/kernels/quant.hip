@@ -239,7 +239,13 @@ extern "C" NC_HIP_API int nc_hip_quantize_rows(int64_t rows, int64_t cols, const
         return check_launch("nc_hip_quantize_rows");
     }
     const bool al = cols % 4 == 0 && aligned16(w) && ((uintptr_t)q & 3u) == 0;
-    if (rows > INT32_MAX || cols > 65536) {
+    // a launch's rows: four a workgroup of 256 lanes in the wave kernels, one a workgroup in the others
+    const int64_t most = cols < 1024 ? kMaxLanes / kWave / 4 * 4 : kWgRowsPerLaunch;
+    if (cols <= 65536 && rows > most) {
+        const int rc = nc_hip_quantize_rows(most, cols, w, q, scale, stream);
+        return rc ? rc : nc_hip_quantize_rows(rows - most, cols, w + most * cols, q + most * cols, scale + most, stream);
+    }
+    if (cols > 65536) {
         const unsigned g = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         hipLaunchKernelGGL(k_quant_blk, g, kQB, 0, st, w, q, scale, rows, cols);
         return check_launch("nc_hip_quantize_rows");

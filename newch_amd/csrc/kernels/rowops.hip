@@ -1173,7 +1173,7 @@ static int vpl_for(int64_t C) {
 #define NC_LN_BWD_PAIR 1  // k_ln_bwd_pair for rows of 512 and 1024 floats
 #endif
 #ifndef NC_ROWS_GRID_PER_CU
-#define NC_ROWS_GRID_PER_CU 65536
+#define NC_ROWS_GRID_PER_CU 32768  // at 256 CUs and 256 lanes 2^31 work-items; more rows are looped over
 #endif
 static unsigned rows_grid(int64_t rows) {
     const int64_t blocks = (rows + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -1266,7 +1266,12 @@ extern "C" NC_HIP_API int nc_hip_softmax_fwd(int log_form, int64_t rows, int64_t
         else if (al) NC_SM_FWD(false, true)
         else NC_SM_FWD(false, false)
 #undef NC_SM_FWD
-    } else if (C <= kWgRowMax && rows <= INT32_MAX) {  // a workgroup per row
+    } else if (C <= kWgRowMax) {  // a workgroup per row
+        if (rows > kWgRowsPerLaunch) {
+            const int rc = nc_hip_softmax_fwd(log_form, kWgRowsPerLaunch, C, x, y, stream);
+            return rc ? rc : nc_hip_softmax_fwd(log_form, rows - kWgRowsPerLaunch, C, x + kWgRowsPerLaunch * C,
+                                                y + kWgRowsPerLaunch * C, stream);
+        }
         if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, true>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
         else NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, false>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
     } else {
@@ -1296,7 +1301,12 @@ extern "C" NC_HIP_API int nc_hip_softmax_bwd(int log_form, int64_t rows, int64_t
         else if (accumulate) NC_SM_BWD(false, true);
         else NC_SM_BWD(false, false);
 #undef NC_SM_BWD
-    } else if (C <= kWgRowMaxBwd && rows <= INT32_MAX) {
+    } else if (C <= kWgRowMaxBwd) {
+        if (rows > kWgRowsPerLaunch) {
+            const int64_t e = kWgRowsPerLaunch * C;
+            const int rc = nc_hip_softmax_bwd(log_form, kWgRowsPerLaunch, C, y, g, gi, accumulate, stream);
+            return rc ? rc : nc_hip_softmax_bwd(log_form, rows - kWgRowsPerLaunch, C, y + e, g + e, gi + e, accumulate, stream);
+        }
         const dim3 grid((unsigned)rows);
         if (log_form && accumulate) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, true>), grid, NT, 0, st, y, g, gi, (int)C))
         else if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, false>), grid, NT, 0, st, y, g, gi, (int)C))
@@ -1322,7 +1332,13 @@ extern "C" NC_HIP_API int nc_hip_layer_norm_fwd(int64_t rows, int64_t D, const f
         const int v = vpl_for(D);
         if (al) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, true>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
         else NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, false>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
-    } else if (D <= kWgRowMax && rows <= INT32_MAX) {  // a workgroup per row
+    } else if (D <= kWgRowMax) {  // a workgroup per row
+        if (rows > kWgRowsPerLaunch) {
+            const int64_t e = kWgRowsPerLaunch * D;
+            const int rc = nc_hip_layer_norm_fwd(kWgRowsPerLaunch, D, x, w, b, eps, y, stats, stream);
+            return rc ? rc : nc_hip_layer_norm_fwd(rows - kWgRowsPerLaunch, D, x + e, w, b, eps, y + e,
+                                                   stats + 2 * kWgRowsPerLaunch, stream);
+        }
         NC_WG_SWITCH(D, hipLaunchKernelGGL((k_ln_fwd_wg<VP, NT>), dim3((unsigned)rows), NT, 0, st, x, w, b, eps, y, stats, (int)D))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);

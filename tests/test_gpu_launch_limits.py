@@ -1,0 +1,82 @@
+"""Row counts whose workgroups, one launch's worth of lanes each, would not fit a launch: a dispatch counts its work-items
+in 32 bits, so such calls run as several launches or loop."""
+import numpy as np
+import pytest
+
+from newch_amd import hip, hipmem
+from oracle import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+PER_LAUNCH = 1 << 21  # rows a launch of the kernels with a workgroup a row
+
+
+@pytest.fixture(scope="module")
+def K():
+    return hip.Kernels()
+
+
+def test_narrow_rows_past_a_launch(K):
+    """[2^26 + 37, 3]: a wave a row is more than 2^32 lanes; softmax loops over the rows, quantization splits."""
+    rows, C, per = (1 << 26) + 37, 3, 1 << 16
+    rng = np.random.default_rng(5)
+    base = rng.standard_normal((per, C)).astype(np.float32)
+    X = hipmem.DeviceBuffer(rows * C * 4)
+    for r0 in (0, rows - per):  # the rows looked at; the others are zeros
+        if r0 == 0:
+            X.zero()
+        X.upload(base, r0 * C * 4)
+    print(f"softmax, quantize {rows}x{C}", flush=True)
+    Y, Q, S = hipmem.DeviceBuffer(rows * C * 4), hipmem.DeviceBuffer(rows * C), hipmem.DeviceBuffer(rows * 4)
+    K.softmax_fwd(False, rows, C, X.ptr, Y.ptr)
+    K.quantize_rows(rows, C, X.ptr, Q.ptr, S.ptr)
+    hipmem.synchronize()
+    e = np.exp(base.astype(np.float64) - base.max(1, keepdims=True))
+    want = e / e.sum(1, keepdims=True)
+    wq, ws = O.quantize_rows(base)
+    for r0 in (0, rows - per):
+        assert np.abs(Y.to_numpy(np.float32, (per, C), r0 * C * 4) - want).max() < 1e-6
+        assert (Q.to_numpy(np.int8, (per, C), r0 * C) == wq).all()
+        assert (S.to_numpy(np.float32, (per,), r0 * 4) == ws).all()
+    mid = PER_LAUNCH * 16  # zeros: equal shares, scale 1
+    assert np.abs(Y.to_numpy(np.float32, (64, C), mid * C * 4) - 1 / 3).max() < 1e-6
+    assert (S.to_numpy(np.float32, (64,), mid * 4) == 1).all()
+
+
+def test_wide_rows_past_a_launch(K):
+    """[2^21 + 3, 1028]: softmax, LayerNorm and quantization run as two launches; rows on both sides of the seam."""
+    rows, C, per = PER_LAUNCH + 3, 1028, 8
+    rng = np.random.default_rng(6)
+    base = rng.standard_normal((per, C)).astype(np.float32)
+    at = rows - per  # five rows of the first launch and all of the second
+    X, Y = hipmem.DeviceBuffer(rows * C * 4), hipmem.DeviceBuffer(rows * C * 4)
+    X.zero()
+    X.upload(base, at * C * 4)
+    x64 = base.astype(np.float64)
+    print(f"softmax, layer_norm, quantize {rows}x{C}", flush=True)
+    K.softmax_fwd(False, rows, C, X.ptr, Y.ptr)
+    hipmem.synchronize()
+    e = np.exp(x64 - x64.max(1, keepdims=True))
+    y = Y.to_numpy(np.float32, (per, C), at * C * 4)
+    assert np.abs(y - e / e.sum(1, keepdims=True)).max() < 1e-6
+    G = hipmem.DeviceBuffer(rows * C * 4)
+    G.zero()
+    g = rng.standard_normal((per, C)).astype(np.float32)
+    G.upload(g, at * C * 4)
+    K.softmax_bwd(False, rows, C, Y.ptr, G.ptr, X.ptr, accumulate=True)  # x + y (g - <y, g>)
+    hipmem.synchronize()
+    y64 = y.astype(np.float64)
+    want = x64 + y64 * (g - (y64 * g).sum(1, keepdims=True))
+    assert np.abs(X.to_numpy(np.float32, (per, C), at * C * 4) - want).max() < 1e-5
+    X.upload(base, at * C * 4)
+    S = hipmem.DeviceBuffer(rows * 8)
+    K.layer_norm_fwd(rows, C, X.ptr, None, None, 1e-5, Y.ptr, S.ptr)
+    hipmem.synchronize()
+    m, v = x64.mean(1, keepdims=True), x64.var(1, keepdims=True)
+    assert np.abs(Y.to_numpy(np.float32, (per, C), at * C * 4) - (x64 - m) / np.sqrt(v + 1e-5)).max() < 1e-5
+    assert np.abs(S.to_numpy(np.float32, (per, 2), at * 8)[:, 0] - m[:, 0]).max() < 1e-6
+    K.quantize_rows(rows, C, X.ptr, Y.ptr, S.ptr)
+    hipmem.synchronize()
+    wq, ws = O.quantize_rows(base)
+    assert (Y.to_numpy(np.int8, (per, C), at * C) == wq).all()
+    assert (S.to_numpy(np.float32, (per,), at * 4) == ws).all()
