@@ -367,9 +367,13 @@ __device__ __forceinline__ f4 vec_load(const float *p, int D, int j) {
 // the squared deviations of a piece, of its first `left` elements where the row ends in it
 template <bool AL>
 __device__ __forceinline__ double ln_sq_dev(f4 v, double mean, int left) {
+    if constexpr (AL) {
+        const double a = (double)v.x - mean, b = (double)v.y - mean, c = (double)v.z - mean, d = (double)v.w - mean;
+        return (a * a + b * b) + (c * c + d * d);
+    }
     double d[4];
 #pragma unroll
-    for (int c = 0; c < 4; c++) d[c] = AL || c < left ? (double)v[c] - mean : 0.0;
+    for (int c = 0; c < 4; c++) d[c] = c < left ? (double)v[c] - mean : 0.0;
     return (d[0] * d[0] + d[1] * d[1]) + (d[2] * d[2] + d[3] * d[3]);
 }
 
@@ -380,7 +384,7 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
                                                       const float *__restrict__ b, float eps, float *__restrict__ y,
                                                       float *__restrict__ stats, int64_t rows, int D) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int nv = (D + 3) / 4;
+    const int nv = AL ? D / 4 : (D + 3) / 4;
     const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock;
     f4 ww[VPL], bv[VPL];
 #pragma unroll
