@@ -966,6 +966,13 @@ __global__ __launch_bounds__(ln_team_threads(TW), 4) void k_ln_bwd_team(const fl
     if (r < rows) load(r, xv, gv);
     for (int par = 0; r < rows; r += step, par ^= 1) {
         const float mean = stats[2 * r], rstd = stats[2 * r + 1];
+        // Places past the row (g = 0; only the last piece has any) take xhat = 0: (0 - mean) rstd is infinite for a row of
+        // the lowest float, and 0 times that is NaN.
+        if (4 * (t + VPT * NL - NL) + 4 > D) {
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                if (4 * (t + VPT * NL - NL) + c >= D) xv[VPT - 1][c] = mean;
+        }
         f4 old[VPT];
         if (ACC && gx) {
 #pragma unroll

@@ -104,3 +104,38 @@ def test_layer_norm_partial_outputs(K, D):
     np.testing.assert_array_equal(only_x[0], full[0])
     np.testing.assert_array_equal(only_c[1], full[1])
     np.testing.assert_array_equal(only_c[2], full[2])
+
+
+# constant rows: the lowest and the largest float, a mask's -1e9, a large one, the smallest normal
+EXTREMES = [np.finfo(np.float32).min, np.finfo(np.float32).max, -1e9, 1e30, np.finfo(np.float32).tiny]
+
+
+@pytest.mark.parametrize("D", [3, 5, 255, 257, 513, 767, 769, 1023, 1028, 2044, 2049, 3001, 4100, 6146, 8188, 8193, 12287])
+@pytest.mark.parametrize("acc", [False, True])
+def test_layer_norm_bwd_of_extreme_rows(K, D, acc):
+    """Rows of one value whose mean times rstd leaves the fp32 range: xhat is 0 in all of the row, and the gradient finite,
+    whatever the places past the row's end hold."""
+    rng = np.random.default_rng(D)
+    x = np.repeat(np.float32(EXTREMES)[:, None], D, axis=1)
+    x = np.concatenate([x, rng.standard_normal((3, D)).astype(np.float32)])
+    rows = len(x)
+    g, old = (rng.standard_normal((rows, D)).astype(np.float32) for _ in range(2))
+    w = (1 + 0.1 * rng.standard_normal(D)).astype(np.float32)
+    dx, dg, dw, dgx = placed(x, 0), placed(g, 0), placed(w, 0), placed(old, 0)
+    y, dst = placed(x, 0), placed(np.zeros((rows, 2)), 0)
+    dgw, dgb = placed(np.zeros(D), 0), placed(np.zeros(D), 0)
+    n = K.layer_norm_bwd_workspace(rows, D)
+    ws = hipmem.DeviceBuffer.from_numpy(np.zeros(n, np.uint8))
+    print(f"layer_norm extreme rows {rows}x{D} acc={acc}", flush=True)
+    K.layer_norm_fwd(rows, D, dx.ptr, dw.ptr, None, EPS, y.ptr, dst.ptr)
+    K.layer_norm_bwd(rows, D, dx.ptr, dw.ptr, dst.ptr, dg.ptr, dgx.ptr, dgw.ptr, dgb.ptr, ws.ptr, n, accumulate=acc)
+    st = read(dst, (rows, 2), 0)
+    mean, rstd = st[:, :1], st[:, 1:]
+    assert (mean[:len(EXTREMES), 0].astype(np.float32) == x[:len(EXTREMES), 0]).all()
+    G, gh, xh = g.astype(np.float64), g.astype(np.float64) * w, (x - mean) * rstd
+    mg, mgx = gh.mean(1, keepdims=True), (gh * xh).mean(1, keepdims=True)
+    size = rstd * (np.abs(gh) + np.abs(gh).mean(1, keepdims=True) + np.abs(xh) * np.abs(gh * xh).mean(1, keepdims=True))
+    o = old if acc else np.zeros_like(old)
+    near(read(dgx, (rows, D), 0), o + rstd * (gh - mg - xh * mgx), size + np.abs(o))
+    near(read(dgw, (D,), 0), (G * xh).sum(0), np.abs(G * xh).sum(0), 2)
+    near(read(dgb, (D,), 0), G.sum(0), np.abs(G).sum(0), 2)
