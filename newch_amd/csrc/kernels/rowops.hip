@@ -932,12 +932,20 @@ __global__ __launch_bounds__(kLnPairWaves *kWave, 4) void k_ln_bwd_pair(const fl
 // TW = 1: eight waves a workgroup, each with its own rows; else the workgroup is the team, the waves' fp64 sums meet in
 // LDS (two sets of slots in turn, so one barrier a row) and are added in wave order.  A lane keeps the gw / gb
 // partials of its columns over the workgroup's rows in fp64 registers, as the element-by-element kernels do;
-// k_ln_cols_combine adds the workgroups'.  HBM-bound: [16384, 767] 57 -> 44 us, [16384, 3001]
-// 270 -> 136, [16384, 8192] 735 -> 341 (4.7 TB/s) against those; [16384, 2048] 113 -> 80 against a wave per row.
+// k_ln_cols_combine adds the workgroups'.  Against those [16384, 767] 56 -> 45 us, [16384, 1023] 69 -> 59, [16384, 3001]
+// 270 -> 138, [16384, 8192] 732 -> 342 (4.7 TB/s); [16384, 2048] 113 -> 81 against a wave per row.  With two pieces a lane
+// HBM is the bound; with three the sums do not fit 128 registers beside two rows and 8 to 27 of them go to scratch (half of
+// [16384, 767]'s time is not its bytes').
 constexpr int ln_team_threads(int tw) { return tw == 1 ? kLnB : tw * kWave; }
 
+// Waves a SIMD that the register allocation leaves room for.  Two where a wave holds the row and four would put much of it in
+// scratch: at four [16384, 1023] took 117 us (80 registers in scratch; 156 us adding to gx, 112) and takes 59 (68),
+// [16384, 767] adding to gx 73 and takes 57, where the element-by-element kernels took 69 (79) and 63.  [16384, 767] storing
+// gx (8 in scratch) is the faster at four, 45 us against 49, and so are the wider teams, [16384, 3001] 138 against 173.
+constexpr int ln_team_waves(int vpt, int tw, bool acc) { return tw == 1 && (vpt > 3 || (vpt == 3 && acc)) ? 2 : 4; }
+
 template <int VPT, int TW, bool ACC>
-__global__ __launch_bounds__(ln_team_threads(TW), 4) void k_ln_bwd_team(const float *__restrict__ x,
+__global__ __launch_bounds__(ln_team_threads(TW), ln_team_waves(VPT, TW, ACC)) void k_ln_bwd_team(const float *__restrict__ x,
                                                                         const float *__restrict__ w,
                                                                         const float *__restrict__ stats,
                                                                         const float *__restrict__ g,
