@@ -54,6 +54,10 @@ NC_HIP_API uint64_t nc_hip_check_intdiv(const uint32_t *divs, int ndivs, const u
  * for any n: the GPU counterpart of the reference's thread-count determinism (threadpool.c:182-186,
  * engine/tests/test_main.c:1169-1246). */
 NC_HIP_API void nc_hip_set_grid_cus(int n);
+/* Test hook (host only, no device work): the kernel that an int8 product of these sizes runs on -- 0 .. 4 the split-K
+ * tiles 16x16, 16x32, 32x32, 64x32, 64x64, 5 and 6 the 128- and 256-wide tiles, 7 the direct-to-LDS ones (aligned: 16-byte
+ * aligned rows) -- and its launch's work-items; -1 for sizes that are refused. */
+NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int aligned, int64_t *lanes);
 
 /* Activation forward over n contiguous floats: y = f(x).  `s` is the leaky_relu slope / scale
  * factor / added scalar / exponent.  Replaces unary_fwd_span, ops_elementwise.c:229-266 (with the

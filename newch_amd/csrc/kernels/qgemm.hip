@@ -592,7 +592,6 @@ static int launch_qgemm_dma(QgArgs p, bool out_f32, hipStream_t st, const char *
     p.tiles_m = (p.M + kDmaRows - 1) / kDmaRows;
     p.tiles_n = (p.N + kDmaRows - 1) / kDmaRows;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
     static bool done[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !done[dev]) {
@@ -637,7 +636,6 @@ static int launch_qgemm_cfg(QgArgs p, bool out_f32, hipStream_t st, const char *
     p.tiles_m = (p.M + C::BM - 1) / C::BM;
     p.tiles_n = (p.N + C::BN - 1) / C::BN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
     const bool aligned = p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) && aligned16(p.B);
     const dim3 grid((unsigned)blocks), block(C::NT);
     qgemm_lds_attr<C>();
@@ -783,7 +781,6 @@ static int launch_qgemm_ks(QgArgs p, bool out_f32, hipStream_t st, const char *w
     p.tiles_m = (p.M + C::BM - 1) / C::BM;
     p.tiles_n = (p.N + C::BN - 1) / C::BN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
     if (out_f32) hipLaunchKernelGGL((k_qgemm_ks<C, true>), dim3((unsigned)blocks), dim3(C::NT), 0, st, p);
     else hipLaunchKernelGGL((k_qgemm_ks<C, false>), dim3((unsigned)blocks), dim3(C::NT), 0, st, p);
     return check_launch(what);
@@ -802,34 +799,59 @@ static int launch_qgemm_ks(QgArgs p, bool out_f32, hipStream_t st, const char *w
 // largest, of which a CU holds one workgroup, by each tile's start and end (1024 x 4096 x 1024: 28.4 against 17.0).
 // The 128 x 128 tile waits for its panels while a CU has one (10 ns a byte of K) and takes 6.2 when two share it; a
 // 256 x 256 tile 17.
-static int launch_qgemm(QgArgs p, bool out_f32, hipStream_t st, const char *what) {
-    const auto rounds = [&](int bm, int bn) {
-        const int64_t tiles = (int64_t)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
-        return (double)((tiles + num_cus() - 1) / num_cus());
-    };
-    const auto ks = [&](int bm, int bn, int tile) {
-        return 4000 + rounds(bm, bn) * (tile + (double)(bm + bn) * p.K / 36);
-    };
-    const int64_t big_tiles = (int64_t)((p.M + QgBig::BM - 1) / QgBig::BM) * ((p.N + QgBig::BN - 1) / QgBig::BN);
-    const bool big = big_tiles >= num_cus();
+enum QgKernel { QG_KS_16x16, QG_KS_16x32, QG_KS_32x32, QG_KS_64x32, QG_KS_64x64, QG_128, QG_256, QG_DMA };
+struct QgTile {
+    int bm, bn, lanes, cost;  // cost: a tile's start and end, ns
+};
+static const QgTile kQkTiles[] = {  // in the order of QgKernel
+    {16, 16, 1024, 0}, {16, 32, 1024, 0}, {32, 32, 512, 0}, {64, 32, 512, 800}, {64, 64, 256, 2000},
+};
+constexpr int kQkTileCount = (int)(sizeof(kQkTiles) / sizeof(kQkTiles[0]));
+
+static int64_t qg_tiles(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+
+// The kernel for a problem; aligned: K a multiple of 128 and 16-byte aligned rows
+static int qg_pick(int64_t M, int64_t N, int64_t K, bool aligned) {
+    const auto rounds = [&](int bm, int bn) { return (double)((qg_tiles(M, N, bm, bn) + num_cus() - 1) / num_cus()); };
+    const bool big = qg_tiles(M, N, QgBig::BM, QgBig::BN) >= num_cus();
     const double r128 = rounds(QgSmall::BM, QgSmall::BN);
-    const double wide = 5000 + (double)p.K * (big ? 17 * rounds(QgBig::BM, QgBig::BN) : r128 > 1 ? 6.2 * r128 : 10);
-    const double c[5] = {ks(16, 16, 0), ks(16, 32, 0), ks(32, 32, 0), ks(64, 32, 800), ks(64, 64, 2000)};
-    int best = 0;
-    for (int i = 1; i < 5; i++)
-        if (c[i] < c[best]) best = i;
-    if (c[best] < wide) switch (best) {
-        case 0: return launch_qgemm_ks<QkCfg<1, 1, 16>>(p, out_f32, st, what);
-        case 1: return launch_qgemm_ks<QkCfg<1, 2, 16>>(p, out_f32, st, what);
-        case 2: return launch_qgemm_ks<QkCfg<2, 2, 8>>(p, out_f32, st, what);
-        case 3: return launch_qgemm_ks<QkCfg<4, 2, 8>>(p, out_f32, st, what);
-        default: return launch_qgemm_ks<QkCfg<4, 4, 4>>(p, out_f32, st, what);
-        }
-    const bool dma_ok = p.K > 0 && p.K % kDmaBK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) &&
-                        aligned16(p.B);
-    if (big && dma_ok) return launch_qgemm_dma(p, out_f32, st, what);
-    if (big) return launch_qgemm_cfg<QgBig>(p, out_f32, st, what);
-    return launch_qgemm_cfg<QgSmall>(p, out_f32, st, what);
+    double least = 5000 + (double)K * (big ? 17 * rounds(QgBig::BM, QgBig::BN) : r128 > 1 ? 6.2 * r128 : 10);
+    int best = big ? aligned ? QG_DMA : QG_256 : QG_128;
+    for (int i = 0; i < kQkTileCount; i++) {
+        const QgTile &t = kQkTiles[i];
+        if (qg_tiles(M, N, t.bm, t.bn) > kMaxLanes / t.lanes) continue;  // more lanes than a launch has
+        const double c = 4000 + rounds(t.bm, t.bn) * (t.cost + (double)(t.bm + t.bn) * K / 36);
+        if (c < least) least = c, best = i;
+    }
+    return best;
+}
+
+// the work-items of that kernel's launch
+static int64_t qg_lanes(int id, int64_t M, int64_t N, int64_t K) {
+    switch (id) {
+    case QG_128: return qg_tiles(M, N, QgSmall::BM, QgSmall::BN) * QgSmall::NT;
+    case QG_256: return qg_tiles(M, N, QgBig::BM, QgBig::BN) * QgBig::NT;
+    case QG_DMA: return qg_tiles(M, N, kDmaRows, kDmaRows) * (K % (2 * kDmaBK) == 0 ? kPipeNT : kDmaNT);
+    default: return qg_tiles(M, N, kQkTiles[id].bm, kQkTiles[id].bn) * kQkTiles[id].lanes;
+    }
+}
+
+static int launch_qgemm(QgArgs p, bool out_f32, hipStream_t st, const char *what) {
+    const bool aligned = p.K > 0 && p.K % kDmaBK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) &&
+                         aligned16(p.B);
+    const int id = qg_pick(p.M, p.N, p.K, aligned);
+    if (qg_lanes(id, p.M, p.N, p.K) > kMaxLanes)
+        return set_error(NC_HIP_ERR_ARG, "%s: %d x %d exceeds one launch", what, p.M, p.N);
+    switch (id) {
+    case QG_KS_16x16: return launch_qgemm_ks<QkCfg<1, 1, 16>>(p, out_f32, st, what);
+    case QG_KS_16x32: return launch_qgemm_ks<QkCfg<1, 2, 16>>(p, out_f32, st, what);
+    case QG_KS_32x32: return launch_qgemm_ks<QkCfg<2, 2, 8>>(p, out_f32, st, what);
+    case QG_KS_64x32: return launch_qgemm_ks<QkCfg<4, 2, 8>>(p, out_f32, st, what);
+    case QG_KS_64x64: return launch_qgemm_ks<QkCfg<4, 4, 4>>(p, out_f32, st, what);
+    case QG_128: return launch_qgemm_cfg<QgSmall>(p, out_f32, st, what);
+    case QG_256: return launch_qgemm_cfg<QgBig>(p, out_f32, st, what);
+    default: return launch_qgemm_dma(p, out_f32, st, what);
+    }
 }
 
 static bool fits_int(int64_t v) { return v >= 0 && v <= INT32_MAX; }
@@ -837,6 +859,13 @@ static bool fits_int(int64_t v) { return v >= 0 && v <= INT32_MAX; }
 }  // namespace nchip
 
 using namespace nchip;
+
+extern "C" NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int aligned, int64_t *lanes) {
+    if (!fits_int(M) || !fits_int(N) || !fits_int(K)) return -1;
+    const int id = qg_pick(M, N, K, aligned && K > 0 && K % kDmaBK == 0);
+    if (lanes) *lanes = qg_lanes(id, M, N, K);
+    return id;
+}
 
 extern "C" NC_HIP_API int nc_hip_gemm_s8_nt(int64_t M, int64_t N, int64_t K, const int8_t *A, int64_t lda,
                                             const int8_t *B, int64_t ldb, int32_t *C, int64_t ldc, void *stream) {

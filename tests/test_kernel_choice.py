@@ -1,0 +1,28 @@
+"""Which kernel the products run on, asked of the library without a device: every choice is one that a launch can hold (a
+dispatch counts its work-items in 32 bits), whatever the sizes."""
+import pytest
+
+from newch_amd import hip
+
+MOST = 2 ** 32 - 1  # work-items of a launch
+
+
+@pytest.fixture(scope="module")
+def K():
+    return hip.Kernels()
+
+
+# long and thin int8 products: 16 x 16 or 16 x 32 tiles of 1024 lanes are the cheapest by what they load, and 2^22 of them are
+# more lanes than a launch has
+@pytest.mark.parametrize("M,N,Kd", [(16, 1 << 27, 64), (1 << 26, 16, 64), ((1 << 26) + 16, 8, 64), (1 << 15, 1 << 15, 0),
+                                    (1 << 26, 16, 1), (1, 1 << 28, 128), (1 << 28, 1, 4096), (16, (1 << 26) + 1, 64),
+                                    (33, 1 << 27, 100), (65, 1 << 26, 7)])
+@pytest.mark.parametrize("aligned", [False, True])
+def test_int8_product_fits_a_launch(K, M, N, Kd, aligned):
+    kernel, lanes = K.gemm_s8_plan(M, N, Kd, aligned)
+    assert kernel >= 0 and 0 < lanes <= MOST
+
+
+def test_int8_product_of_refused_sizes(K):
+    assert K.gemm_s8_plan(-1, 1, 1, True)[0] == -1
+    assert K.gemm_s8_plan(1, 1 << 31, 1, True)[0] == -1
