@@ -58,6 +58,11 @@ NC_HIP_API void nc_hip_set_grid_cus(int n);
  * tiles 16x16, 16x32, 32x32, 64x32, 64x64, 5 and 6 the 128- and 256-wide tiles, 7 the direct-to-LDS ones (aligned: 16-byte
  * aligned rows) -- and its launch's work-items; -1 for sizes that are refused. */
 NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int aligned, int64_t *lanes);
+/* The same for `count` fp32 products in one call: tiles 0 .. 13 (128x64, 96x96 / 2, 96x64, 96x64 / 2, 64x96 / 2, 64x64, 64x64 / 2,
+ * 64x32 / 4, 32x64 / 4, 32x32 / 4, 32x32 / 8, 32x16 / 8, 16x32 / 8, 16x16 / 16; / n: K over n groups of waves), 14 the
+ * 256x256 direct-to-LDS kernel; -1 where no launch holds them. */
+NC_HIP_API int nc_hip_gemm_f32_plan(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t count, int aligned,
+                                    int64_t *lanes);
 
 /* Activation forward over n contiguous floats: y = f(x).  `s` is the leaky_relu slope / scale
  * factor / added scalar / exponent.  Replaces unary_fwd_span, ops_elementwise.c:229-266 (with the

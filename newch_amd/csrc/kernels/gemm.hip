@@ -287,7 +287,6 @@ static int sg_launch_dma(SgArgs &p, int64_t count, hipStream_t st, const char *w
     p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * count;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
     static bool done[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && !done[dev]) {
@@ -341,22 +340,31 @@ static float sg_cost(const float *c, int64_t tiles, float panels) {
     return t > 4.5f ? t : 4.5f;  // a launch
 }
 
-// the cheapest tile's id, or -1 for the direct-to-LDS kernel (dma: the problem is one it takes)
-static int sg_pick(const SgArgs &p, bool ak, bool bk, bool dma, int64_t count) {
-    const float panels = (float)((p.K + 31) / 32);
+// The cheapest kernel for M x N x K: a tile's id, kSgDmaId for the direct-to-LDS kernel (vec: 16-byte aligned rows), or -1
+// where no launch holds the problem.  *lanes: its work-items.
+constexpr int kSgDmaId = kSgTileCount;
+
+static int sg_pick(int64_t M, int64_t N, int64_t K, bool ak, bool bk, bool vec, int64_t count, int64_t *lanes) {
+    // the direct-to-LDS kernel clamps M/N-contiguous chunks onto the last 4 rows: at least 4 rows there, and whole chunks
+    const bool dma = vec && K > 0 && K % (kSgBK * kSgPanel) == 0 && (ak || (M >= 4 && M % 4 == 0)) &&
+                     (bk || (N >= 4 && N % 4 == 0));
+    const float panels = (float)((K + 31) / 32);
     const int mc = !ak + !bk;
     int best = -1;
+    float least = 3e38f;
+    const auto offer = [&](int id, int bm, int bn, int nt, float margin, const float *c) {
+        const int64_t each = tiles_of(M, N, bm, bn);
+        if (each > kMaxLanes / nt / count) return;  // more lanes than a launch has
+        const float cost = margin * sg_cost(c, each * count, panels);
+        if (cost >= least) return;
+        best = id;
+        least = cost;
+        *lanes = each * count * nt;
+    };
     // Another tile has to beat the direct-to-LDS kernel by more than the fits are off: predicted 0.8% ahead of it at
     // x[8192,4096] W[4096,4096]^T, the 64 x 64 tile ran 2176 us against its 2085.
-    float least = dma ? 0.94f * sg_cost(kSgDma, tiles_of(p.M, p.N, SgBig::BM, SgBig::BN) * count, panels) : 3e38f;
-    for (int i = 0; i < kSgTileCount; i++) {
-        const SgTile &t = kSgTiles[i];
-        const int64_t tiles = tiles_of(p.M, p.N, t.bm, t.bn) * count;
-        const float c = sg_cost(t.c[mc], tiles, panels);
-        if (tiles > kMaxLanes / t.lanes) continue;  // more lanes than a launch has
-        if (c < least) least = c, best = i;
-    }
-    if (best < 0 && !dma) return 5;  // no tile's launch is small enough: 64 x 64, whose launch then fails
+    if (dma) offer(kSgDmaId, SgBig::BM, SgBig::BN, SgBig::NT, 0.94f, kSgDma);
+    for (int i = 0; i < kSgTileCount; i++) offer(i, kSgTiles[i].bm, kSgTiles[i].bn, kSgTiles[i].lanes, 1.0f, kSgTiles[i].c[mc]);
     return best;
 }
 
@@ -368,11 +376,11 @@ static int sg_run(SgArgs &p, int ta, int tb, int64_t count, hipStream_t st, cons
     bool vec = !p.pa && aligned16(p.A) && aligned16(p.B) && p.lda % 4 == 0 && p.ldb % 4 == 0;
     for (int d = 0; d < p.bat.nb; d++) vec = vec && p.bat.st[0][d] % 4 == 0 && p.bat.st[1][d] % 4 == 0;
     const bool ak = !ta, bk = tb != 0;
-    // M/N-contiguous chunks are clamped onto the last 4 rows: at least 4 rows there, and whole chunks
-    const bool dma = vec && p.K > 0 && p.K % (kSgBK * kSgPanel) == 0 && (ak || (p.M >= 4 && p.M % 4 == 0)) &&
-                     (bk || (p.N >= 4 && p.N % 4 == 0));
-    const int id = sg_pick(p, ak, bk, dma, count);
-    if (id < 0) {
+    int64_t lanes = 0;
+    const int id = sg_pick(p.M, p.N, p.K, ak, bk, vec, count, &lanes);
+    if (id < 0)
+        return set_error(NC_HIP_ERR_ARG, "%s: %lld products of %d x %d exceed one launch", what, (long long)count, p.M, p.N);
+    if (id == kSgDmaId) {
 #define NC_SG_DMA(AK_, BK_) \
     if (ak == AK_ && bk == BK_) return sg_launch_dma<SgBig, AK_, BK_>(p, count, st, what);
         NC_SG_DMA(true, true)
@@ -443,6 +451,15 @@ static int64_t host_batch_off(const SgBatch &bd, int o, int64_t idx) {
 }  // namespace nchip
 
 using namespace nchip;
+
+extern "C" NC_HIP_API int nc_hip_gemm_f32_plan(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t count, int aligned,
+                                               int64_t *lanes) {
+    int64_t l = 0;
+    const bool ok = fits_int(M) && fits_int(N) && fits_int(K) && M > 0 && N > 0 && count > 0;
+    const int id = ok ? sg_pick(M, N, K, !ta, tb != 0, aligned != 0, count, &l) : -1;
+    if (lanes) *lanes = l;
+    return id;
+}
 
 extern "C" NC_HIP_API int nc_hip_gemm_f32(int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const float *A,
                                           int64_t lda, const float *B, int64_t ldb, float beta, float *C, int64_t ldc,

@@ -324,7 +324,6 @@ static int sg_tile_launch(SgArgs &p, int64_t count, hipStream_t st, const char *
     p.tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM;
     p.tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
     const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n * count;
-    if (blocks > INT32_MAX) return set_error(NC_HIP_ERR_ARG, "%s: %lld tiles exceed one launch", what, (long long)blocks);
     if constexpr (lds > 64 * 1024) {
         // dynamic LDS above 64 KiB has to be allowed per kernel, once per device
         static bool done[64] = {};

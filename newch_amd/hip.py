@@ -37,6 +37,7 @@ SIGNATURES = {
     "nc_hip_device_count": (c_int, []),
     "nc_hip_check_intdiv": (c_uint64, [POINTER(c_uint32), c_int, POINTER(c_uint32), c_int]),
     "nc_hip_set_grid_cus": (None, [c_int]),
+    "nc_hip_gemm_f32_plan": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int, I64P]),
     "nc_hip_gemm_s8_plan": (c_int, [c_int64, c_int64, c_int64, c_int, I64P]),
     "nc_hip_unary_fwd": (c_int, [c_int, c_float, P, P, c_int64, P]),
     "nc_hip_unary_bwd": (c_int, [c_int, c_float, P, P, P, P, c_int64, c_int, P]),
@@ -126,6 +127,11 @@ class Kernels:
         """Grids of grid-stride kernels sized for n CUs (0: the device's own count); results must not
         change."""
         self.lib.nc_hip_set_grid_cus(int(n))
+
+    def gemm_f32_plan(self, ta, tb, M, N, K, count=1, aligned=True):
+        """(kernel, work-items of its launch) of `count` fp32 products; no device needed."""
+        lanes = c_int64()
+        return self.lib.nc_hip_gemm_f32_plan(ta, tb, M, N, K, count, int(aligned), ctypes.byref(lanes)), lanes.value
 
     def gemm_s8_plan(self, M, N, K, aligned):
         """(kernel, work-items of its launch) of an int8 product; no device needed."""

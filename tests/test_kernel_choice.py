@@ -26,3 +26,16 @@ def test_int8_product_fits_a_launch(K, M, N, Kd, aligned):
 def test_int8_product_of_refused_sizes(K):
     assert K.gemm_s8_plan(-1, 1, 1, True)[0] == -1
     assert K.gemm_s8_plan(1, 1 << 31, 1, True)[0] == -1
+
+
+# batches of small matrices whose 256 x 256 tiles (512 lanes each) no launch holds: another tile runs them, or the call says so
+@pytest.mark.parametrize("M,N,Kd,count,runs", [(256, 256, 32, 1 << 23, False), (4, 4, 32, (1 << 23) + 1, True),
+                                               (32, 32, 32, 16777215, True), (32, 32, 32, 1 << 24, False),
+                                               (16, 16, 4096, 1 << 24, False), (1 << 27, 16, 32, 1, True),
+                                               (2 ** 31 - 1, 1, 1, 1, False), (64, 1 << 28, 64, 1, True)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("aligned", [False, True])
+def test_fp32_product_fits_a_launch(K, ta, tb, M, N, Kd, count, runs, aligned):
+    kernel, lanes = K.gemm_f32_plan(ta, tb, M, N, Kd, count, aligned)
+    assert lanes <= MOST
+    assert (kernel >= 0) == runs
