@@ -73,7 +73,7 @@ typedef int i4u __attribute__((ext_vector_type(4), aligned(1)));
 
 // 16 bytes of a row from r, column k; those from column K on are zeros and not read
 __device__ __forceinline__ i4 row16(const int8_t *r, int k, int K) {
-    if (k + 16 <= K) return (i4) * (const i4u *)r;
+    if (k <= K - 16) return (i4) * (const i4u *)r;
     uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int b = 0; b < 16; b++)
@@ -703,18 +703,19 @@ __global__ __launch_bounds__(C::NT) void k_qgemm_ks(QgArgs p) {
                 for (int j = 0; j < TN; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(s.b[j][h], s.a[i][h], acc[i][j], 0, 0, 0);
     };
+    // counted down: K may end within a turn of 2^31, and the index of the step after its last lie past that
     const int whole = p.K / 128 * 128;
-    int k = wid * 128;
+    int left = whole - wid * 128;
     Step u, v;
-    if (k < whole) load(k, u);
-    while (k < whole) {
-        if (k + 128 * KS < whole) load(k + 128 * KS, v);
+    if (left > 0) load(whole - left, u);
+    while (left > 0) {
+        if (left > 128 * KS) load(whole - left + 128 * KS, v);
         work(u);
-        k += 128 * KS;
-        if (k >= whole) break;
-        if (k + 128 * KS < whole) load(k + 128 * KS, u);
+        left -= 128 * KS;
+        if (left <= 0) break;
+        if (left > 128 * KS) load(whole - left + 128 * KS, u);
         work(v);
-        k += 128 * KS;
+        left -= 128 * KS;
     }
     if (whole < p.K && wid == whole / 128 % KS) {  // the step K ends inside, by the wave whose turn it is
         Step s;

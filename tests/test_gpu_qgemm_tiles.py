@@ -71,3 +71,19 @@ def test_linear_int8_equals_its_steps(K, M, N, Kd, bias):
     q, s = dq.to_numpy(np.int8, M * Kd).reshape(M, Kd), ds.to_numpy(np.float32, M)
     want = product(q, w).astype(np.float32) * s[:, None] * ws + b
     np.testing.assert_array_equal(dy.to_numpy(np.float32, M * N).reshape(M, N), want)
+
+
+@pytest.mark.parametrize("Kd", [2 ** 31 - 1, 2 ** 31 - 129, 2 ** 31 - 2048])
+def test_gemm_s8_longest_rows(K, Kd):
+    """Rows that end at or just short of 2^31 bytes: a step index of 32 bits with a sign would pass its end and go negative.
+    Ones against zeros but for a few places around the steps' edges and the row's end."""
+    a, b = hipmem.DeviceBuffer(Kd), hipmem.DeviceBuffer(Kd)
+    K.fill(a.ptr, 1, 1, Kd)
+    b.zero()
+    at = [0, 127, 128, Kd // 2, Kd - 2049, Kd - 130, Kd - 17, Kd - 16, Kd - 1]
+    for i in at:
+        b.upload(np.array([7], np.int8), i)
+    c = hipmem.DeviceBuffer.from_numpy(np.full(2, GUARD, np.int32))
+    print(f"gemm_s8 1x1x{Kd}", flush=True)
+    K.gemm_s8_nt(1, 1, Kd, a.ptr, Kd, b.ptr, Kd, c.ptr, 1)
+    assert c.to_numpy(np.int32, 2).tolist() == [7 * len(at), GUARD]
