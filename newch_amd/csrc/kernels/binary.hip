@@ -956,7 +956,8 @@ static bool plan_cols(const RedPlan &pl, int mode, ColArgs &c) {
         c.chunk = (pl.K + P - 1) / P;
         c.P = (pl.K + c.chunk - 1) / c.chunk;
     }
-    return true;
+    // the widest column counts (32 rows of 2^27 - 31 columns and more) are more lanes than a launch has
+    return (int64_t)((pl.M + kColW - 1) / kColW) * c.P <= kMaxLanes / kColB;
 }
 
 template <int MODE>

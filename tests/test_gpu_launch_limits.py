@@ -80,3 +80,29 @@ def test_wide_rows_past_a_launch(K):
     wq, ws = O.quantize_rows(base)
     assert (Y.to_numpy(np.int8, (per, C), at * C) == wq).all()
     assert (S.to_numpy(np.float32, (per,), at * 4) == ws).all()
+
+
+def test_column_sums_past_a_launch(K):
+    """[32, 2^27 - 1] summed over its rows: 2^22 groups of 32 columns, 1024 lanes each, are 2^32 lanes."""
+    rows, cols, per = 32, (1 << 27) - 1, 1 << 14
+    assert rows * cols < 2 ** 32 - 1
+    rng = np.random.default_rng(7)
+    G, X = hipmem.DeviceBuffer(rows * cols * 4), hipmem.DeviceBuffer(cols * 4)
+    K.fill(G.ptr, 4, 0x3f800000, rows * cols)
+    starts = (0, cols // 2, cols - per)
+    parts = [rng.standard_normal((rows, per)).astype(np.float32) for _ in starts]
+    for c0, part in zip(starts, parts):
+        for r in range(rows):
+            G.upload(part[r], (r * cols + c0) * 4)
+    n = K.binary_bwd_workspace((rows, cols), (0, 1))
+    ws = hipmem.DeviceBuffer(max(n, 8))
+    print(f"column sums {rows}x{cols}", flush=True)
+    K.binary_bwd("add", 1, (rows, cols), G.ptr, (cols, 1), G.ptr, (cols, 1), G.ptr, (0, 1), X.ptr, (0, 1), ws.ptr, n,
+                 accumulate=False)
+    hipmem.synchronize()
+    for c0, part in zip(starts, parts):
+        t = part.astype(np.float64)
+        got, want = X.to_numpy(np.float32, (per,), c0 * 4), t.sum(0)
+        # an fp64 sum of 32 terms, one rounding to fp32
+        assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -46 * np.abs(t).sum(0)).all()
+    assert (X.to_numpy(np.float32, (per,), per * 4) == rows).all()
