@@ -725,7 +725,7 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
         int64_t ko[4];
         offsets<4>(pl.kept, mi, ko);
         const uint32_t k0 = p * pl.chunk;
-        const uint32_t k1 = min(pl.K, k0 + pl.chunk);
+        const uint32_t k1 = k0 + min(pl.chunk, pl.K - k0);  // K and the chunks' ends reach 2^32: no sum may pass it
         const float *gk = g + ko[0], *q1 = p1 + ko[1], *q2 = p2 + ko[2];
         double inv = 1.0;
         if (one) {
@@ -738,11 +738,12 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
             return grad_d<MODE>((double)gv, (double)v1, (double)v2, alpha);
         };
         double acc = 0.0;
-        for (uint32_t k = k0 + 4 * threadIdx.x; k < k1; k += 4 * kB) {
+        for (uint32_t at = 4 * threadIdx.x; at < k1 - k0; at += 4 * kB) {
+            const uint32_t k = k0 + at;
             int64_t ro[3];
             offsets<3>(pl.red, k, ro);
             const f4 z = {0.f, 0.f, 0.f, 0.f};
-            if (k + 4 <= k1) {
+            if (k1 - k >= 4) {
                 const bool in_row = k - pl.red.div[in].div(k) * w + 4 <= w;
                 const f4 gv = row4<3>(gk, pl.red, 0, ro[0], k, in_row);
                 const f4 v1 = MODE != 0 && !(MODE == 2 && one) ? row4<3>(q1, pl.red, 1, ro[1], k, in_row) : z;

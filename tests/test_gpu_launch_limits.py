@@ -106,3 +106,21 @@ def test_column_sums_past_a_launch(K):
         # an fp64 sum of 32 terms, one rounding to fp32
         assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -46 * np.abs(t).sum(0)).all()
     assert (X.to_numpy(np.float32, (per,), per * 4) == rows).all()
+
+
+@pytest.mark.parametrize("n", [2 ** 32 - 2048, 2 ** 32 - 2047, 2 ** 32 - 1023, 2 ** 32 - 2])
+def test_full_sum_up_to_2_32_elements(K, n):
+    """The gradient of a scalar operand, summed over just under 2^32 elements: the last part of the sum ends where 32 bits do.
+    Ones, and larger values in the last part, at its start and at the very end."""
+    G, X = hipmem.DeviceBuffer(n * 4), hipmem.DeviceBuffer(4)
+    K.fill(G.ptr, 4, 0x3f800000, n)
+    extra = {0: 3e9, n // 2: 1e9, n - (1 << 21): 5e8, n - 4: 2.5e8, n - 2: 1.25e8, n - 1: 2.0 ** 27}
+    for i, v in extra.items():
+        G.upload(np.float32([v]), i * 4)
+    ws_bytes = K.binary_bwd_workspace((n,), (0,))
+    ws = hipmem.DeviceBuffer(max(ws_bytes, 8))
+    print(f"full sum of {n}", flush=True)
+    K.binary_bwd("add", 1, (n,), G.ptr, (1,), G.ptr, (1,), G.ptr, (0,), X.ptr, (0,), ws.ptr, ws_bytes, accumulate=False)
+    hipmem.synchronize()
+    # whole numbers below 2^53: the fp64 sum is exact, and rounded once
+    assert X.to_numpy(np.float32, 1)[0] == np.float32(n - len(extra) + sum(float(np.float32(v)) for v in extra.values()))
