@@ -708,20 +708,25 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_col(const float *__restrict_
 // 16-byte pieces where the operand's innermost stride is 1.  A divisor that is the same for all reduced indices is
 // inverted once, in fp64, where terms like 0 / 0 stay what they are.  The sum over all but the middle dim of
 // [704, 704, 128] with division took 190 us with an element a lane and a division each, and takes 115 (4.4 TB/s).
-template <int MODE>
+// L: the lanes of an item, the workgroup's or a wave's.  Where K is short (row_waves) a workgroup has a few of its lanes at
+// work, and an item's bounds, division and exchange are what it takes: [65536, 7] summed over rows 100 us (168 with
+// division) by workgroups, 64 (116) with an element a lane and no division taken out, 28 (40) by waves.
+template <int MODE, int L>
 __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict__ g, const float *__restrict__ p1,
                                                         const float *__restrict__ p2, RedPlan pl, double alpha,
                                                         double *__restrict__ part) {
     __shared__ double sh[kB / kWave];
+    constexpr uint32_t kItems = kB / L;
     const uint64_t total = (uint64_t)pl.M * pl.P;
+    const uint32_t lane = threadIdx.x % L, sub = kItems == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / L);
     const int in = pl.red.nd - 1;
     const uint32_t w = pl.red.size[in];
     const int od = MODE == 2 ? 1 : 2;  // the divisor's operand
     bool one = MODE == 2 || MODE == 3;
     for (int d = 0; d <= in; d++) one = one && pl.red.st[od][d] == 0;
-    for (uint64_t item = blockIdx.x; item < total; item += gridDim.x) {  // block-uniform loop
-        const uint32_t mi = (uint32_t)(item % pl.M);
-        const uint32_t p = (uint32_t)(item / pl.M);
+    for (uint64_t item = (uint64_t)blockIdx.x * kItems + sub; item < total; item += (uint64_t)gridDim.x * kItems) {  // uniform over an item's lanes
+        const uint32_t p = pl.P == 1 ? 0 : (uint32_t)(item / pl.M);
+        const uint32_t mi = (uint32_t)(item - (uint64_t)p * pl.M);
         int64_t ko[4];
         offsets<4>(pl.kept, mi, ko);
         const uint32_t k0 = p * pl.chunk;
@@ -738,7 +743,13 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
             return grad_d<MODE>((double)gv, (double)v1, (double)v2, alpha);
         };
         double acc = 0.0;
-        for (uint32_t at = 4 * threadIdx.x; at < k1 - k0; at += 4 * kB) {
+        const bool single = L == kWave && pl.K <= kWave;  // an element a lane
+        if (single && lane < pl.K) {
+            int64_t ro[3];
+            offsets<3>(pl.red, lane, ro);
+            acc = term(gk[ro[0]], MODE != 0 ? q1[ro[1]] : 0.0f, MODE == 3 ? q2[ro[2]] : 0.0f);
+        }
+        for (uint32_t at = 4 * lane; !single && at < k1 - k0; at += 4 * L) {
             const uint32_t k = k0 + at;
             int64_t ro[3];
             offsets<3>(pl.red, k, ro);
@@ -758,6 +769,10 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
             }
         }
         acc = wave_sum(acc);
+        if constexpr (L == kWave) {
+            if (lane == 0) part[(size_t)p * pl.M + mi] = acc;
+            continue;
+        }
         if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x / kWave] = acc;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -848,6 +863,9 @@ static bool plan_reduce(const Prepared &p, RedPlan &pl, size_t *ws_need) {
     *ws_need = (size_t)pl.P * pl.M * sizeof(double);
     return true;
 }
+
+// Row mode by waves: short rows, or those of up to four passes of a wave where there are waves enough to fill the CUs.
+static bool row_waves(const RedPlan &pl) { return pl.K <= 4 * kWave || (pl.K <= 16 * kWave && pl.M >= 16 * kPlanCUs); }
 
 // Column sums of one kept and one reduced dim, g[k gr + m] (a bias gradient): a workgroup takes 32 columns and up to
 // `chunk` rows, 16 lanes (two columns, 8 bytes each) by 64 row slices, eight rows of loads in flight a lane; the
@@ -1045,8 +1063,11 @@ static int launch_grad(const float *g, const float *p1, const float *p2, float *
         const unsigned grid = (unsigned)(blocks < 1048576 ? blocks : 1048576);
         hipLaunchKernelGGL(k_grad_reduce_col<MODE>, dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
     } else {
-        const unsigned grid = (unsigned)(items < 1048576 ? items : 1048576);
-        hipLaunchKernelGGL(k_grad_reduce_row<MODE>, dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
+        const bool waves = row_waves(pl);
+        const uint64_t blocks = waves ? (items + kB / kWave - 1) / (kB / kWave) : items;
+        const unsigned grid = (unsigned)(blocks < 1048576 ? blocks : 1048576);
+        if (waves) hipLaunchKernelGGL((k_grad_reduce_row<MODE, kWave>), dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
+        else hipLaunchKernelGGL((k_grad_reduce_row<MODE, kB>), dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
     }
     const unsigned fg = (pl.M + kB - 1) / kB;
     if (acc)

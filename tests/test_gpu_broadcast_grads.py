@@ -94,3 +94,39 @@ def test_strided_operands(K):
         np.testing.assert_array_equal(gx.to_numpy(np.float32, (H, W)), g * view)
     K.binary_bwd("mul", 0, (H, W), dt.ptr, (1, H), da.ptr, c, da.ptr, c, gx.ptr, c, None, 0, accumulate=False)
     np.testing.assert_array_equal(gx.to_numpy(np.float32, (H, W)), g * a)
+
+
+@pytest.mark.parametrize("C", [2, 3, 5, 63, 64, 65, 66, 255, 256, 257, 1023, 1024, 1025])
+@pytest.mark.parametrize("rows", [2, 5, 4095, 4096, 4099])
+@pytest.mark.parametrize("op,which,small", [("add", 1, "b"), ("mul", 1, "b"), ("div", 0, "a"), ("div", 1, "b")])
+def test_row_sums(K, rows, C, op, which, small):
+    """A gradient kept over the rows: by a wave an element or a group a lane, or by a workgroup; divisors of 0, infinity, NaN
+    and subnormals among the rows' shared ones."""
+    rng = np.random.default_rng(rows + C)
+    shape, keep = (rows, C), (1, 0)
+    sha, shb = ((rows, 1), shape) if small == "a" else (shape, (rows, 1))
+    g, a = rng.standard_normal(shape).astype(np.float32), rng.standard_normal(sha).astype(np.float32)
+    b = rng.uniform(0.5, 2, shb).astype(np.float32)
+    if small == "b" and op == "div":
+        special = np.float32([0, np.inf, np.nan, 1e-42, -0.0])[:rows]
+        b[:len(special), 0] = special
+        g[0, 1] = 0
+    full, kept = (C, 1), (1, 0)
+    sa, sb = (kept, full) if small == "a" else (full, kept)
+    old = rng.standard_normal((rows, 1)).astype(np.float32)
+    dg, da, db, dgx = placed(g, 1), placed(a, 1), placed(b, 1), placed(old, 1)
+    n = K.binary_bwd_workspace(shape, kept)
+    ws = hipmem.DeviceBuffer.from_numpy(np.full(n + 8, 0x55, np.uint8))
+    K.binary_bwd(op, which, shape, dg.ptr + 4, full, da.ptr + 4, sa, db.ptr + 4, sb, dgx.ptr + 4, kept, ws.ptr, n,
+                 accumulate=True)
+    assert (ws.to_numpy(np.uint8, n + 8)[n:] == 0x55).all(), "wrote past the workspace"
+    flat = dgx.to_numpy(np.float32, rows + 5)
+    assert flat[0] == 77 and (flat[rows + 1:] == 77).all(), "wrote outside"
+    with np.errstate(all="ignore"):
+        t = parts(op, which, *(v.astype(np.float64) for v in (g, a, b)))
+        want, mag = old[:, 0] + t.sum(1), np.abs(old[:, 0]) + np.abs(t).sum(1)
+        got, plain = flat[1:rows + 1], np.abs(want) < 3e38
+        np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+        np.testing.assert_array_equal(got[~plain & ~np.isnan(want)], want[~plain & ~np.isnan(want)].astype(np.float32))
+        # fp64 sums of up to 1025 terms of a few roundings each, then one rounding to fp32
+        assert (np.abs(got - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -40 * mag)[plain].all()
