@@ -887,8 +887,12 @@ __global__ __launch_bounds__(kColB) void k_grad_cols(const float *__restrict__ g
     typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
     __shared__ double sh[kColB / kWave][kColW];
     const int x = threadIdx.x % kColLanes, y = threadIdx.x / kColLanes;
-    const uint32_t groups = (c.M + kColW - 1) / kColW, p = blockIdx.x / groups;
-    const uint32_t m0 = (blockIdx.x - p * groups) * kColW, m = m0 + 2 * x;
+    // XCD i (blocks b with b % 8 == i) takes the i-th of 8 runs of neighbouring column groups: where rows are not 128-byte
+    // aligned two groups share each row's cache line between them
+    const uint32_t xcd = blockIdx.x & 7, per = gridDim.x >> 3, rem = gridDim.x & 7;
+    const uint32_t id = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    const uint32_t groups = (c.M + kColW - 1) / kColW, p = id / groups;
+    const uint32_t m0 = (id - p * groups) * kColW, m = m0 + 2 * x;
     const uint32_t k0 = p * c.chunk, k1 = min(c.K, k0 + c.chunk);
     // the last column of an odd number is the second of the pair before it
     const bool two = m + 1 < c.M;
@@ -960,23 +964,31 @@ __global__ __launch_bounds__(kColB) void k_grad_cols(const float *__restrict__ g
 
 // The plan's column sums as k_grad_cols takes them.  One chunk up to 2048 rows (32 a lane): splitting further costs the
 // combining launch, about 4 us.  Past that chunks of 512 to 2048 rows, the shorter the fewer column groups there
-// are to fill the CUs; never more partials than the general plan's, which sizes the workspace.
+// are to fill the CUs; with a division of its own for every term 32 of them one after another are the longer wait, and few
+// groups split from 1024 rows on ([2048, 3]: 19.5 us in one chunk, 10.2 in two).  Never more partials than the general plan's,
+// which sizes the workspace.
+// The general plan's lane a column stays for columns enough to fill the CUs so: [32, 1000000] takes 40 us that way, 76
+// here, where a workgroup's start and exchange are paid for 32 rows; with a divisor a column, whose inverse is not paid
+// back over few rows, 61 and 193.
 static bool plan_cols(const RedPlan &pl, int mode, ColArgs &c) {
     if (!pl.inner_kept || pl.kept.nd != 1 || pl.red.nd != 1 || pl.M < 2 || pl.kept.st[0][0] != 1) return false;
     if (pl.K < 32 && pl.M > 4096) return false;  // most slices idle, and columns enough for a lane each
+    if (pl.M >= (1u << 17) && pl.K < (mode == 3 ? 256u : 96u)) return false;
     const auto k01 = [&](int o) { return pl.kept.st[o][0] == 0 || pl.kept.st[o][0] == 1; };
     if ((mode != 0 && !k01(1)) || (mode == 3 && !k01(2))) return false;
     c = ColArgs{pl.M, pl.K, pl.K, 1, pl.red.st[0][0], pl.kept.st[1][0], pl.red.st[1][0], pl.kept.st[2][0],
                 pl.red.st[2][0], pl.kept.st[3][0]};
-    if (pl.K > 2048) {
-        const uint32_t groups = (pl.M + kColW - 1) / kColW;
-        uint32_t P = std::max((pl.K + 2047) / 2048, (kPlanCUs + groups - 1) / groups);
+    const uint32_t groups = (pl.M + kColW - 1) / kColW;
+    const bool divides = (mode == 2 && c.p1r != 0) || (mode == 3 && c.p2r != 0);
+    const uint32_t most = divides && groups <= kPlanCUs / 4 ? 1024 : 2048;
+    if (pl.K > most) {
+        uint32_t P = std::max((pl.K + most - 1) / most, (kPlanCUs + groups - 1) / groups);
         P = std::min({P, (pl.K + 511) / 512, pl.P});
         c.chunk = (pl.K + P - 1) / P;
         c.P = (pl.K + c.chunk - 1) / c.chunk;
     }
     // the widest column counts (32 rows of 2^27 - 31 columns and more) are more lanes than a launch has
-    return (int64_t)((pl.M + kColW - 1) / kColW) * c.P <= kMaxLanes / kColB;
+    return (int64_t)groups * c.P <= kMaxLanes / kColB;
 }
 
 template <int MODE>

@@ -81,3 +81,11 @@ def test_column_sums_not_finite(K):
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     np.testing.assert_allclose(got[ok], want[ok], rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("rows,cols", [(63, 1 << 17), (95, (1 << 17) + 1), (97, (1 << 17) - 1), (255, 1 << 17), (257, (1 << 17) + 3),
+                                       (1024, 5), (1025, 5), (1025, 2049), (2049, 40)])
+@pytest.mark.parametrize("op,which", [("add", 1), ("div", 1), ("div", 0)])
+def test_column_sums_at_the_choice(K, rows, cols, op, which):
+    """Sizes on both sides of the line between a lane a column and the column kernel, and of its first split."""
+    test_column_sums(K, rows, cols, op, which, 0, True)
