@@ -55,9 +55,9 @@ NC_HIP_API uint64_t nc_hip_check_intdiv(const uint32_t *divs, int ndivs, const u
  * engine/tests/test_main.c:1169-1246). */
 NC_HIP_API void nc_hip_set_grid_cus(int n);
 /* Test hook (host only, no device work): the kernel that an int8 product of these sizes runs on -- 0 .. 4 the split-K
- * tiles 16x16, 16x32, 32x32, 64x32, 64x64, 5 and 6 the 128- and 256-wide tiles, 7 the direct-to-LDS ones (aligned: 16-byte
- * aligned rows) -- and its launch's work-items; -1 for sizes that are refused. */
-NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int aligned, int64_t *lanes);
+ * tiles 16x16, 16x32, 32x32, 64x32, 64x64, 5 and 6 the 128- and 256-wide tiles, 7 the direct-to-LDS ones (align: of the
+ * rows, in bytes; f32: with linear_int8's epilogue) -- and its launch's work-items; -1 for sizes that are refused. */
+NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int align, int f32, int64_t *lanes);
 /* The same for `count` fp32 products in one call: tiles 0 .. 13 (128x64, 96x96 / 2, 96x64, 96x64 / 2, 64x96 / 2, 64x64, 64x64 / 2,
  * 64x32 / 4, 32x64 / 4, 32x32 / 4, 32x32 / 8, 32x16 / 8, 16x32 / 8, 16x16 / 16; / n: K over n groups of waves), 14 the
  * 256x256 direct-to-LDS kernel; -1 where no launch holds them. */

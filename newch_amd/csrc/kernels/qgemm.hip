@@ -787,8 +787,13 @@ static int launch_qgemm_ks(QgArgs p, bool out_f32, hipStream_t st, const char *w
     return check_launch(what);
 }
 
-// Which kernel: the one that the costs below call the cheapest, in ns over K bytes for a CU's share of the tiles.
-// The sums are exact in any order, so the choice may follow the device's CU count.  Measured, us (one box):
+// Which kernel: the cheapest by a + L (s + c K + t [K % 128 != 0] + b [K % 16 != 0]) + e K microseconds, L the most tiles a CU
+// gets: a the latency of a launch, s what a tile's start and exchange cost where others run beside it, c its bytes, t and b the
+// step that K ends inside (by 16 bytes, and by single ones); e, of the 128 x 128 tile, the wait for its panels while a CU has
+// one; and f + L g for the float epilogue of the wide tiles.  Least-squares fits, for rows that are 16-byte, 4-byte or not
+// aligned, of all tiles' times at 27 shapes from 1 x 4096 to 8192 x 4096 and K from 1 to 8192: 10 to 25% off on average, the
+// tile chosen by them 1.0% slower than the best on the geometric mean, 1.3% with the float epilogue (by bytes alone, without
+// s, t, b and f, the loss was 39%: 4099 x 4096 x 8 went to 32 x 32 tiles, 172 us against 23).  Measured, us (one box):
 //   M x N x K          16x16  16x32  32x32  64x32  64x64  128x128
 //   16 x 4096 x 4096     6.3    8.1    8.5    9.7   13.4    39.4
 //   16 x 8192 x 8192    17.7   14.4   15.2   17.0   23.8    79.9
@@ -796,53 +801,59 @@ static int launch_qgemm_ks(QgArgs p, bool out_f32, hipStream_t st, const char *w
 //   128 x 4096 x 4096   31.9   26.8   18.3   15.0   19.2    41.6
 //   512 x 4096 x 4096    113     98     61     50     37      46
 //   1024 x 4096 x 4096   224    195    120    100     71      50
-// The split-K tiles go by what they load: (BM + BN) K bytes a tile at about 36 bytes a ns and CU, and the two
-// largest, of which a CU holds one workgroup, by each tile's start and end (1024 x 4096 x 1024: 28.4 against 17.0).
-// The 128 x 128 tile waits for its panels while a CU has one (10 ns a byte of K) and takes 6.2 when two share it; a
-// 256 x 256 tile 17.
+// The 256 x 256 tiles stand for problems that give every CU one; the direct-to-LDS ones among them take 17 ns a byte of K.
+// The sums are exact in any order, so the choice may follow the device's CU count.
 enum QgKernel { QG_KS_16x16, QG_KS_16x32, QG_KS_32x32, QG_KS_64x32, QG_KS_64x64, QG_128, QG_256, QG_DMA };
+struct QgCost {
+    float a, s, c, t, b, e;
+};
 struct QgTile {
-    int bm, bn, lanes, cost;  // cost: a tile's start and end, ns
+    int bm, bn, lanes;
+    float f, g;
+    QgCost by[3];  // rows aligned to 16 bytes, to 4, to none
 };
-static const QgTile kQkTiles[] = {  // in the order of QgKernel
-    {16, 16, 1024, 0}, {16, 32, 1024, 0}, {32, 32, 512, 0}, {64, 32, 512, 800}, {64, 64, 256, 2000},
+static const QgTile kQgTiles[] = {  // in the order of QgKernel
+    {16, 16, 1024, 0, 0, {{3.37f, 0.483f, 0.00062f, 0.28f, 0, 0}, {3.23f, 0.457f, 0.00066f, 0, 0.72f, 0}, {3.23f, 0.616f, 0.00227f, 0.15f, 0.38f, 0}}},
+    {16, 32, 1024, 0, 0, {{3.03f, 0.709f, 0.00108f, 0.79f, 0, 0}, {2.57f, 0.717f, 0.00117f, 0, 1.96f, 0}, {2.69f, 0.975f, 0.00378f, 0.59f, 1.07f, 0}}},
+    {32, 32, 512, 0, 0, {{3.18f, 0.585f, 0.00134f, 0.69f, 0, 0}, {3.14f, 0.534f, 0.00142f, 0, 1.55f, 0}, {3.14f, 0.898f, 0.00472f, 0.34f, 0.80f, 0}}},
+    {64, 32, 512, 0, 0, {{2.96f, 1.760f, 0.00198f, 1.70f, 0, 0}, {2.44f, 1.898f, 0.00215f, 0.17f, 3.85f, 0}, {2.20f, 2.498f, 0.00675f, 1.26f, 2.21f, 0}}},
+    {64, 64, 256, 0, 0, {{2.12f, 3.382f, 0.00289f, 2.33f, 0, 0}, {1.76f, 3.471f, 0.00311f, 0.29f, 5.32f, 0}, {1.68f, 4.096f, 0.00969f, 1.82f, 3.14f, 0}}},
+    {128, 128, QgSmall::NT, 3.7f, 0.45f, {{3.65f, 1.514f, 0.00418f, 0.45f, 0, 0.00474f}, {5.11f, 0, 0.00646f, 0.05f, 2.75f, 0.00547f}, {5.03f, 0.229f, 0.00747f, 1.13f, 1.52f, 0.00469f}}},
+    {256, 256, QgBig::NT, 20, 2.5f, {{0, 13, 0.0140f, 1.1f, 0, 0}, {0, 14, 0.0165f, 3, 2, 0}, {0, 15, 0.0180f, 3, 2, 0}}},
+    {kDmaRows, kDmaRows, kDmaNT, 0, 0, {{5, 0, 0.017f, 0, 0, 0}, {}, {}}},
 };
-constexpr int kQkTileCount = (int)(sizeof(kQkTiles) / sizeof(kQkTiles[0]));
 
 static int64_t qg_tiles(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
-// The kernel for a problem; aligned: K a multiple of 128 and 16-byte aligned rows
-static int qg_pick(int64_t M, int64_t N, int64_t K, bool aligned) {
-    const auto rounds = [&](int bm, int bn) { return (double)((qg_tiles(M, N, bm, bn) + num_cus() - 1) / num_cus()); };
+// The kernel for a problem whose rows are aligned to `align` bytes, -1 where no launch holds it
+static int qg_pick(int64_t M, int64_t N, int64_t K, int align, bool f32) {
+    const int al = align % 16 == 0 && K % 16 == 0 ? 0 : align % 4 == 0 ? 1 : 2;
     const bool big = qg_tiles(M, N, QgBig::BM, QgBig::BN) >= num_cus();
-    const double r128 = rounds(QgSmall::BM, QgSmall::BN);
-    double least = 5000 + (double)K * (big ? 17 * rounds(QgBig::BM, QgBig::BN) : r128 > 1 ? 6.2 * r128 : 10);
-    int best = big ? aligned ? QG_DMA : QG_256 : QG_128;
-    for (int i = 0; i < kQkTileCount; i++) {
-        const QgTile &t = kQkTiles[i];
-        if (qg_tiles(M, N, t.bm, t.bn) > kMaxLanes / t.lanes) continue;  // more lanes than a launch has
-        const double c = 4000 + rounds(t.bm, t.bn) * (t.cost + (double)(t.bm + t.bn) * K / 36);
-        if (c < least) least = c, best = i;
+    const bool dma = big && al == 0 && K > 0 && K % kDmaBK == 0;
+    float least = 3e38f;
+    int best = -1;
+    for (int i = 0; i <= QG_DMA; i++) {
+        const QgTile &t = kQgTiles[i];
+        if (i == QG_DMA ? !dma : i == QG_256 ? !big || dma : false) continue;
+        const int64_t tiles = qg_tiles(M, N, t.bm, t.bn);
+        if (tiles > kMaxLanes / t.lanes) continue;  // more lanes than a launch has
+        const QgCost &c = t.by[al];
+        const float L = (float)((tiles + num_cus() - 1) / num_cus()), k = (float)K;
+        float cost = c.a + L * (c.s + c.c * k + (K % 128 ? c.t : 0) + (K % 16 ? c.b : 0)) + c.e * k;
+        if (f32) cost += t.f + L * t.g;
+        if (cost < least) least = cost, best = i;
     }
     return best;
 }
 
-// the work-items of that kernel's launch
-static int64_t qg_lanes(int id, int64_t M, int64_t N, int64_t K) {
-    switch (id) {
-    case QG_128: return qg_tiles(M, N, QgSmall::BM, QgSmall::BN) * QgSmall::NT;
-    case QG_256: return qg_tiles(M, N, QgBig::BM, QgBig::BN) * QgBig::NT;
-    case QG_DMA: return qg_tiles(M, N, kDmaRows, kDmaRows) * (K % (2 * kDmaBK) == 0 ? kPipeNT : kDmaNT);
-    default: return qg_tiles(M, N, kQkTiles[id].bm, kQkTiles[id].bn) * kQkTiles[id].lanes;
-    }
+static int64_t qg_lanes(int id, int64_t M, int64_t N) {
+    return qg_tiles(M, N, kQgTiles[id].bm, kQgTiles[id].bn) * kQgTiles[id].lanes;
 }
 
 static int launch_qgemm(QgArgs p, bool out_f32, hipStream_t st, const char *what) {
-    const bool aligned = p.K > 0 && p.K % kDmaBK == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) &&
-                         aligned16(p.B);
-    const int id = qg_pick(p.M, p.N, p.K, aligned);
-    if (qg_lanes(id, p.M, p.N, p.K) > kMaxLanes)
-        return set_error(NC_HIP_ERR_ARG, "%s: %d x %d exceeds one launch", what, p.M, p.N);
+    const uint64_t any = (uint64_t)p.lda | (uint64_t)p.ldb | (uintptr_t)p.A | (uintptr_t)p.B;
+    const int id = qg_pick(p.M, p.N, p.K, any % 16 == 0 ? 16 : any % 4 == 0 ? 4 : 1, out_f32);
+    if (id < 0) return set_error(NC_HIP_ERR_ARG, "%s: %d x %d exceeds one launch", what, p.M, p.N);
     switch (id) {
     case QG_KS_16x16: return launch_qgemm_ks<QkCfg<1, 1, 16>>(p, out_f32, st, what);
     case QG_KS_16x32: return launch_qgemm_ks<QkCfg<1, 2, 16>>(p, out_f32, st, what);
@@ -861,10 +872,10 @@ static bool fits_int(int64_t v) { return v >= 0 && v <= INT32_MAX; }
 
 using namespace nchip;
 
-extern "C" NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int aligned, int64_t *lanes) {
+extern "C" NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int align, int f32, int64_t *lanes) {
     if (!fits_int(M) || !fits_int(N) || !fits_int(K)) return -1;
-    const int id = qg_pick(M, N, K, aligned && K > 0 && K % kDmaBK == 0);
-    if (lanes) *lanes = qg_lanes(id, M, N, K);
+    const int id = qg_pick(M, N, K, align, f32 != 0);
+    if (lanes) *lanes = id < 0 ? 0 : qg_lanes(id, M, N);
     return id;
 }
 

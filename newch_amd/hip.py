@@ -38,7 +38,7 @@ SIGNATURES = {
     "nc_hip_check_intdiv": (c_uint64, [POINTER(c_uint32), c_int, POINTER(c_uint32), c_int]),
     "nc_hip_set_grid_cus": (None, [c_int]),
     "nc_hip_gemm_f32_plan": (c_int, [c_int, c_int, c_int64, c_int64, c_int64, c_int64, c_int, I64P]),
-    "nc_hip_gemm_s8_plan": (c_int, [c_int64, c_int64, c_int64, c_int, I64P]),
+    "nc_hip_gemm_s8_plan": (c_int, [c_int64, c_int64, c_int64, c_int, c_int, I64P]),
     "nc_hip_unary_fwd": (c_int, [c_int, c_float, P, P, c_int64, P]),
     "nc_hip_unary_bwd": (c_int, [c_int, c_float, P, P, P, P, c_int64, c_int, P]),
     "nc_hip_binary_fwd": (c_int, [c_int, c_int, I64P, P, I64P, P, I64P, P, I64P, P]),
@@ -133,10 +133,10 @@ class Kernels:
         lanes = c_int64()
         return self.lib.nc_hip_gemm_f32_plan(ta, tb, M, N, K, count, int(aligned), ctypes.byref(lanes)), lanes.value
 
-    def gemm_s8_plan(self, M, N, K, aligned):
+    def gemm_s8_plan(self, M, N, K, align, f32=False):
         """(kernel, work-items of its launch) of an int8 product; no device needed."""
         lanes = c_int64()
-        return self.lib.nc_hip_gemm_s8_plan(M, N, K, int(aligned), ctypes.byref(lanes)), lanes.value
+        return self.lib.nc_hip_gemm_s8_plan(M, N, K, align, int(f32), ctypes.byref(lanes)), lanes.value
 
     def unary_fwd(self, kind, x, y, n, s=0.0, stream=None):
         self._ok(self.lib.nc_hip_unary_fwd(UN[kind], s, x, y, n, stream), "unary_fwd")

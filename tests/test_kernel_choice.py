@@ -17,15 +17,16 @@ def K():
 @pytest.mark.parametrize("M,N,Kd", [(16, 1 << 27, 64), (1 << 26, 16, 64), ((1 << 26) + 16, 8, 64), (1 << 15, 1 << 15, 0),
                                     (1 << 26, 16, 1), (1, 1 << 28, 128), (1 << 28, 1, 4096), (16, (1 << 26) + 1, 64),
                                     (33, 1 << 27, 100), (65, 1 << 26, 7)])
-@pytest.mark.parametrize("aligned", [False, True])
-def test_int8_product_fits_a_launch(K, M, N, Kd, aligned):
-    kernel, lanes = K.gemm_s8_plan(M, N, Kd, aligned)
+@pytest.mark.parametrize("align", [1, 4, 16])
+@pytest.mark.parametrize("f32", [False, True])
+def test_int8_product_fits_a_launch(K, M, N, Kd, align, f32):
+    kernel, lanes = K.gemm_s8_plan(M, N, Kd, align, f32)
     assert kernel >= 0 and 0 < lanes <= MOST
 
 
 def test_int8_product_of_refused_sizes(K):
-    assert K.gemm_s8_plan(-1, 1, 1, True)[0] == -1
-    assert K.gemm_s8_plan(1, 1 << 31, 1, True)[0] == -1
+    assert K.gemm_s8_plan(-1, 1, 1, 16)[0] == -1
+    assert K.gemm_s8_plan(1, 1 << 31, 1, 16)[0] == -1
 
 
 # batches of small matrices whose 256 x 256 tiles (512 lanes each) no launch holds: another tile runs them, or the call says so
@@ -39,3 +40,11 @@ def test_fp32_product_fits_a_launch(K, ta, tb, M, N, Kd, count, runs, aligned):
     kernel, lanes = K.gemm_f32_plan(ta, tb, M, N, Kd, count, aligned)
     assert lanes <= MOST
     assert (kernel >= 0) == runs
+
+
+def test_int8_products_of_short_rows_take_wide_tiles(K):
+    """A tile's start and exchange count where K is short: many small tiles of a few bytes each are not the cheapest."""
+    for M, N, Kd in ((4099, 4096, 8), (3072, 1024, 16), (8192, 300, 32), (768, 3072, 16), (256, 8192, 16), (2048, 1000, 1)):
+        for align in (1, 4, 16):
+            assert K.gemm_s8_plan(M, N, Kd, align)[0] >= 5, (M, N, Kd, align)
+    assert K.gemm_s8_plan(16, 4096, 4096, 16)[0] == 0 and K.gemm_s8_plan(16, 4096, 4096, 16, True)[0] == 0
