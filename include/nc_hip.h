@@ -59,8 +59,8 @@ NC_HIP_API void nc_hip_set_grid_cus(int n);
  * rows, in bytes; f32: with linear_int8's epilogue) -- and its launch's work-items; -1 for sizes that are refused. */
 NC_HIP_API int nc_hip_gemm_s8_plan(int64_t M, int64_t N, int64_t K, int align, int f32, int64_t *lanes);
 /* The same for `count` fp32 products in one call: tiles 0 .. 13 (128x64, 96x96 / 2, 96x64, 96x64 / 2, 64x96 / 2, 64x64, 64x64 / 2,
- * 64x32 / 4, 32x64 / 4, 32x32 / 4, 32x32 / 8, 32x16 / 8, 16x32 / 8, 16x16 / 16; / n: K over n groups of waves), 14 the
- * 256x256 direct-to-LDS kernel; -1 where no launch holds them. */
+ * 64x32 / 4, 32x64 / 4, 32x32 / 4, 32x32 / 8, 32x16 / 8, 16x32 / 8, 16x16 / 16; / n: K over n groups of waves), 14 and 15 the
+ * 256x256 and 128x128 direct-to-LDS kernels; -1 where no launch holds them. */
 NC_HIP_API int nc_hip_gemm_f32_plan(int ta, int tb, int64_t M, int64_t N, int64_t K, int64_t count, int aligned,
                                     int64_t *lanes);
 

@@ -48,7 +48,8 @@ struct SgCfg {
     static constexpr int SLAB_A = 64 * BM, SLAB_B = 64 * BN;
     static constexpr int STAGE = SLAB_A + SLAB_B;
 };
-using SgBig = SgCfg<8, 4, 2, 4>;  // 256 x 256
+using SgBig = SgCfg<8, 4, 2, 4>;   // 256 x 256
+using SgHalf = SgCfg<2, 4, 4, 2>;  // 128 x 128, 8 waves
 
 // ---- operand panels of the direct-to-LDS kernel ---------------------------------------------------
 // One stage of an operand: R rows (M or N) by 16 k in 16-byte chunks.
@@ -175,14 +176,14 @@ __device__ __forceinline__ void write_tiles(const SgArgs &p, const TileAt &at, c
 }
 
 // ------------------------------------------------------------------------------------------------
-// Large aligned problems with K a multiple of 32: the 256 x 256 tile, its operand panels loaded straight
+// Large aligned problems with K a multiple of 32: the 256 x 256 tile (or 128 x 128), its operand panels loaded straight
 // from global memory into LDS (global_load_lds_dwordx4) a summation panel (two stages) ahead through
 // four LDS stages, with no staging registers and no LDS write instructions; one barrier per summation
 // panel.  A stage of an R-row panel is R / 16 load
 // instructions of 1 KiB each: 16 rows of a K-contiguous panel (lane l: row l / 4, the chunk that
 // belongs at position l % 4 under the row's permutation) or 256 / R k-rows of a M/N-contiguous one
 // (lane l: k-row l / (R / 4), position l % (R / 4), loading the rows the k-row's permutation puts
-// there).  The 32 instructions of a stage (16 for A, 16 for B) are dealt four to a wave.  Rows past
+// there).  The 32 (16) instructions of a stage, half of them for A, are dealt four (two) to a wave.  Rows past
 // the matrix are clamped onto its last row (last 4-row chunk), so every load is in bounds.
 constexpr int kSgDmaStages = 4;
 
@@ -331,6 +332,8 @@ static const SgTile kSgTiles[] = {  // in the order of sg_tile_run
 constexpr int kSgTileCount = (int)(sizeof(kSgTiles) / sizeof(kSgTiles[0]));
 // The 256 x 256 direct-to-LDS kernel, one tile per CU at a time
 static const float kSgDma[4] = {3.0f, 0.0f, 8.3f, 8.05f};
+// The 128 x 128 one, two tiles per CU at a time
+static const float kSgHalf[3][4] = {{5.0f, 0.0f, 1.7f, 2.13f}, {5.0f, 0.0f, 1.9f, 2.18f}, {5.0f, 0.0f, 2.0f, 2.24f}};
 
 static int64_t tiles_of(int64_t M, int64_t N, int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
 
@@ -340,9 +343,9 @@ static float sg_cost(const float *c, int64_t tiles, float panels) {
     return t > 4.5f ? t : 4.5f;  // a launch
 }
 
-// The cheapest kernel for M x N x K: a tile's id, kSgDmaId for the direct-to-LDS kernel (vec: 16-byte aligned rows), or -1
-// where no launch holds the problem.  *lanes: its work-items.
-constexpr int kSgDmaId = kSgTileCount;
+// The cheapest kernel for M x N x K: a tile's id, kSgDmaId or kSgHalfId for the direct-to-LDS kernels (vec: 16-byte aligned
+// rows), or -1 where no launch holds the problem.  *lanes: its work-items.
+constexpr int kSgDmaId = kSgTileCount, kSgHalfId = kSgTileCount + 1;
 
 static int sg_pick(int64_t M, int64_t N, int64_t K, bool ak, bool bk, bool vec, int64_t count, int64_t *lanes) {
     // the direct-to-LDS kernel clamps M/N-contiguous chunks onto the last 4 rows: at least 4 rows there, and whole chunks
@@ -365,6 +368,10 @@ static int sg_pick(int64_t M, int64_t N, int64_t K, bool ak, bool bk, bool vec, 
     // x[8192,4096] W[4096,4096]^T, the 64 x 64 tile ran 2176 us against its 2085.
     if (dma) offer(kSgDmaId, SgBig::BM, SgBig::BN, SgBig::NT, 0.94f, kSgDma);
     for (int i = 0; i < kSgTileCount; i++) offer(i, kSgTiles[i].bm, kSgTiles[i].bn, kSgTiles[i].lanes, 1.0f, kSgTiles[i].c[mc]);
+    // The 128 x 128 direct-to-LDS kernel takes over from the tiles that do not split K: the same sums in the same order.  An
+    // operand that is M/N-contiguous costs it next to nothing, the staged tiles 10-15%: A^T B of 8192 x 1024 x 1024 took
+    // 168 us on 64 x 64 tiles, 150 on the staged 128 x 128 ones before them, and 152 here (A^T B^T 170, 156 and 149).
+    if (dma && (best == 0 || best == 2 || best == 5)) offer(kSgHalfId, SgHalf::BM, SgHalf::BN, SgHalf::NT, 1.0f, kSgHalf[mc]);
     return best;
 }
 
@@ -380,9 +387,10 @@ static int sg_run(SgArgs &p, int ta, int tb, int64_t count, hipStream_t st, cons
     const int id = sg_pick(p.M, p.N, p.K, ak, bk, vec, count, &lanes);
     if (id < 0)
         return set_error(NC_HIP_ERR_ARG, "%s: %lld products of %d x %d exceed one launch", what, (long long)count, p.M, p.N);
-    if (id == kSgDmaId) {
-#define NC_SG_DMA(AK_, BK_) \
-    if (ak == AK_ && bk == BK_) return sg_launch_dma<SgBig, AK_, BK_>(p, count, st, what);
+    if (id >= kSgDmaId) {
+#define NC_SG_DMA(AK_, BK_)                                                                  \
+    if (ak == AK_ && bk == BK_)                                                              \
+        return id == kSgDmaId ? sg_launch_dma<SgBig, AK_, BK_>(p, count, st, what) : sg_launch_dma<SgHalf, AK_, BK_>(p, count, st, what);
         NC_SG_DMA(true, true)
         NC_SG_DMA(true, false)
         NC_SG_DMA(false, true)

@@ -1,5 +1,5 @@
-"""The fp32 GEMM's register-staged tiles at their edges, against fp64: every tile shape in every operand layout, with
-rows, columns and k that end inside a tile or a panel, operands that start off 16 bytes with odd leading dims, and
+"""The fp32 GEMM's kernels at their edges, against fp64: every kernel in every operand layout (each asserted), with rows,
+columns and k that end inside a tile or a panel, operands that start off 16 bytes with odd leading dims, and
 matrices of 1 to 3 rows.  What lies between the rows of the operands is NaN (nothing outside them may reach a
 sum) and of C a guard value.  The bound is the K-term one of the other GEMM tests (pyoracle.gemm_excess)."""
 import ctypes
@@ -14,8 +14,7 @@ pytestmark = pytest.mark.gpu
 
 GUARD = np.float32(12345.0)
 
-# by layout (ta, tb), sizes that the choice by shape sends to 16 x 16 / 16 ways, 16 x 32, 32 x 16, 32 x 32 / 4 and / 8,
-# 32 x 64, 64 x 32, 64 x 64 / 1 and / 2, 64 x 96, 96 x 64 / 1 and / 2, 96 x 96 and 128 x 64 tiles
+# by layout (ta, tb): small and thin sizes, short K, K within a panel (which kernel each runs on: BY_KERNEL below)
 SIZES = {
     (0, 1): [(1, 1, 476), (8, 520, 700), (1, 1, 220), (4760, 2, 269), (1, 1, 75), (199, 615, 559), (156, 2863, 36),
              (1, 1, 36), (33, 65, 31), (1, 1, 1), (2763, 170, 172), (204, 5476, 5), (137, 5793, 2), (1482, 689, 107),
@@ -92,3 +91,51 @@ def test_gemm_f32_tiles_pointer_batch(K, ta, tb, M, N, Kd, count):
         assert (flat[:i % 3] == GUARD).all() and (flat[i % 3 + M * N:] == GUARD).all(), "wrote outside C"
         opA, opB = (A[i].T if ta else A[i]).astype(np.float64), (B[i].T if tb else B[i]).astype(np.float64)
         assert O.gemm_excess(got, opA @ opB, np.abs(opA) @ np.abs(opB), Kd) <= 1.0, f"matrix {i}"
+
+
+# by layout, one size for each kernel in gemm_f32_plan's order: the 14 register-staged tiles (operands not 16-byte aligned, K
+# ending inside a panel), then the 256 x 256 and 128 x 128 direct-to-LDS ones (aligned operands)
+BY_KERNEL = {
+    (0, 0): [(4674, 644, 34), (3447, 604, 33), (129, 5702, 34), (1355, 739, 65), (5001, 266, 33), (68, 6068, 33),
+             (6097, 67, 139), (33, 4411, 73), (37, 4183, 33), (1, 1, 33), (4892, 17, 490), (1, 1, 225), (1, 4186, 262),
+             (1, 1, 323), (2308, 5152, 96), (584, 4900, 96)],
+    (0, 1): [(3375, 2244, 33), (3447, 604, 33), (129, 5702, 34), (353, 2761, 98), (5001, 266, 33), (68, 6068, 33),
+             (65, 5896, 178), (1, 1, 33), (79, 4110, 34), (1, 1, 65), (18, 4171, 570), (4397, 1, 283), (1, 1, 193),
+             (1, 1, 385), (2116, 5732, 96), (584, 4900, 96)],
+    (1, 0): [(938, 5749, 33), (3447, 604, 33), (461, 6186, 41), (4603, 309, 35), (129, 5702, 34), (68, 6068, 33),
+             (5914, 71, 65), (37, 4183, 33), (79, 4110, 34), (1, 1, 33), (17, 4297, 334), (1, 1, 225), (1, 4186, 262),
+             (1, 1, 257), (2308, 4572, 96), (584, 4900, 96)],
+    (1, 1): [(4674, 644, 34), (3447, 604, 33), (129, 5702, 34), (1355, 739, 65), (5001, 266, 33), (68, 6068, 33),
+             (6097, 67, 139), (33, 4411, 73), (37, 4183, 33), (1, 1, 33), (4892, 17, 490), (1, 1, 225), (1, 4186, 262),
+             (1, 1, 323), (2308, 5152, 96), (584, 4900, 96)],
+}
+
+
+@pytest.mark.parametrize("ta,tb,kernel", [(ta, tb, k) for ta, tb in BY_KERNEL for k in range(16)])
+def test_gemm_f32_by_kernel(K, ta, tb, kernel):
+    M, N, Kd = BY_KERNEL[ta, tb][kernel]
+    aligned = kernel >= 14
+    assert K.gemm_f32_plan(ta, tb, M, N, Kd, 1, aligned)[0] == kernel, "the choice has moved: another size has to cover it"
+    if not aligned:
+        test_gemm_f32_tiles(K, ta, tb, M, N, Kd)
+        return
+    rng = np.random.default_rng(M + 3 * N + 7 * Kd + ta + 2 * tb)
+    A = rng.standard_normal((Kd, M) if ta else (M, Kd)).astype(np.float32)
+    B = rng.standard_normal((N, Kd) if tb else (Kd, N)).astype(np.float32)
+    lda, ldb, ldc = A.shape[1] + 4, B.shape[1] + 8, N + 1
+    print(f"gemm kernel {kernel} ta={ta} tb={tb} {M}x{N}x{Kd}", flush=True)
+    Ad, Bd = padded(A, lda, 4), padded(B, ldb, 8)
+    Cd = hipmem.DeviceBuffer.from_numpy(np.full((M, ldc), GUARD, np.float32))
+    K.gemm_f32(ta, tb, M, N, Kd, 1.0, Ad.ptr + 16, lda, Bd.ptr + 32, ldb, 0.0, Cd.ptr, ldc)
+    hipmem.synchronize()
+    got = Cd.to_numpy(np.float32, (M, ldc))
+    assert (got[:, N:] == GUARD).all(), "wrote past N"
+    opA, opB = (A.T if ta else A).astype(np.float64), (B.T if tb else B).astype(np.float64)
+    assert O.gemm_excess(got[:, :N], opA @ opB, np.abs(opA) @ np.abs(opB), Kd) <= 1.0
+    # the same sums from operands that are not aligned, which go to a staged tile: the same bits where it does not split K
+    other = K.gemm_f32_plan(ta, tb, M, N, Kd, 1, False)[0]
+    if other in (0, 2, 5):
+        Au, Bu = padded(A, A.shape[1] + 3, 1), padded(B, B.shape[1] + 1, 2)
+        K.gemm_f32(ta, tb, M, N, Kd, 1.0, Au.ptr + 4, A.shape[1] + 3, Bu.ptr + 8, B.shape[1] + 1, 0.0, Cd.ptr, ldc)
+        hipmem.synchronize()
+        np.testing.assert_array_equal(Cd.to_numpy(np.float32, (M, ldc)), got)
