@@ -151,14 +151,14 @@ static nc_status loss_shape(nc_node *n, OutSpec &out) {
     return NC_OK;
 }
 
-// The loss forwards' bad-label key lands in a pinned host word the kernel writes directly (mapped
-// into the device's address space), so the host reads it after the stream synchronisation the
-// reference's synchronous error needs anyway, with no device-to-host copy.  Null when the host
-// allocation is refused: the key then goes through arena memory and a copy.
+// The loss forwards' bad-label key lands in a pinned, coherent host word the kernel stores to at system scope (mapped into the
+// device's address space), so the host sees it while the stream still runs, with no device-to-host copy: the
+// reference's error is a synchronous one.  Null when the host allocation is refused: the key then goes through arena memory
+// and a copy.
 static uint64_t *loss_flag_dev(nc_ctx *ctx) {
     if (!ctx->loss_flag) {
         void *h = nullptr, *d = nullptr;
-        if (hipHostMalloc(&h, sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable) != hipSuccess || !h) {
+        if (hipHostMalloc(&h, sizeof(uint64_t), hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess || !h) {
             (void)hipGetLastError();
             return nullptr;
         }

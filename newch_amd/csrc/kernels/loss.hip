@@ -377,7 +377,9 @@ __global__ __launch_bounds__(kLB) void k_loss_finish(const double *__restrict__ 
     block_sum_min(t, kb, S, kb);
     if (threadIdx.x == 0) {
         *loss = sum ? (float)S : N ? (float)(S / (double)N) : __builtin_nanf("");
-        *bad = kb;
+        // at system scope: *bad may be host memory that the host watches while the kernel runs.  It reads nothing else there
+        // that this kernel wrote, so the store needs no order
+        __hip_atomic_store(bad, kb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
