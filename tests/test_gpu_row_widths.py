@@ -128,3 +128,41 @@ def test_cross_entropy_widths(K, C):
     K.cross_entropy_fwd(rows, C, X.ptr, L2.ptr, S.ptr, loss.ptr, bad.ptr, ws.ptr, nws)
     hipmem.synchronize()
     assert bad.to_numpy(np.uint64, 1)[0] == np.uint64((5 << 32) | C)
+
+
+@pytest.mark.parametrize("C", [1025, 1028, 4097, 16385, 16388, 50257])
+@pytest.mark.parametrize("off", [0, 1])
+def test_cross_entropy_special_rows(K, C, off):
+    """Rows with NaN first, NaN in a late wave, nothing but -inf, +inf in one wave, and whole waves of -inf beside finite
+    values: one row a call, so that each loss stands for its row; against the oracle's loss and statistics."""
+    rng = np.random.default_rng(C)
+    base = (rng.standard_normal(C) * 3).astype(np.float32)
+    rows = {name: base.copy() for name in ("plain", "nan first", "nan late", "all -inf", "inf early", "inf late", "waves of -inf",
+                                            "last alone")}
+    rows["nan first"][0] = np.nan
+    rows["nan late"][C - 2] = np.nan
+    rows["all -inf"][:] = -np.inf
+    rows["inf early"][5] = np.inf
+    rows["inf late"][C - 1] = np.inf
+    rows["waves of -inf"][:C // 2] = -np.inf
+    rows["last alone"][:C - 1] = -np.inf
+    nws = K.loss_workspace(1, C)
+    S, loss, bad, ws = (hipmem.DeviceBuffer(n) for n in (8, 4, 8, max(nws, 8)))
+    for name, x in rows.items():
+        for label in (0, C // 3, C - 1):
+            X, Lb = Off(x[None], off), hipmem.DeviceBuffer.from_numpy(np.array([label], np.int32))
+            print(f"cross entropy 1x{C} offset {off}: {name}, label {label}", flush=True)
+            K.cross_entropy_fwd(1, C, X.ptr, Lb.ptr, S.ptr, loss.ptr, bad.ptr, ws.ptr, nws)
+            hipmem.synchronize()
+            got = loss.to_numpy(np.float32, 1)[0]
+            with np.errstate(all="ignore"):
+                want, prob_o = O.cross_entropy_fwd(x[None], np.array([label], np.int32))
+                prob = ce_prob(x[None], S.to_numpy(np.float32, (1, 2)))
+            assert bad.to_numpy(np.uint64, 1)[0] == np.uint64(0xFFFFFFFFFFFFFFFF)
+            assert (np.isnan(prob) == np.isnan(prob_o)).all(), f"{name}: statistics"
+            ok = ~np.isnan(prob_o)
+            assert np.allclose(prob[ok], prob_o[ok], rtol=1e-5, atol=1e-30), f"{name}: statistics"
+            if not np.isfinite(want):
+                assert np.array_equal(got, np.float32(want), equal_nan=True), (name, got, want)
+            else:  # log(sum) rounded, the label's difference, their difference
+                assert abs(got - want) <= 4 * 2.0 ** -24 * (abs(want) + 12), (name, got, want)
