@@ -286,13 +286,14 @@ __device__ __forceinline__ void dma16(const void *g, uint32_t lds) {
 // ------------------------------------------------------------------------------------------------
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// piece j of a row of C floats, `pad` in the places past its end; AL: the row is 16-byte aligned and C % 4 == 0
-template <bool AL>
+// piece j of a row of C floats, `pad` in the places past its end; AL: the row is 16-byte aligned and C % 4 == 0; NT: other rows
+// streamed past the caches as well
+template <bool AL, bool NT = true>
 __device__ __forceinline__ f4 row_load(const float *row, int C, int j, float pad) {
     if constexpr (AL) {
         return __builtin_nontemporal_load((const f4 *)row + j);
     } else {
-        if (4 * j + 4 <= C) return __builtin_nontemporal_load((const f4u *)(row + 4 * j));
+        if (4 * j + 4 <= C) return NT ? __builtin_nontemporal_load((const f4u *)(row + 4 * j)) : *(const f4u *)(row + 4 * j);
         f4 v = {pad, pad, pad, pad};
 #pragma unroll
         for (int e = 0; e < 3; e++)

@@ -107,8 +107,11 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
 }
 
 // One wave per row; the row's gi (when accumulating) and the next row's y, g are requested before
-// the current row is reduced.
-template <int VPL, bool LOG, bool ACC, bool AL>
+// the current row is reduced.  NT (rows that are not aligned): loads that stream past the caches, for tensors that do not
+// fit them.  Where they do, rows whose lines are shared by two pieces and two rows are the slower for it: with y, g and gi
+// in the caches [20000, 767] takes 40 us so and 31 without (30 element by element), [65536, 767], 600 MB, 117 and 115,
+// [65536, 640] 77 and 89.
+template <int VPL, bool LOG, bool ACC, bool AL, bool NT>
 __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restrict__ y, const float *__restrict__ g,
                                                            float *__restrict__ gi, int64_t rows, int C) {
     const int lane = threadIdx.x & (kWave - 1);
@@ -119,8 +122,8 @@ __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restri
         for (int k = 0; k < VPL; k++) {
             const int j = lane + k * kWave;
             if (j < nv) {
-                vy[k] = row_load<AL>(y + r * C, C, j, 0.0f);
-                vg[k] = row_load<AL>(g + r * C, C, j, 0.0f);
+                vy[k] = row_load<AL, NT>(y + r * C, C, j, 0.0f);
+                vg[k] = row_load<AL, NT>(g + r * C, C, j, 0.0f);
             }
         }
     };
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(kRowB) void k_softmax_bwd_reg(const float *__restri
         if (ACC) {
 #pragma unroll
             for (int k = 0; k < VPL; k++)
-                if (lane + k * kWave < nv) go[k] = row_load<AL>(orow, C, lane + k * kWave, 0.0f);
+                if (lane + k * kWave < nv) go[k] = row_load<AL, NT>(orow, C, lane + k * kWave, 0.0f);
         }
         if (r + stride < rows) load(r + stride, ny, ng);
         double s = 0.0;
@@ -1310,16 +1313,22 @@ extern "C" NC_HIP_API int nc_hip_softmax_bwd(int log_form, int64_t rows, int64_t
     const int v = C <= kWaveRowMax ? vpl_for(C) : 0;
     const unsigned rg = rows_grid(rows);
     if (v) {
-#define NC_SM_BWD(LOG_, ACC_)                                                                                                      \
-    do {                                                                                                                           \
-        if (al) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, LOG_, ACC_, true>), rg, kRowB, 0, st, y, g, gi, rows, (int)C)) \
-        else NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, LOG_, ACC_, false>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))   \
+        // 96 MiB a tensor: the three of them, about what the last cache holds
+        const bool cached = rows * C <= (int64_t(24) << 20);
+#define NC_SM_BWD_AS(LOG_, ACC_, AL_, NT_) \
+    NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_softmax_bwd_reg<VP, LOG_, ACC_, AL_, NT_>), rg, kRowB, 0, st, y, g, gi, rows, (int)C))
+#define NC_SM_BWD(LOG_, ACC_)                               \
+    do {                                                    \
+        if (al) NC_SM_BWD_AS(LOG_, ACC_, true, true)        \
+        else if (cached) NC_SM_BWD_AS(LOG_, ACC_, false, false) \
+        else NC_SM_BWD_AS(LOG_, ACC_, false, true)          \
     } while (0)
         if (log_form && accumulate) NC_SM_BWD(true, true);
         else if (log_form) NC_SM_BWD(true, false);
         else if (accumulate) NC_SM_BWD(false, true);
         else NC_SM_BWD(false, false);
 #undef NC_SM_BWD
+#undef NC_SM_BWD_AS
     } else if (C <= kWgRowMaxBwd) {
         if (rows > kWgRowsPerLaunch) {
             const int64_t e = kWgRowsPerLaunch * C;

@@ -166,3 +166,40 @@ def test_cross_entropy_special_rows(K, C, off):
                 assert np.array_equal(got, np.float32(want), equal_nan=True), (name, got, want)
             else:  # log(sum) rounded, the label's difference, their difference
                 assert abs(got - want) <= 4 * 2.0 ** -24 * (abs(want) + 12), (name, got, want)
+
+
+@pytest.mark.parametrize("C", [77, 257, 513, 1023])
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("log_form,acc", [(False, True), (True, False)])
+def test_softmax_bwd_around_the_caches(K, C, over, log_form, acc):
+    """The last row count of unaligned rows that is loaded through the caches, and the first that is not."""
+    rows = (24 << 20) // C + over
+    rng = np.random.default_rng(C + over)
+    per = 64
+    at = [0, rows // 2, rows - per]
+    parts = [[rng.standard_normal((per, C)).astype(np.float32) for _ in range(3)] for _ in at]
+    bufs = [hipmem.DeviceBuffer((rows * C + 5) * 4) for _ in range(3)]
+    for b in bufs:
+        b.zero()
+        b.upload(np.float32([GUARD]), 0)
+        b.upload(np.full(4, GUARD, np.float32), (rows * C + 1) * 4)
+    for r0, part in zip(at, parts):
+        for b, a in zip(bufs, part):
+            b.upload(a, (r0 * C + 1) * 4)
+    y, g, gi = (b.ptr + 4 for b in bufs)
+    print(f"softmax bwd {rows}x{C} log={log_form}", flush=True)
+    K.softmax_bwd(log_form, rows, C, y, g, gi, accumulate=acc)
+    hipmem.synchronize()
+    for r0, (py, pg, old) in zip(at, parts):
+        got = bufs[2].to_numpy(np.float32, (per, C), (r0 * C + 1) * 4)
+        Y, G = py.astype(np.float64), pg.astype(np.float64)
+        if log_form:
+            p = np.exp(Y)
+            want, size = G - p * G.sum(1, keepdims=True), np.abs(G) + p * np.abs(G).sum(1, keepdims=True)
+        else:
+            want = Y * (G - (G * Y).sum(1, keepdims=True))
+            size = np.abs(Y) * (np.abs(G) + np.abs(G * Y).sum(1, keepdims=True))
+        o = old if acc else np.zeros_like(old)
+        assert_close64(got, o + want, np.abs(o) + size, f"rows {r0}")
+    assert bufs[2].to_numpy(np.float32, 1)[0] == GUARD
+    assert (bufs[2].to_numpy(np.float32, 4, (rows * C + 1) * 4) == GUARD).all()
