@@ -48,14 +48,14 @@ __global__ __launch_bounds__(kRowB) void k_softmax_fwd_reg(const float *__restri
         m = wave_max_nan_skip(m);
         m = row_max_finish(m, lane0_f32(v[0].x));  // lane 0 holds the row's first element
         // the row sum: plain softmax needs exp8's values themselves (outputs); log_softmax only their
-        // sum, whose terms come from the hardware exponential (exp_sum_term) on aligned rows
+        // sum, whose terms come from the hardware exponential (exp_sum_term) on aligned rows of up to 1024 floats
         double s = 0.0;
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
             const int j = lane + k * kWave;
             if (j < nv) {
                 f4 e;
-                if (LOG && AL) {
+                if (LOG && AL && VPL <= 4) {
                     e.x = exp_sum_term(v[k].x - m);
                     e.y = exp_sum_term(v[k].y - m);
                     e.z = exp_sum_term(v[k].z - m);
@@ -351,6 +351,12 @@ __global__ __launch_bounds__(NT) void k_softmax_bwd_wg(const float *__restrict__
 // Rows of up to 1024 floats: a wave per row.  A ragged [65536, 197] ran 84 us forward element by element, 28 as a wave.
 constexpr int64_t kWaveRowMax = 1024, kWgRowMax = 65536;
 constexpr int64_t kWgRowMaxBwd = 32768;  // two rows in registers
+// Aligned rows of up to 2048 floats: forward, a wave per row is the faster while there are waves enough and the tensors stay
+// in the caches, a workgroup per row otherwise.  us, wave / workgroup: softmax of [1000, 2048] 5.5 / 4.8, [4000, 2048]
+// 9.2 / 13.0, [4000, 1280] 6.6 / 9.4, [16384, 2048] 45 / 41; LayerNorm 5.4 / 5.1, 12.7 / 14.9, 8.4 / 11.0, 47 / 44.
+static bool wave_of_8(int64_t rows, int64_t C, bool al) {
+    return al && C <= 2048 && rows >= 6 * kPlanCUs && rows * C <= (int64_t(16) << 20);
+}
 
 // ------------------------------------------------------------------------------------------------
 // LayerNorm
@@ -1288,6 +1294,9 @@ extern "C" NC_HIP_API int nc_hip_softmax_fwd(int log_form, int64_t rows, int64_t
         else if (al) NC_SM_FWD(false, true)
         else NC_SM_FWD(false, false)
 #undef NC_SM_FWD
+    } else if (wave_of_8(rows, C, al)) {
+        if (log_form) hipLaunchKernelGGL((k_softmax_fwd_reg<8, true, true>), rows_grid(rows), kRowB, 0, st, x, y, rows, (int)C);
+        else hipLaunchKernelGGL((k_softmax_fwd_reg<8, false, true>), rows_grid(rows), kRowB, 0, st, x, y, rows, (int)C);
     } else if (C <= kWgRowMax) {  // a workgroup per row
         if (rows > kWgRowsPerLaunch) {
             const int rc = nc_hip_softmax_fwd(log_form, kWgRowsPerLaunch, C, x, y, stream);
@@ -1360,6 +1369,8 @@ extern "C" NC_HIP_API int nc_hip_layer_norm_fwd(int64_t rows, int64_t D, const f
         const int v = vpl_for(D);
         if (al) NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, true>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
         else NC_VPL_SWITCH4(v, hipLaunchKernelGGL((k_ln_fwd_reg<VP, false>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D))
+    } else if (wave_of_8(rows, D, al)) {
+        hipLaunchKernelGGL((k_ln_fwd_reg<8, true>), rows_grid(rows), kRowB, 0, st, x, w, b, eps, y, stats, rows, (int)D);
     } else if (D <= kWgRowMax) {  // a workgroup per row
         if (rows > kWgRowsPerLaunch) {
             const int64_t e = kWgRowsPerLaunch * D;

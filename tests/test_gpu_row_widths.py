@@ -203,3 +203,33 @@ def test_softmax_bwd_around_the_caches(K, C, over, log_form, acc):
         assert_close64(got, o + want, np.abs(o) + size, f"rows {r0}")
     assert bufs[2].to_numpy(np.float32, 1)[0] == GUARD
     assert (bufs[2].to_numpy(np.float32, 4, (rows * C + 1) * 4) == GUARD).all()
+
+
+@pytest.mark.parametrize("rows,C", [(1535, 1028), (1536, 1028), (1537, 1536), (8192, 2048), (8193, 2048), (1600, 2044), (1536, 2052)])
+def test_forward_rows_at_the_choice_by_rows(K, rows, C):
+    """Aligned rows of 1028 to 2048 floats on both sides of where a wave takes a row: softmax, log_softmax and LayerNorm."""
+    rng = np.random.default_rng(rows + C)
+    x = (rng.standard_normal((rows, C)) * 3).astype(np.float32)
+    x[0, C - 1] = x[0].max() + 1
+    x[1, C // 2] = -np.inf
+    x[2] = np.finfo(np.float32).min
+    w, b = rng.standard_normal(C).astype(np.float32), rng.standard_normal(C).astype(np.float32)
+    X, Y, W, B = Off(x, 0), Off(np.zeros_like(x), 0), Off(w, 0), Off(b, 0)
+    x64 = x.astype(np.float64)
+    d = x64 - x64.max(1, keepdims=True)
+    lse = np.log(np.exp(d).sum(1, keepdims=True))
+    for log_form in (False, True):
+        print(f"softmax {rows}x{C} log={log_form}", flush=True)
+        K.softmax_fwd(log_form, rows, C, X.ptr, Y.ptr)
+        hipmem.synchronize()
+        assert_close64(Y.read(), d - lse if log_form else np.exp(d - lse), 1.0 if log_form else 0.0, f"log={log_form}")
+    x[1, C // 2] = 0
+    x[2] = 1
+    x64 = x.astype(np.float64)
+    X, S = Off(x, 0), Off(np.zeros((rows, 2)), 0)
+    K.layer_norm_fwd(rows, C, X.ptr, W.ptr, B.ptr, 1e-5, Y.ptr, S.ptr)
+    hipmem.synchronize()
+    m, r = x64.mean(1, keepdims=True), 1 / np.sqrt(x64.var(1, keepdims=True) + 1e-5)
+    xh = (x64 - m) * r
+    # (x - m) r w + b: the mean, rstd and four operations rounded once each
+    assert (np.abs(Y.read() - (xh * w + b)) <= 8 * 2.0 ** -24 * ((np.abs(x64) + np.abs(m)) * r * np.abs(w) + np.abs(b))).all()
