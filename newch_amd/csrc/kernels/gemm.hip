@@ -23,11 +23,13 @@
 // where a tile's waves split K, wave group g of S sums panels g, g + S, ... so and the S totals are added in
 // order.  A small panel sum is not rounded against the whole running total, so the error of a K-term dot product
 // grows like that of a blocked sum rather than like K sequential additions.  A panel that K ends inside comes
-// first.  The tile, and with it the split, is chosen from the problem's shape and layout alone (sg_pick), so
-// results are identical run to run and on any device.  The order differs from the reference's serial one, so
+// first.  The kernel, and with it S, is chosen (sg_pick) from M, N, K, the layout, the number of matrices in the call and
+// whether the operands' rows are 16-byte aligned: the same call gives the same bits run to run and on any device, but a
+// row of a batch, or a matrix of a batched product, may be summed in another order alone than in company, and aligned
+// operands in another than unaligned ones.  The order differs from the reference's serial one too, so
 // the parity bar is the fp32 error bound of a K-term dot product.
 //
-// Kernels: k_sgemm_dma (256 x 256 tiles, panels loaded straight into LDS) for aligned problems that give every CU
+// Kernels: k_sgemm_dma (256 x 256 or 128 x 128 tiles, panels loaded straight into LDS) for aligned problems that give every CU
 // such tiles, the register-staged tiles of gemm_tile.hpp for the rest.  Blocks are remapped so each XCD
 // (blocks b with b % 8 equal) works a contiguous run of tiles, and tiles run in groups of 8 tile-rows so
 // neighbouring blocks share panels in L2.
@@ -307,8 +309,8 @@ static int sg_launch_dma(SgArgs &p, int64_t count, hipStream_t st, const char *w
 // the tiles are the ones that a choice by them over sizes from 1 to 8192 takes, and together cost 0.2% over the whole
 // family of shapes tried.  Small tiles split K over the waves of a workgroup: a product with few tiles still fills
 // the chip (x[8,4096] W[4096,4096]^T: 109 us on the 64 x 64 tile that was the smallest, 14 us on 16 x 16 with 16
-// waves).  The choice fixes how K is split, so it depends on the shape and layout alone: planned for kPlanCUs,
-// never for the device.
+// waves).  The choice fixes how K is split, so it depends on the call alone -- sizes, layout, count and alignment -- and is
+// planned for kPlanCUs, never for the device.
 struct SgTile {
     int bm, bn, lanes;
     float c[3][4];  // a0, a1, s0, s1 by M/N-contiguous operands

@@ -185,8 +185,8 @@ __global__ __launch_bounds__(kLB) void k_ce_fwd_reg_long(const float *__restrict
 }
 
 // Other rows, up to 65536 floats of any length and alignment: a workgroup of NT threads per row, the row in
-// its registers (VPT 16-byte pieces a thread, read once), rows in a grid-stride loop; the row sum in fp64
-// throughout.  HBM-bound; the element-by-element two-pass kernel that longer rows still take ran [2048, 50257] in
+// its registers (VPT 16-byte pieces a thread, read once; past 40960 floats 5, past 53248 29 registers of a lane in scratch), rows
+// in a grid-stride loop; the row sum in fp64 throughout.  HBM-bound; the element-by-element two-pass kernel that longer rows still take ran [2048, 50257] in
 // 576 us, [4096, 6000] in 76 us (here 77 and 20).  With 1024 threads only one or two workgroups fit a CU, so a barrier
 // between the maximum and the sum would have all of them load, then all of them compute (90 us): EARLY, each wave
 // takes its own maximum m_w and sums exp(x - m_w) as soon as its part of the row is there, and wave 0 forms the

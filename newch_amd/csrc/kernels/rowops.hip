@@ -1,9 +1,9 @@
 // Row kernels: softmax / log_softmax (ops_nn.c:22-71) and LayerNorm (ops_nn.c:434-522).
 //
-// A row is held in registers by one wave64 or one workgroup (VPL 128-bit vectors per lane), so each op
-// reads its inputs from HBM exactly once and writes its outputs once; the row statistics (max,
-// sums) are wave64 shuffle reductions.  The longest rows (and LayerNorm's unaligned ones) take a
-// workgroup-per-row path that re-reads the row from global memory (L2-resident) per pass.
+// A row is held by one wave64 or one workgroup (VPL or VPT 16-byte pieces a lane), in registers but for a few lanes' worth
+// where a kernel says so, so each op reads its inputs from HBM exactly once and writes its outputs once; the row
+// statistics (max, sums) are wave64 shuffle reductions.  Rows past 65536 floats (softmax backward 32768, LayerNorm backward
+// 12288) take workgroup-per-row kernels that re-read the row from global memory (L2-resident) per pass.
 //
 // Per element the fp32 expressions are the reference's (exp8 for the softmax exponentials, the
 // same association everywhere), so given the row statistics each output is the reference's
@@ -333,21 +333,36 @@ __global__ __launch_bounds__(NT) void k_softmax_bwd_wg(const float *__restrict__
     }
 }
 
-// (pieces a thread, threads) of the workgroup kernels for a row length
-#define NC_WG_SWITCH(C, CALL)                                                            \
-    if ((C) <= 2048) { constexpr int VP = 2, NT = 256; CALL; }                           \
-    else if ((C) <= 3072) { constexpr int VP = 3, NT = 256; CALL; }                      \
-    else if ((C) <= 4096) { constexpr int VP = 4, NT = 256; CALL; }                      \
-    else if ((C) <= 6144) { constexpr int VP = 6, NT = 256; CALL; }                      \
-    else if ((C) <= 8192) { constexpr int VP = 8, NT = 256; CALL; }                      \
-    else if ((C) <= 12288) { constexpr int VP = 6, NT = 512; CALL; }                     \
-    else if ((C) <= 16384) { constexpr int VP = 8, NT = 512; CALL; }                     \
-    else if ((C) <= 20480) { constexpr int VP = 5, NT = 1024; CALL; }                    \
-    else if ((C) <= 24576) { constexpr int VP = 6, NT = 1024; CALL; }                    \
-    else if ((C) <= 32768) { constexpr int VP = 8, NT = 1024; CALL; }                    \
-    else if ((C) <= 40960) { constexpr int VP = 10, NT = 1024; CALL; }                   \
-    else if ((C) <= 53248) { constexpr int VP = 13, NT = 1024; CALL; }                   \
-    else { constexpr int VP = 16, NT = 1024; CALL; }
+// (pieces a thread, threads) of the workgroup kernels for a row length of up to MAX floats
+template <int VP_, int NT_>
+struct WgShape {
+    static constexpr int VP = VP_, NT = NT_;
+};
+template <int64_t MAX, class F>
+static void wg_switch(int64_t C, F call) {
+    if (C <= 2048) return call(WgShape<2, 256>());
+    if (C <= 3072) return call(WgShape<3, 256>());
+    if (C <= 4096) return call(WgShape<4, 256>());
+    if (C <= 6144) return call(WgShape<6, 256>());
+    if (C <= 8192) return call(WgShape<8, 256>());
+    if (C <= 12288) return call(WgShape<6, 512>());
+    if (C <= 16384) return call(WgShape<8, 512>());
+    if (C <= 20480) return call(WgShape<5, 1024>());
+    if (C <= 24576) return call(WgShape<6, 1024>());
+    if (C <= 32768) return call(WgShape<8, 1024>());
+    if constexpr (MAX > 32768) {
+        if (C <= 40960) return call(WgShape<10, 1024>());
+        if (C <= 53248) return call(WgShape<13, 1024>());
+        call(WgShape<16, 1024>());
+    }
+}
+#define NC_WG_SWITCH(MAX, C, CALL)                                                              \
+    {                                                                                           \
+        wg_switch<MAX>(C, [&](auto shape) {                                                     \
+            constexpr int VP = decltype(shape)::VP, NT = decltype(shape)::NT;                   \
+            CALL;                                                                               \
+        });                                                                                     \
+    }
 // Rows of up to 1024 floats: a wave per row.  A ragged [65536, 197] ran 84 us forward element by element, 28 as a wave.
 constexpr int64_t kWaveRowMax = 1024, kWgRowMax = 65536;
 constexpr int64_t kWgRowMaxBwd = 32768;  // two rows in registers
@@ -451,7 +466,8 @@ __global__ __launch_bounds__(kRowB) void k_ln_fwd_reg(const float *__restrict__ 
 }
 
 // Rows of more than 1024 floats (up to 65536), any length and alignment: a workgroup of NT threads per row, the row in
-// its registers, so x is read once where k_ln_fwd_blk reads it three times.  HBM-bound: [16384, 3001] 223 ->
+// its registers (past 32768 floats 14, 54 or 163 of a lane's values in scratch), so x is read once where k_ln_fwd_blk reads it
+// three times.  HBM-bound: [16384, 3001] 223 ->
 // 73 us, [16384, 8192] 574 -> 192 (5.6 TB/s); [16384, 4096] 102 -> 90 against a wave per row.
 template <int VPT, int NT>
 __global__ __launch_bounds__(NT) void k_ln_fwd_wg(const float *__restrict__ x, const float *__restrict__ w,
@@ -1181,14 +1197,10 @@ __global__ __launch_bounds__(kCombCols *kCombSlices) void k_ln_cols_combine(cons
     }
 }
 
+// 16-byte pieces a lane of a wave that holds a row of up to 1024 floats; 0 past that
 static int vpl_for(int64_t C) {
     const int64_t nv = (C + 3) / 4;
-    if (nv <= 64) return 1;
-    if (nv <= 128) return 2;
-    if (nv <= 256) return 4;
-    if (nv <= 512) return 8;
-    if (nv <= 1024) return 16;
-    return 0;
+    return nv <= 64 ? 1 : nv <= 128 ? 2 : nv <= 256 ? 4 : 0;
 }
 
 #ifndef NC_LN_BWD_BLOCKS_PER_CU
@@ -1231,8 +1243,7 @@ struct LnPlan {
 
 static LnPlan ln_plan(int64_t rows, int64_t D, bool aligned, bool has_gx) {
     LnPlan p{};
-    p.vpl = (D % 4 == 0 && aligned) ? vpl_for(D) : 0;
-    if (p.vpl > 4) p.vpl = 0;  // rows past 1024 floats go to teams of waves
+    p.vpl = (D % 4 == 0 && aligned) ? vpl_for(D) : 0;  // rows past 1024 floats go to teams of waves
     p.reg = p.vpl != 0;
     p.team = !p.reg && D <= kLnTeamMax;
     if (p.team) {
@@ -1246,7 +1257,7 @@ static LnPlan ln_plan(int64_t rows, int64_t D, bool aligned, bool has_gx) {
         if (p.blocks < 1) p.blocks = 1;
         p.ws = (size_t)p.blocks * 2 * D * sizeof(double);
     } else if (p.reg) {
-        p.full = has_gx && p.vpl <= 4 && D == (int64_t)p.vpl * 4 * kWave;
+        p.full = has_gx && D == (int64_t)p.vpl * 4 * kWave;
         p.pair = NC_LN_BWD_PAIR && p.full && (p.vpl == 2 || p.vpl == 4);
         if (p.pair) {  // one workgroup per CU of a 256-CU part, rows dealt to its pairs in turn
             p.blocks = std::min<int64_t>(kPlanCUs, (rows + kLnPairs - 1) / kLnPairs);
@@ -1255,7 +1266,7 @@ static LnPlan ln_plan(int64_t rows, int64_t D, bool aligned, bool has_gx) {
             p.ws = (size_t)p.blocks * 2 * D * sizeof(double);
             return p;
         }
-        const int per_cu = p.full ? NC_LN_BWD_PP_BLOCKS_PER_CU : p.vpl <= 4 ? NC_LN_BWD_BLOCKS_PER_CU : 1;
+        const int per_cu = p.full ? NC_LN_BWD_PP_BLOCKS_PER_CU : NC_LN_BWD_BLOCKS_PER_CU;
         // the resident workgroups of a 256-CU part: rows_per_block fixes which rows each gw/gb
         // partial holds, so it depends on the shape only
         int64_t want = (int64_t)kPlanCUs * per_cu;
@@ -1303,8 +1314,8 @@ extern "C" NC_HIP_API int nc_hip_softmax_fwd(int log_form, int64_t rows, int64_t
             return rc ? rc : nc_hip_softmax_fwd(log_form, rows - kWgRowsPerLaunch, C, x + kWgRowsPerLaunch * C,
                                                 y + kWgRowsPerLaunch * C, stream);
         }
-        if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, true>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
-        else NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, false>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
+        if (log_form) NC_WG_SWITCH(kWgRowMax, C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, true>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
+        else NC_WG_SWITCH(kWgRowMax, C, hipLaunchKernelGGL((k_softmax_fwd_wg<VP, NT, false>), dim3((unsigned)rows), NT, 0, st, x, y, (int)C))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         if (log_form) hipLaunchKernelGGL(k_softmax_fwd_blk<true>, grid, kRowB, 0, st, x, y, rows, C);
@@ -1345,10 +1356,10 @@ extern "C" NC_HIP_API int nc_hip_softmax_bwd(int log_form, int64_t rows, int64_t
             return rc ? rc : nc_hip_softmax_bwd(log_form, rows - kWgRowsPerLaunch, C, y + e, g + e, gi + e, accumulate, stream);
         }
         const dim3 grid((unsigned)rows);
-        if (log_form && accumulate) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, true>), grid, NT, 0, st, y, g, gi, (int)C))
-        else if (log_form) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, false>), grid, NT, 0, st, y, g, gi, (int)C))
-        else if (accumulate) NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, true>), grid, NT, 0, st, y, g, gi, (int)C))
-        else NC_WG_SWITCH(C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, false>), grid, NT, 0, st, y, g, gi, (int)C))
+        if (log_form && accumulate) NC_WG_SWITCH(kWgRowMaxBwd, C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, true>), grid, NT, 0, st, y, g, gi, (int)C))
+        else if (log_form) NC_WG_SWITCH(kWgRowMaxBwd, C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, true, false>), grid, NT, 0, st, y, g, gi, (int)C))
+        else if (accumulate) NC_WG_SWITCH(kWgRowMaxBwd, C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, true>), grid, NT, 0, st, y, g, gi, (int)C))
+        else NC_WG_SWITCH(kWgRowMaxBwd, C, hipLaunchKernelGGL((k_softmax_bwd_wg<VP, NT, false, false>), grid, NT, 0, st, y, g, gi, (int)C))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         if (log_form && accumulate) hipLaunchKernelGGL((k_softmax_bwd_blk<true, true>), grid, kRowB, 0, st, y, g, gi, rows, C);
@@ -1378,7 +1389,7 @@ extern "C" NC_HIP_API int nc_hip_layer_norm_fwd(int64_t rows, int64_t D, const f
             return rc ? rc : nc_hip_layer_norm_fwd(rows - kWgRowsPerLaunch, D, x + e, w, b, eps, y + e,
                                                    stats + 2 * kWgRowsPerLaunch, stream);
         }
-        NC_WG_SWITCH(D, hipLaunchKernelGGL((k_ln_fwd_wg<VP, NT>), dim3((unsigned)rows), NT, 0, st, x, w, b, eps, y, stats, (int)D))
+        NC_WG_SWITCH(kWgRowMax, D, hipLaunchKernelGGL((k_ln_fwd_wg<VP, NT>), dim3((unsigned)rows), NT, 0, st, x, w, b, eps, y, stats, (int)D))
     } else {
         const unsigned grid = (unsigned)(rows < num_cus() * 8 ? rows : num_cus() * 8);
         hipLaunchKernelGGL(k_ln_fwd_blk, grid, kRowB, 0, st, x, w, b, eps, y, stats, rows, D);
