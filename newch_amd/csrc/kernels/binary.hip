@@ -711,7 +711,9 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_col(const float *__restrict_
 // L: the lanes of an item, the workgroup's or a wave's.  Where K is short (row_waves) a workgroup has a few of its lanes at
 // work, and an item's bounds, division and exchange are what it takes: [65536, 7] summed over rows 100 us (168 with
 // division) by workgroups, 64 (116) with an element a lane and no division taken out, 28 (40) by waves.
-template <int MODE, int L>
+// NEAR: K within a step of 2^32, where the index could pass it: counted from the chunk's start (which costs 5% elsewhere, in
+// scalar registers: [704, 704, 128] over all but the middle dim with division 115 -> 120 us).
+template <int MODE, int L, bool NEAR>
 __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict__ g, const float *__restrict__ p1,
                                                         const float *__restrict__ p2, RedPlan pl, double alpha,
                                                         double *__restrict__ part) {
@@ -725,12 +727,12 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
     bool one = MODE == 2 || MODE == 3;
     for (int d = 0; d <= in; d++) one = one && pl.red.st[od][d] == 0;
     for (uint64_t item = (uint64_t)blockIdx.x * kItems + sub; item < total; item += (uint64_t)gridDim.x * kItems) {  // uniform over an item's lanes
-        const uint32_t p = pl.P == 1 ? 0 : (uint32_t)(item / pl.M);
-        const uint32_t mi = (uint32_t)(item - (uint64_t)p * pl.M);
+        const uint32_t mi = (uint32_t)(item % pl.M);
+        const uint32_t p = (uint32_t)(item / pl.M);
         int64_t ko[4];
         offsets<4>(pl.kept, mi, ko);
         const uint32_t k0 = p * pl.chunk;
-        const uint32_t k1 = k0 + min(pl.chunk, pl.K - k0);  // K and the chunks' ends reach 2^32: no sum may pass it
+        const uint32_t k1 = k0 + min(pl.chunk, pl.K - k0);  // the last chunk's end may be 2^32 by sum
         const float *gk = g + ko[0], *q1 = p1 + ko[1], *q2 = p2 + ko[2];
         double inv = 1.0;
         if (one) {
@@ -743,18 +745,18 @@ __global__ __launch_bounds__(kB) void k_grad_reduce_row(const float *__restrict_
             return grad_d<MODE>((double)gv, (double)v1, (double)v2, alpha);
         };
         double acc = 0.0;
-        const bool single = L == kWave && pl.K <= kWave;  // an element a lane
+        bool single = false;
+        if constexpr (L == kWave) single = pl.K <= kWave;  // an element a lane
         if (single && lane < pl.K) {
             int64_t ro[3];
             offsets<3>(pl.red, lane, ro);
             acc = term(gk[ro[0]], MODE != 0 ? q1[ro[1]] : 0.0f, MODE == 3 ? q2[ro[2]] : 0.0f);
         }
-        for (uint32_t at = 4 * lane; !single && at < k1 - k0; at += 4 * L) {
-            const uint32_t k = k0 + at;
+        for (uint32_t k = k0 + 4 * lane; !single && (NEAR ? k - k0 < k1 - k0 : k < k1); k += 4 * L) {
             int64_t ro[3];
             offsets<3>(pl.red, k, ro);
             const f4 z = {0.f, 0.f, 0.f, 0.f};
-            if (k1 - k >= 4) {
+            if (NEAR ? k1 - k >= 4 : k + 4 <= k1) {
                 const bool in_row = k - pl.red.div[in].div(k) * w + 4 <= w;
                 const f4 gv = row4<3>(gk, pl.red, 0, ro[0], k, in_row);
                 const f4 v1 = MODE != 0 && !(MODE == 2 && one) ? row4<3>(q1, pl.red, 1, ro[1], k, in_row) : z;
@@ -1078,8 +1080,10 @@ static int launch_grad(const float *g, const float *p1, const float *p2, float *
         const bool waves = row_waves(pl);
         const uint64_t blocks = waves ? (items + kB / kWave - 1) / (kB / kWave) : items;
         const unsigned grid = (unsigned)(blocks < 1048576 ? blocks : 1048576);
-        if (waves) hipLaunchKernelGGL((k_grad_reduce_row<MODE, kWave>), dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
-        else hipLaunchKernelGGL((k_grad_reduce_row<MODE, kB>), dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part);
+        const auto launch = [&](auto *kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(kB), 0, st, g, p1, p2, pl, (double)alpha, part); };
+        if (waves) launch(k_grad_reduce_row<MODE, kWave, false>);
+        else if (pl.K > UINT32_MAX - 4 * kB) launch(k_grad_reduce_row<MODE, kB, true>);
+        else launch(k_grad_reduce_row<MODE, kB, false>);
     }
     const unsigned fg = (pl.M + kB - 1) / kB;
     if (acc)
