@@ -889,10 +889,13 @@ __global__ __launch_bounds__(kColB) void k_grad_cols(const float *__restrict__ g
     typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
     __shared__ double sh[kColB / kWave][kColW];
     const int x = threadIdx.x % kColLanes, y = threadIdx.x / kColLanes;
-    // XCD i (blocks b with b % 8 == i) takes the i-th of 8 runs of neighbouring column groups: where rows are not 128-byte
-    // aligned two groups share each row's cache line between them
-    const uint32_t xcd = blockIdx.x & 7, per = gridDim.x >> 3, rem = gridDim.x & 7;
-    const uint32_t id = xcd * per + min(xcd, rem) + (blockIdx.x >> 3);
+    // Where rows are not 128-byte aligned two neighbouring column groups share a cache line of each row: XCD i (blocks b with
+    // b % 8 == i) takes the i-th of 8 runs of groups.  Aligned rows go over the XCDs in turn ([2048, 768]: 6.7 us, 7.1 in runs).
+    uint32_t id = blockIdx.x;
+    if (((uintptr_t)g | (uint64_t)c.gr * 4) & 127) {
+        const uint32_t xcd = id & 7, per = gridDim.x >> 3, rem = gridDim.x & 7;
+        id = xcd * per + min(xcd, rem) + (id >> 3);
+    }
     const uint32_t groups = (c.M + kColW - 1) / kColW, p = id / groups;
     const uint32_t m0 = (id - p * groups) * kColW, m = m0 + 2 * x;
     const uint32_t k0 = p * c.chunk, k1 = min(c.K, k0 + c.chunk);
