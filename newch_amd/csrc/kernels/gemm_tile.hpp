@@ -166,9 +166,10 @@ struct TilePanel {
 // Bound by the matrix cores and, at one workgroup per CU, by what its waves wait for together (LDS reads after
 // the barrier, the barrier itself): x[2048,3072] W[768,3072]^T, 256 tiles of 64 x 96 with 2 K groups, 135 us on the
 // 64 x 64 tile of 16-k stages before (384 tiles over 256 CUs, one stage of loads in flight), 105 us with the panel
-// loaded and stored between two panels and the reads left to the compiler, 86 us (112 TFLOP/s) in this order.  A third
-// LDS buffer with the next panel's fragments read ahead timed no better (105 us).  M/N-contiguous operands cost
-// 10-15% more (their reads into LDS are as many, their fragments 2 to 4 reads).
+// loaded and stored between two panels and the reads left to the compiler, 86 us (112 TFLOP/s) in this order timed
+// alone and 94 among a training step's launches.  A third LDS buffer with the next panel's fragments read ahead
+// timed no better (105 us).  M/N-contiguous operands cost 10-15% more (their reads into LDS are as many, their
+// fragments 2 to 4 reads).
 template <class Cfg, bool AK, bool BK>
 __global__ __launch_bounds__(Cfg::NT) void k_sgemm_tile(SgArgs p) {
     constexpr int TM = Cfg::TM, TN = Cfg::TN, KS = Cfg::KS;

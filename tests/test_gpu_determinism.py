@@ -177,10 +177,9 @@ def test_losses_independent_of_cus(K, N, C):
     across_cus(K, run)
 
 
-# fp32 GEMM: the tile size follows the CU count (256 x 256 tiles when they give every CU one, else
-# 128 x 128 or 64 x 64), and every tile size sums an output's K products in the same order, so the
-# bits do not change; shapes straddle the tile-size thresholds for 32 .. 1024 CUs, with K below and
-# above the direct-to-LDS threshold and a ragged one
+# fp32 GEMM: the tile, and with it the order in which an output's K products are summed, is chosen from the
+# call's sizes, layout, count and alignment for a fixed 256 CUs, so neither it nor the bits change with the
+# device's count; the shapes run the direct-to-LDS and the register-staged tiles, with a ragged K
 GEMM = [(1024, 1024, 512, 0, 1), (2048, 1536, 256, 0, 0), (512, 768, 1040, 1, 1), (3000, 1000, 300, 1, 0),
         (4096, 2048, 64, 0, 1)]
 
